@@ -537,10 +537,17 @@ void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int r
   hipLaunchKernelGGL(k_ov_close, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d, rounds);
 }
 
+// the reference's order: the entries each atom can meet, then the walk
+void enq_overlap_exact(dml_ctx *c, const double *u, int64_t n_u, int max_passes) {
+  if (!c->d.ovx_n) return;  // no replica in this mode
+  hipLaunchKernelGGL(k_ov_contacts<8>, dim3((unsigned)(c->P * 8 / DML_BLOCK)), dim3(DML_BLOCK), 0,
+                     c->st, c->d);
+  hipLaunchKernelGGL(k_ov_exact, dim3(c->nrep), dim3(OVX_BLOCK), 0, c->st, c->d, u, n_u,
+                     max_passes);
+}
+
 void enq_overlap(dml_ctx *c) {
-  if (c->any_exact)
-    hipLaunchKernelGGL(k_ov_exact, dim3(c->nrep), dim3(64), 0, c->st, c->d, (const double *)nullptr,
-                       (int64_t)0, 100000);
+  if (c->any_exact) enq_overlap_exact(c, nullptr, 0, 100000);
   if (c->any_rounds) enq_overlap_rounds(c, nullptr, 0, c->rounds, 0);
 }
 
@@ -736,6 +743,27 @@ double *upload_tmp(dml_ctx *c, const double *h, int64_t n) {
     return nullptr;
   hipMemcpyAsync(d, h, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->st);
   return d;
+}
+
+// the lists of the reference-order overlap pass, once a replica asks for it
+int ensure_exact(dml_ctx *c) {
+  if (c->d.ovx_n) return DML_OK;
+  int any = 0;
+  for (auto &h : c->reps) any |= h.p.overlap_mode == DML_OVERLAP_EXACT;
+  if (!any) return DML_OK;
+  uint8_t *n = nullptr;
+  int32_t *l = nullptr;
+  unsigned long long *m = nullptr;
+  if (dalloc(&n, c->P) || dalloc(&l, c->P * (int64_t)OVX_MAX) || dalloc(&m, c->P / 64)) {
+    hipFree(n);
+    hipFree(l);
+    hipFree(m);
+    return DML_E_NOMEM;
+  }
+  c->d.ovx_n = n;
+  c->d.ovx_l = l;
+  c->d.ovx_m = m;
+  return DML_OK;
 }
 
 void refresh_modes(dml_ctx *c) {
@@ -938,7 +966,7 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
     for (int q = 0; q < c->reps[r].p.pcap / DML_BLOCK; q++)
       b2r[c->reps[r].p.poff / DML_BLOCK + q] = r;
   hipMemcpyAsync(d.blk2rep, b2r.data(), sizeof(int32_t) * b2r.size(), hipMemcpyHostToDevice, c->st);
-  if (alloc_cells(c) || upload_params(c)) {
+  if (ensure_exact(c) || alloc_cells(c) || upload_params(c)) {
     dml_destroy(c);
     return DML_E_NOMEM;
   }
@@ -971,7 +999,7 @@ int dml_destroy(dml_ctx *c) {
                   d.species, d.flags, d.rowflag, d.bkey, d.pid, d.ref_order, d.ref_tmp,
                   d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ov_rev,
                   d.ov_st, d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
-                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ovr[0], d.ovr[1], d.ov_more, d.pf4, d.bf4, d.gc_order,
+                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ovr[0], d.ovr[1], d.ov_more, d.ovx_n, d.ovx_l, d.ovx_m, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
                   d.cm_rep, d.cm_cell, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
                   d.gb_pt, d.gb_u, d.gb_du, d.gb_g, d.gb_kind, d.gb_cell, d.gb_nblk, d.gb_blk,
@@ -1393,8 +1421,7 @@ int dml_overlap_moveback(dml_ctx *c, const double *u_contact, int64_t n_u, int32
   // n_u uniforms per replica, replica r at [r*n_u, (r+1)*n_u)
   if (u_contact && n_u <= 0) return DML_E_ARG;
   double *du = u_contact ? upload_tmp(c, u_contact, n_u * c->nrep) : nullptr;
-  hipLaunchKernelGGL(k_ov_exact, dim3(c->nrep), dim3(64), 0, c->st, c->d, (const double *)du, n_u,
-                     max_passes > 0 ? max_passes : 100000);
+  enq_overlap_exact(c, du, n_u, max_passes > 0 ? max_passes : 100000);
   int rc = finish(c);
   hipFree(du);
   return rc;
@@ -1950,6 +1977,7 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   p.halted = HALT_PAUSED;  // until dml_set_state
   h.cfg = g;
   h.p = p;
+  if ((rc = ensure_exact(c))) return rc;
   if (rows_for(g) > c->d.maxnn) {
     // wider rows than the context has: grow them (keeps every row)
     int nm = next_pow2(rows_for(g));

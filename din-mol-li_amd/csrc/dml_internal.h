@@ -17,6 +17,8 @@
 
 #define DML_BLOCK 256
 #define OVA_PER 8  // items per thread of one k_ov_apply block pass
+#define OVX_MAX 16  // row entries listed per atom for the reference-order overlap pass
+#define OVX_BLOCK 1024
 #define NEAR_MAX 4  // row positions within rcut listed per atom by the row build
 #define DML_GCMC_BLOCK 256  // one workgroup per GCMC replica
 
@@ -305,6 +307,12 @@ struct DevState {
   int32_t *wl_cnt;
   int32_t *ovw[2], *ovr[2];
   int32_t *ov_more;       // [3][nrep]: the replica reverted or deferred in a round
+  // reference-order overlap pass (only with such a replica): per ref position
+  // the row entries it can meet (count, 255 = more than listed), and the
+  // masks of positions to visit of replicas too large for LDS
+  uint8_t *ovx_n;
+  int32_t *ovx_l;         // OVX_MAX per ref position
+  unsigned long long *ovx_m;
   int32_t *gc_order;      // gcmc group in list order (global slots)
   int32_t *b2slot;        // hs%b index -> global slot, -1 when free
   int32_t *seq;           // creation number: the order of sys%alist

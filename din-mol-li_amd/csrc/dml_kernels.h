@@ -22,6 +22,8 @@ __global__ void k_ghost_scatter(DevState s, int only_ermak);
 __global__ void k_ermak_b(DevState s, int only_if_ghost);
 __global__ void k_brownian(DevState s, const double *noise, const double *udep);
 __global__ void k_ermak_a(DevState s, const double *noise, const double *udep);
+template <int LPA>
+__global__ void k_ov_contacts(DevState s);
 __global__ void k_ov_exact(DevState s, const double *u, int64_t n_u, int max_passes);
 __global__ void k_ov_begin(DevState s);
 __global__ void k_ov_apply_r(DevState s, int round);
