@@ -766,6 +766,23 @@ int ensure_exact(dml_ctx *c) {
   return DML_OK;
 }
 
+// a replica's counters: the sum of its shards
+int read_counters(dml_ctx *c, int rep, DevCounters *out) {
+  const int n = c->d.ncsh;
+  std::vector<DevCounters> v(n);
+  HIPCHECK(hipMemcpy(v.data(), c->d.cnt + (int64_t)rep * n, sizeof(DevCounters) * n,
+                     hipMemcpyDeviceToHost));
+  constexpr int words = sizeof(DevCounters) / sizeof(unsigned long long);
+  unsigned long long sum[words] = {};
+  for (int q = 0; q < n; q++) {
+    unsigned long long one[words];
+    memcpy(one, &v[q], sizeof(DevCounters));
+    for (int k = 0; k < words; k++) sum[k] += one[k];
+  }
+  memcpy(out, sum, sizeof(DevCounters));
+  return DML_OK;
+}
+
 void refresh_modes(dml_ctx *c) {
   c->any_ermak = c->any_brown = c->any_rounds = c->any_exact = c->any_piston = c->any_gcmc = 0;
   c->any_chunks = 0;
@@ -895,7 +912,12 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   e |= dalloc(&d.part_i, 2 * (P / DML_BLOCK));
   e |= dalloc(&d.blk2rep, P / DML_BLOCK);
   e |= dalloc(&d.rp, nrep);
-  e |= dalloc(&d.cnt, nrep);
+  // a few thousand shards in all: a single large system needs the most (its
+  // row build adds from some ten thousand waves), the replicas of an ensemble
+  // are each other's shards
+  d.ncsh = 512;
+  while (d.ncsh > 8 && (int64_t)d.ncsh * nrep > 4096) d.ncsh /= 2;
+  e |= dalloc(&d.cnt, (int64_t)nrep * d.ncsh);
   e |= dalloc(&d.err, 1);
   e |= dalloc(&d.wl[0], P);
   e |= dalloc(&d.wl[1], P);
@@ -959,7 +981,7 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   hipMemsetAsync(d.b2slot, 0xff, sizeof(int32_t) * P, c->st);
   hipMemsetAsync(d.gc_order, 0xff, sizeof(int32_t) * P, c->st);
   hipMemsetAsync(d.seq, 0, sizeof(int32_t) * P, c->st);
-  hipMemsetAsync(d.cnt, 0, sizeof(DevCounters) * nrep, c->st);
+  hipMemsetAsync(d.cnt, 0, sizeof(DevCounters) * nrep * d.ncsh, c->st);
   hipMemsetAsync(d.err, 0, sizeof(int32_t), c->st);
   std::vector<int32_t> b2r(P / DML_BLOCK);
   for (int r = 0; r < nrep; r++)
@@ -1911,10 +1933,6 @@ int dml_progress(dml_ctx *c, int64_t *steps, int32_t *status, int32_t *running) 
   if (!c) return DML_E_ARG;
   int rc = fetch_params(c);
   if (rc) return rc;
-  std::vector<DevCounters> h(c->nrep);
-  if (steps) {
-    HIPCHECK(hipMemcpy(h.data(), c->d.cnt, sizeof(DevCounters) * c->nrep, hipMemcpyDeviceToHost));
-  }
   for (int r = 0; r < c->nrep; r++) {
     const RepParams &p = c->reps[r].p;
     if (steps) steps[r] = (int64_t)p.step;
@@ -1992,7 +2010,7 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
     c->d.maxnn = nm;
   }
   hipMemsetAsync(c->d.cell_cnt + p.coff, 0, sizeof(int32_t) * p.ccap, c->st);
-  hipMemsetAsync(c->d.cnt + rep, 0, sizeof(DevCounters), c->st);
+  hipMemsetAsync(c->d.cnt + (int64_t)rep * c->d.ncsh, 0, sizeof(DevCounters) * c->d.ncsh, c->st);
   hipMemsetAsync(c->d.ov_near + p.poff, 0xff, (size_t)p.pcap, c->st);
   refresh_modes(c);
   return upload_params(c);
@@ -2007,7 +2025,7 @@ int dml_last_run_ms(dml_ctx *c, double *ms) {
 int dml_get_counters(dml_ctx *c, int32_t rep, dml_counters *out) {
   if (!c || rep < 0 || rep >= c->nrep || !out) return DML_E_ARG;
   DevCounters h;
-  HIPCHECK(hipMemcpy(&h, c->d.cnt + rep, sizeof(h), hipMemcpyDeviceToHost));
+  if (int rc = read_counters(c, rep, &h)) return rc;
   out->try_ = (int64_t)h.try_;
   out->depo = (int64_t)h.depo;
   out->choques = (int64_t)h.choques;
@@ -2026,7 +2044,7 @@ int dml_get_counters(dml_ctx *c, int32_t rep, dml_counters *out) {
 int dml_list_stats(dml_ctx *c, int32_t rep, double *mean_nn, int64_t *rebuilds, int64_t *steps) {
   if (!c || rep < 0 || rep >= c->nrep) return DML_E_ARG;
   DevCounters h;
-  HIPCHECK(hipMemcpy(&h, c->d.cnt + rep, sizeof(h), hipMemcpyDeviceToHost));
+  if (int rc = read_counters(c, rep, &h)) return rc;
   if (mean_nn) *mean_nn = h.nn_rows ? (double)h.nn_sum / (double)h.nn_rows : 0.0;
   if (rebuilds) *rebuilds = (int64_t)h.nupd;
   if (steps) *steps = (int64_t)h.steps;

@@ -161,7 +161,11 @@ __host__ __device__ inline int tessellate_rep(RepParams &p, int first) {
   return 0;
 }
 
-struct DevCounters {
+// one shard of a replica's counters, on lines of its own: atomics on one
+// address are done one after the other (about 17 ns each when they come from
+// all the XCDs), so kernels in which every wave adds pick a shard by wave
+// and the host sums the shards
+struct alignas(128) DevCounters {
   unsigned long long try_, depo, choques, choques3, nupd, ins, del, passes;
   unsigned long long nn_sum, nn_rows, steps, ov_unfinished;
   unsigned long long particle_steps;  // sum over steps of the atoms alive
@@ -333,7 +337,8 @@ struct DevState {
   // tables
   int32_t *blk2rep;
   RepParams *rp;
-  DevCounters *cnt;
+  DevCounters *cnt;       // [nrep][ncsh]
+  int32_t ncsh;           // counter shards per replica (a power of two)
   int32_t *err;
   // batched GCMC.  Per trial (pool of every batched replica, gb_off + t):
   // point, (u1, u2), energy, kind (0 insertion, 1 deletion, 2 point outside

@@ -8,6 +8,11 @@
 
 #define WAVE 64
 
+// the counters of replica r that wave (or atom, ...) k adds to
+__device__ inline DevCounters &cnt_of(const DevState &s, int r, int k) {
+  return s.cnt[(int64_t)r * s.ncsh + (k & (s.ncsh - 1))];
+}
+
 __device__ inline int same_pos(const DevState &s, int i) {
   return s.px[i] == s.cx[i] && s.py[i] == s.cy[i] && s.pz[i] == s.cz[i];
 }
@@ -146,7 +151,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_dispmax_final(DevState s) {
       // new rows: the cell-tile and wave-per-cell row builds list their
       // entries within rcut
       Pw->ovn_stamp = Pw->lb_kind != 1 ? Pw->step + 1 : 0;
-      atomicAdd(&s.cnt[r].nupd, 1ull);
+      atomicAdd(&cnt_of(s, r, 0).nupd, 1ull);
     }
   }
 }
@@ -161,7 +166,7 @@ __global__ void k_force_rebuild(DevState s) {
   Pw->any_ghost = 0;
   Pw->nlimbo = 0;
   Pw->ovn_stamp = Pw->lb_kind != 1 ? Pw->step + 1 : 0;
-  atomicAdd(&s.cnt[r].nupd, 1ull);
+  atomicAdd(&cnt_of(s, r, 0).nupd, 1ull);
 }
 
 // ------------------------------------------------------------------------
@@ -366,8 +371,8 @@ __global__ void __launch_bounds__(WPB *WAVE) k_listbuild(DevState s) {
     s.nn[i] = nn;
     s.rowflag[i] = (uint8_t)ghost;
     if (ghost) s.rp[r].any_ghost = 1;
-    atomicAdd(&s.cnt[r].nn_sum, (unsigned long long)nn);
-    atomicAdd(&s.cnt[r].nn_rows, 1ull);
+    atomicAdd(&cnt_of(s, r, t).nn_sum, (unsigned long long)nn);
+    atomicAdd(&cnt_of(s, r, t).nn_rows, 1ull);
   }
 }
 
@@ -550,8 +555,8 @@ __global__ void __launch_bounds__(DML_BLOCK) k_listbuild_cells(DevState s) {
     }
     __syncthreads();  // sh_A and the LDS tiles are rewritten by the next cell
     if (tid == 0 && sh_rows) {
-      atomicAdd(&s.cnt[r].nn_sum, sh_nnsum);
-      atomicAdd(&s.cnt[r].nn_rows, sh_rows);
+      atomicAdd(&cnt_of(s, r, c).nn_sum, sh_nnsum);
+      atomicAdd(&cnt_of(s, r, c).nn_rows, sh_rows);
       sh_nnsum = 0;
       sh_rows = 0;
     }
@@ -672,8 +677,8 @@ k_listbuild_wc(DevState s) {
     const RepParams &P = s.rp[r];
     if (r != cur_r) {
       if (cur_r >= 0 && lane == 0 && acc_rows) {
-        atomicAdd(&s.cnt[cur_r].nn_sum, acc_nn);
-        atomicAdd(&s.cnt[cur_r].nn_rows, acc_rows);
+        atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
+        atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
       }
       cur_r = r;
       acc_nn = acc_rows = 0;
@@ -884,8 +889,8 @@ k_listbuild_wc(DevState s) {
     }
   }
   if (cur_r >= 0 && lane == 0 && acc_rows) {
-    atomicAdd(&s.cnt[cur_r].nn_sum, acc_nn);
-    atomicAdd(&s.cnt[cur_r].nn_rows, acc_rows);
+    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
+    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
   }
 }
 
@@ -990,8 +995,8 @@ k_listbuild_wr(DevState s) {
       const RepParams &P = s.rp[r];
       if (r != cur_r) {
         if (cur_r >= 0 && lane == 0 && acc_rows) {
-          atomicAdd(&s.cnt[cur_r].nn_sum, acc_nn);
-          atomicAdd(&s.cnt[cur_r].nn_rows, acc_rows);
+          atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
+          atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
         }
         cur_r = r;
         acc_nn = acc_rows = 0;
@@ -1301,8 +1306,8 @@ k_listbuild_wr(DevState s) {
     }
   }
   if (cur_r >= 0 && lane == 0 && acc_rows) {
-    atomicAdd(&s.cnt[cur_r].nn_sum, acc_nn);
-    atomicAdd(&s.cnt[cur_r].nn_rows, acc_rows);
+    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
+    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
   }
 }
 
@@ -1735,7 +1740,7 @@ __device__ inline int atom_pbc(const DevState &s, const RepParams &P, int r,
     }
   }
   if (z <= 0.0) {
-    atomicAdd(&s.cnt[r].try_, 1ull);
+    atomicAdd(&cnt_of(s, r, i / WAVE).try_, 1ull);
     double ne;
     if (udep) {
       ne = udep[t];
@@ -1744,7 +1749,7 @@ __device__ inline int atom_pbc(const DevState &s, const RepParams &P, int r,
       ne = u01_from(w.x, w.y);
     }
     if (ne < P.prob) {
-      atomicAdd(&s.cnt[r].depo, 1ull);
+      atomicAdd(&cnt_of(s, r, i / WAVE).depo, 1ull);
       s.species[i] = SP_F;
       s.rp[r].any_f = 1;
       depos = 1;
@@ -2097,11 +2102,11 @@ __global__ void __launch_bounds__(OVX_BLOCK) k_ov_exact(DevState s, const double
     }
   }
   if (lane == 0) {
-    atomicAdd(&s.cnt[r].try_, n_try);
-    atomicAdd(&s.cnt[r].depo, n_depo);
-    atomicAdd(&s.cnt[r].choques, n_ch);
-    atomicAdd(&s.cnt[r].choques3, n_ch3);
-    atomicAdd(&s.cnt[r].passes, n_pass);
+    atomicAdd(&cnt_of(s, r, 0).try_, n_try);
+    atomicAdd(&cnt_of(s, r, 0).depo, n_depo);
+    atomicAdd(&cnt_of(s, r, 0).choques, n_ch);
+    atomicAdd(&cnt_of(s, r, 0).choques3, n_ch3);
+    atomicAdd(&cnt_of(s, r, 0).passes, n_pass);
   }
 }
 
@@ -2139,6 +2144,7 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
   const int gtid = bid * DML_BLOCK + threadIdx.x;
   const int sub = gtid % LPA;
   const int64_t stride = (int64_t)nbk * (DML_BLOCK / LPA);
+  const int wv = gtid / WAVE;  // counter shard
   // one ref position: its verdict, and what it adds to its replica's
   // counters (k_r = the replica, -1 when the position is not scanned)
   auto scan_one = [&](int64_t item, int &k_try, int &k_ch, int &k_ch3, int &k_more, int &k_r) {
@@ -2239,7 +2245,13 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
         s.ov_rev[j] = stamp;  // k_ov_apply walks every ref position in round 0
       } else if (atomicExch(&s.ov_rev[j], stamp) != stamp) {
         // first to revert j in this round: it is applied from the list
-        const int q = atomicAdd(&s.wl_cnt[2 + round % 2], 1);
+        // (one atomic for the lanes that are here together)
+        const unsigned long long m = __ballot(1);
+        const int lead = __builtin_ctzll(m);
+        int q = 0;
+        if ((int)(threadIdx.x % WAVE) == lead) q = atomicAdd(&s.wl_cnt[2 + round % 2], __popcll(m));
+        q = __shfl(q, lead) + (int)__builtin_amdgcn_mbcnt_hi(
+                                  (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
         if (q < ptotal) s.ovr[round % 2][q] = j;
       }
       return 0;
@@ -2312,15 +2324,15 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
       const int t_ch3 = __builtin_amdgcn_readlane(wave_scan_incl(k_ch3), WAVE - 1);
       const bool more = __ballot(k_more) != 0;
       if (threadIdx.x % WAVE == 0) {
-        if (t_try) atomicAdd(&s.cnt[r0].try_, (unsigned long long)(uint32_t)t_try);
-        if (t_ch) atomicAdd(&s.cnt[r0].choques, (unsigned long long)(uint32_t)t_ch);
-        if (t_ch3) atomicAdd(&s.cnt[r0].choques3, (unsigned long long)(uint32_t)t_ch3);
+        if (t_try) atomicAdd(&cnt_of(s, r0, wv).try_, (unsigned long long)(uint32_t)t_try);
+        if (t_ch) atomicAdd(&cnt_of(s, r0, wv).choques, (unsigned long long)(uint32_t)t_ch);
+        if (t_ch3) atomicAdd(&cnt_of(s, r0, wv).choques3, (unsigned long long)(uint32_t)t_ch3);
         if (more) s.ov_more[cur * s.nrep + r0] = 1;
       }
     } else if (k_r >= 0) {
-      if (k_try) atomicAdd(&s.cnt[k_r].try_, (unsigned long long)(uint32_t)k_try);
-      if (k_ch) atomicAdd(&s.cnt[k_r].choques, (unsigned long long)(uint32_t)k_ch);
-      if (k_ch3) atomicAdd(&s.cnt[k_r].choques3, (unsigned long long)(uint32_t)k_ch3);
+      if (k_try) atomicAdd(&cnt_of(s, k_r, wv).try_, (unsigned long long)(uint32_t)k_try);
+      if (k_ch) atomicAdd(&cnt_of(s, k_r, wv).choques, (unsigned long long)(uint32_t)k_ch);
+      if (k_ch3) atomicAdd(&cnt_of(s, k_r, wv).choques3, (unsigned long long)(uint32_t)k_ch3);
       if (k_more) s.ov_more[cur * s.nrep + k_r] = 1;
     }
   }
@@ -2346,7 +2358,7 @@ __device__ inline int ov_apply_one(const DevState &s, int r, const RepParams &P,
   int moved = 0;
   if ((st & 1) && !(st & 2)) f |= DML_FL_SKIP;
   if (st & 4) {
-    atomicAdd(&s.cnt[r].depo, 1ull);
+    atomicAdd(&cnt_of(s, r, i / WAVE).depo, 1ull);
     s.species[i] = SP_F;
     s.rp[r].any_f = 1;
     moved = 1;
@@ -2496,7 +2508,7 @@ __global__ void k_ov_end(DevState s, int rounds, int err_if_pending) {
   if (s.rp[r].overlap_mode != DML_OVERLAP_ROUNDS || s.rp[r].halted) return;
   if (s.ov_more[((rounds - 1) % 3) * s.nrep + r]) {
     if (err_if_pending) rep_fail(s, r, ERR_OVERLAP);
-    atomicAdd(&s.cnt[r].ov_unfinished, 1ull);
+    atomicAdd(&cnt_of(s, r, 0).ov_unfinished, 1ull);
   }
 }
 
@@ -2507,7 +2519,7 @@ __global__ void k_ov_close(DevState s, int rounds) {
   RepParams *Pw = s.rp + r;
   if (Pw->overlap_mode != DML_OVERLAP_ROUNDS) return;
   Pw->ov_round += rounds + 2;
-  atomicAdd(&s.cnt[r].passes, 1ull);
+  atomicAdd(&cnt_of(s, r, 0).passes, 1ull);
 }
 
 __global__ void k_init_pf4(DevState s, int64_t n) {
@@ -2787,8 +2799,8 @@ __global__ void k_rep_op(DevState s, int op) {
     }
   } else {
     Pw->step += 1;
-    s.cnt[r].steps += 1;
-    s.cnt[r].particle_steps += (unsigned long long)Pw->nat;
+    cnt_of(s, r, 0).steps += 1;
+    cnt_of(s, r, 0).particle_steps += (unsigned long long)Pw->nat;
     if (Pw->step_limit > 0 && Pw->step >= Pw->step_limit) Pw->halted |= HALT_PAUSED;
   }
 }
@@ -2807,8 +2819,8 @@ __global__ void k_step_end(DevState s) {
   }
   Pw->rho_count = 0;
   Pw->step += 1;
-  s.cnt[r].steps += 1;
-  s.cnt[r].particle_steps += (unsigned long long)Pw->nat;
+  cnt_of(s, r, 0).steps += 1;
+  cnt_of(s, r, 0).particle_steps += (unsigned long long)Pw->nat;
   if (Pw->step_limit > 0 && Pw->step >= Pw->step_limit) Pw->halted |= HALT_PAUSED;
 }
 
@@ -3696,8 +3708,8 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
     Pw->pid_next = pid_next;
     Pw->seq_next = seq_next;
     Pw->gcmc_calls = call + 1;
-    if (n_ins) atomicAdd(&s.cnt[r].ins, n_ins);
-    if (n_del) atomicAdd(&s.cnt[r].del, n_del);
+    if (n_ins) atomicAdd(&cnt_of(s, r, 0).ins, n_ins);
+    if (n_del) atomicAdd(&cnt_of(s, r, 0).del, n_del);
     if (fail) rep_fail(s, r, fail);
   }
 }
@@ -4765,8 +4777,8 @@ __global__ void __launch_bounds__(WAVE) k_gb_commit(DevState s, int r, const dou
     Pw->gc_pending = 2;
     if (nins || ndel) Pw->ovn_stamp = 0;
     Pw->gcmc_calls = call + 1;
-    if (nins) atomicAdd(&s.cnt[r].ins, (unsigned long long)nins);
-    if (ndel) atomicAdd(&s.cnt[r].del, (unsigned long long)ndel);
+    if (nins) atomicAdd(&cnt_of(s, r, 0).ins, (unsigned long long)nins);
+    if (ndel) atomicAdd(&cnt_of(s, r, 0).del, (unsigned long long)ndel);
   }
 }
 
