@@ -295,6 +295,9 @@ int build_maps(dml_ctx *c) {
   if ((rc = put(&c->d.cm_rep, &capc, cr))) return rc;
   capc = c->cap_cm;
   if ((rc = put(&c->d.cm_cell, &capc, cc))) return rc;
+  capc = c->cap_cm;
+  std::fill(cc.begin(), cc.end(), 0);
+  if ((rc = put(&c->d.cm_nref, &capc, cc))) return rc;
   c->cap_cm = capc;
   if ((rc = put(&c->d.tm_rep, &capt, tr))) return rc;
   capt = c->cap_tm;
@@ -381,6 +384,29 @@ int alloc_cells(dml_ctx *c) {
 // ---- phases -------------------------------------------------------------
 unsigned clamp_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(n, 65535)); }
 
+// waves per cell (2^sl) and workgroups of the register-resident row build.
+// A cell of ~24 ref atoms is ~60 us of one wave's time, so a system with fewer
+// dense cells than the chip has wave slots (7,168) is split: 4 waves a cell
+// below 24,000 ref atoms (4,000 particles 83 -> 31 us, 12,000 59 -> 36), 2
+// below 200,000 (37,000: 92 -> 68, 100,000: 94 -> 79), none above (2M: 835,
+// split 930); sparse cells (a few atoms) are never split (1,505 ions of a
+// chunks run: 10.6, split 12.3).  Dense cells want more workgroups than
+// resident ones to even out the tail (16 dense replicas 141 -> 115 us, 2M 980
+// -> 835), sparse ones the fewest (24 mixed replicas 336 -> 320)
+void wr_shape(const dml_ctx *c, int *sl, int *g) {
+  int64_t nref = 0, cells = 0;
+  for (auto &h : c->reps) {
+    const RepParams &p = h.p;
+    if (p.halted || p.lb_kind != 3) continue;
+    nref += p.nref;
+    cells += p.use_cells ? (int64_t)p.ncells[0] * p.ncells[1] * p.ncells[2] : 1;
+  }
+  const bool dense = nref >= 4 * cells;
+  *sl = !dense || nref >= 200000 ? 0 : nref >= 24000 ? 1 : 2;
+  const int64_t need = ((c->d.n_cm << *sl) + 3) / 4, most = dense ? 7168 : 1792;
+  *g = (int)(std::min(std::max<int64_t>(need, 8), most) + 7) / 8 * 8;
+}
+
 void enq_listbuild(dml_ctx *c) {
   if (c->any_lb[0] && c->d.n_tm > 0)
     hipLaunchKernelGGL(k_listbuild_cells, dim3(clamp_grid(c->d.n_tm)), dim3(DML_BLOCK), 0, c->st,
@@ -395,14 +421,14 @@ void enq_listbuild(dml_ctx *c) {
     hipLaunchKernelGGL(k_listbuild_wc, dim3(g), dim3(DML_BLOCK), 0, c->st, c->d);
   }
   if (c->any_lb[3]) {
-    unsigned g = clamp_grid((c->d.n_cm + 3) / 4);
-    g = std::max(8u, g / 8 * 8);
-    // 3 chunks of 64 a pass at 7 waves per SIMD (4 at 6 waves, 2 at 8 were
-    // slower on the 256-replica ensemble); 2 chunks at 8 waves a choice
+    int sl, g;
+    wr_shape(c, &sl, &g);
+    // 3 chunks of 64 a pass at 7 waves per SIMD (4 chunks or 6 waves: within
+    // 3 % either way); 2 chunks at 8 waves a choice
     if (c->lb_mode == 5)
-      hipLaunchKernelGGL((k_listbuild_wr<2, 8>), dim3(g), dim3(DML_BLOCK), 0, c->st, c->d);
+      hipLaunchKernelGGL((k_listbuild_wr<2, 8>), dim3(g), dim3(DML_BLOCK), 0, c->st, c->d, sl);
     else
-      hipLaunchKernelGGL((k_listbuild_wr<3, 7>), dim3(g), dim3(DML_BLOCK), 0, c->st, c->d);
+      hipLaunchKernelGGL((k_listbuild_wr<3, 7>), dim3(g), dim3(DML_BLOCK), 0, c->st, c->d, sl);
   }
 }
 
@@ -1023,7 +1049,7 @@ int dml_destroy(dml_ctx *c) {
                   d.ov_st, d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
                   d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ovr[0], d.ovr[1], d.ov_more, d.ovx_n, d.ovx_l, d.ovx_m, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
-                  d.cm_rep, d.cm_cell, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
+                  d.cm_rep, d.cm_cell, d.cm_nref, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
                   d.gb_pt, d.gb_u, d.gb_du, d.gb_g, d.gb_kind, d.gb_cell, d.gb_nblk, d.gb_blk,
                   d.gb_ncf, d.gb_cf, d.gb_res, d.gb_slot, d.gi_trial, d.gi_next, d.gi_del,
                   d.gi_tmpl, d.gd_trial, d.gd_vpos, d.gd_slot, d.gd_bso, d.gd_brank,
@@ -1807,7 +1833,9 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
   }
   // what the captured step depends on: the phases present and the launch
   // shapes (rounds <= 32, lanes <= 64)
-  const int64_t modes = (int64_t)c->any_ermak | c->any_brown << 1 | c->any_rounds << 2 |
+  int lb_sl, lb_g;
+  wr_shape(c, &lb_sl, &lb_g);
+  const int64_t modes = (int64_t)lb_sl << 36 | (int64_t)lb_g << 38 | (int64_t)c->any_ermak | c->any_brown << 1 | c->any_rounds << 2 |
                         c->any_exact << 3 | c->any_piston << 4 | c->any_gcmc << 5 |
                         (int64_t)c->any_chunks << 31 |
                         (int64_t)c->rounds << 6 | (int64_t)c->lpa << 12 |

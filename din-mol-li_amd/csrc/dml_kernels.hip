@@ -33,6 +33,7 @@ __device__ inline float4 bucket_f4(const DevState &s, int i) {
   f.w = __int_as_float((__float_as_int(f.w) & 0xff) | (int)s.flags[i] << 8);
   return f;
 }
+__device__ inline bool bucket_ref(float4 f) { return (__float_as_int(f.w) >> 8 & DML_FL_REF) != 0; }
 // squared minimum-image distance in FP32.  A pair is decided in FP32 only
 // outside the band cutoff^2 +- RepParams::pf_margin (set by the host from
 // the largest box and the list radius, see pf_margin_for); inside it the FP64
@@ -186,6 +187,7 @@ __device__ inline int want_cells(const RepParams &P, int gcs) {
 __global__ void k_zero_cells(DevState s, int gcs) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < s.n_cm;
        g += (int64_t)gridDim.x * blockDim.x) {
+    s.cm_nref[g] = 0;
     const RepParams &P = s.rp[s.cm_rep[g]];
     const int c = s.cm_cell[g];
     if (P.halted || !want_cells(P, gcs) || c >= ncell_total(P)) continue;
@@ -608,6 +610,16 @@ __device__ inline int wave_scan_incl(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
   return v;
 }
+// inclusive running maximum over the wave (values >= 0), the same moves
+__device__ inline int wave_max_incl(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return v;
+}
 // the same within each row of 16 lanes, and within each half of 32
 __device__ inline int row_scan16(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
@@ -895,111 +907,100 @@ k_listbuild_wc(DevState s) {
 }
 
 // ------------------------------------------------------------------------
-// Rows of one centre cell with its candidates held in registers: a wave
-// loads up to NCH chunks of 64 candidates of the 27-cell stream at a time
-// (WPE waves per SIMD: the walk is latency-bound, occupancy pays),
-// then walks the cell's ref atoms one at a time; each atom's count, row
+// Rows of a centre cell with its candidates held in registers: a wave loads
+// up to NCH chunks of 64 candidates of the 27-cell stream at a time, then
+// walks its ref atoms of the cell one at a time; each atom's count, row
 // address and position stay in scalar registers across the chunks, and a
 // chunk's hits are one compare, one ballot and one store of the chunk's
 // lanes in stream order (stencil order, then chain order: ngroup_cells,
 // Neighbor.F90:509-535, strict '<'; ngroup_verlet, ':358-424', rejects on
 // '>').  FP32 prefilter with margin, FP64 in the band.  Entries within
 // rcut (FP32 with margin) are listed like k_listbuild_wc lists them.
+//
+// The cell list is dealt to the XCDs in blocks of LB_BLK cells, round robin,
+// so that a half-empty box or replicas of uneven density load them evenly
+// while an XCD's L2 still holds the candidates of neighbouring cells; inside an XCD
+// its nwx waves take the cells one by one in list order.  2^sl waves share a
+// cell (LB_PART ref atoms a wave or more): wave v takes part v % 2^sl of every
+// (nwx >> sl)-th cell.  The cells to do come from cm_nref (ref atoms per cell,
+// by k_cell_sort_w; 0 for a cell that is not rebuilt), 64 per load, so an
+// empty cell costs a lane of one load.
+//
+// What bounds it: instruction issue (about 30 instructions a chunk of 64 pair
+// tests) with the wait for a pass's candidates behind it.  Before, each wave
+// took one contiguous run of cells, an XCD one eighth of the list, every cell
+// was looked at through its replica's parameters and a stencil lane wrote its
+// cell's entries one by one: 100,000 particles 265 -> 79 us a build, 24 mixed
+// replicas 472 -> 320, 2M 1,775 -> 835, 1,505 ions in sparse cells 37 -> 11.
 // ------------------------------------------------------------------------
+#define LB_PART 6
+#define LB_BLK 64
 template <int NCH, int WPE>
 __global__ void __launch_bounds__(DML_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
-k_listbuild_wr(DevState s) {
-  // one wave's LDS slice, at a wave-uniform base (one lane offset serves
-  // every array)
+k_listbuild_wr(DevState s, int sl) {
+  // bucket entries of a pass's stream positions, and a lane's row length at
+  // the start of a pass: one wave's LDS slice, at a wave-uniform base
   struct Slice {
-    int32_t pos[NCH * WAVE];  // bucket entries of a pass's stream positions
-    // the 64 cells of a batch (replica, cell, count, x, y|z|ghost, image
-    // reference x, y), kept here rather than in registers
-    int32_t bat[7][WAVE];
-    int32_t nn0[WAVE];  // a lane's row length at the start of a pass
-    int4 ctr[WAVE];     // the cell's current centre atoms: slot, FP32 position
+    int32_t pos[NCH * WAVE];
+    int32_t nn0[WAVE];
   };
   __shared__ Slice lbr[DML_BLOCK / WAVE];
-  Slice &L = lbr[__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)];
-  int32_t *wpos = L.pos;
-  int32_t(*bat)[WAVE] = L.bat;
-  int32_t *nn0s = L.nn0;
-  int4 *ctr = L.ctr;
+  const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  int32_t *wpos = lbr[wib].pos;
+  int32_t *nn0s = lbr[wib].nn0;
   const int lane = threadIdx.x % WAVE;
   const int maxnn = s.maxnn;
   const int kofs = lane < 27 ? (kMap[lane][0] + 1) | (kMap[lane][1] + 1) << 4 |
                                    (kMap[lane][2] + 1) << 8
                              : 0x111;
-  // XCD-aware runs of cells, as in k_listbuild_wc
-  const int nb = gridDim.x;  // a multiple of 8
-  const int64_t vb = (int64_t)(blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8;
-  const int64_t wid =
-      vb * (DML_BLOCK / WAVE) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-  // (32-bit division: the cell list holds fewer than 2^31 cells)
-  const uint32_t nwv = (uint32_t)nb * (DML_BLOCK / WAVE);
-  const int64_t run = (int64_t)(((uint32_t)s.n_cm + nwv - 1u) / nwv);
-  const int64_t g_end = min(s.n_cm, (wid + 1) * run);
+  // workgroups are dealt round-robin to the 8 XCDs (gridDim.x: a multiple
+  // of 8; nwx: of 2^sl)
+  const int xcd = blockIdx.x % 8;
+  const int wv = (int)(blockIdx.x / 8) * (DML_BLOCK / WAVE) + wib;
+  const int nwx = (int)(gridDim.x / 8) * (DML_BLOCK / WAVE);
+  const int part = wv & ((1 << sl) - 1);
+  const int step_g = nwx >> sl;
   int cur_r = -1;
   unsigned long long acc_nn = 0, acc_rows = 0;
   // the current replica's parameters, read once per replica (the parameter
   // block is written by this kernel's rare error paths, so its fields are
   // vector loads; read in the cell loop they would be a chain of waits)
   int64_t q_boff = 0;
-  int q_cells = 0, q_n0 = 0, q_n1 = 0, q_n2 = 0, q_coff = 0, q_bcap = 0, q_img = 0;
+  int q_cells = 0, q_n0 = 0, q_n1 = 0, q_n2 = 0, q_coff = 0, q_bcap = 0, q_img = 0, q_go = 0;
   double q_rl2 = 0.0;
   float q_lo = 0.f, q_hi = 0.f, q_rcf = 0.f, q_bx = 0.f, q_by = 0.f, q_ibx = 0.f, q_iby = 0.f;
-  float q_bandw = 0.f;
-  for (int64_t g0 = wid * run; g0 < g_end; g0 += WAVE) {
-    // 64 cells of the run, one per lane: count, coordinates (y, z packed,
-    // the ghost-layer flag in bit 31) and the image reference point, so
-    // the cell loop below needs no division and no parameter reads
-    int lr = 0, lc = 0, lcnt = 0, lx = 0, lyz = 0;
-    float lmx = 0.f, lmy = 0.f;
-    if (g0 + lane < g_end) {
-      lr = s.cm_rep[g0 + lane];
-      lc = s.cm_cell[g0 + lane];
-      const RepParams &Q = s.rp[lr];
-      if (!Q.halted && Q.rebuild && Q.lb_kind == 3 && lc < ncell_total(Q)) {
-        lcnt = min(s.cell_cnt[Q.coff + lc], Q.bcap);
-        if (Q.use_cells) {
-          const int w0 = Q.ncells[0] + 2, w1 = Q.ncells[1] + 2;
-          const int x = lc % w0, y = lc / w0 % w1, z = lc / (w0 * w1);
-          const int gh = x < 1 || y < 1 || z < 1 || x > Q.ncells[0] || y > Q.ncells[1] ||
-                         z > Q.ncells[2];
-          lx = x;
-          lyz = y | z << 16 | gh << 31;
-          lmx = (float)((x - 0.5) * Q.cell[0]);
-          lmy = (float)((y - 0.5) * Q.cell[1]);
-        }
+  float q_cx = 0.f, q_cy = 0.f;
+  // (a later place in the XCD's order is a later block of the list)
+  for (int64_t j0 = wv >> sl; (j0 / LB_BLK * 8 + xcd) * LB_BLK < s.n_cm;
+       j0 += (int64_t)WAVE * step_g) {
+    int lr = 0, lc = 0, ln = 0;
+    {
+      const int64_t j = j0 + (int64_t)lane * step_g;
+      const int64_t g = (j / LB_BLK * 8 + xcd) * LB_BLK + j % LB_BLK;
+      if (g < s.n_cm) {
+        ln = s.cm_nref[g];
+        lr = s.cm_rep[g];
+        lc = s.cm_cell[g];
       }
     }
-    unsigned long long work = __ballot(lcnt > 0);
-    __builtin_amdgcn_wave_barrier();
-    bat[0][lane] = lr;
-    bat[1][lane] = lc;
-    bat[2][lane] = lcnt;
-    bat[3][lane] = lx;
-    bat[4][lane] = lyz;
-    bat[5][lane] = __float_as_int(lmx);
-    bat[6][lane] = __float_as_int(lmy);
-    __builtin_amdgcn_wave_barrier();
+    // a cell of few ref atoms is not split into all the parts
+    unsigned long long work = __ballot(ln > part * LB_PART);
     while (work) {
       const int q = __builtin_ctzll(work);
       work &= work - 1;
-      const int r = rfl_i(bat[0][q]);
-      const int c = rfl_i(bat[1][q]);
-      const int ccnt = rfl_i(bat[2][q]);
-      const int cx0 = rfl_i(bat[3][q]);
-      const int cyz = rfl_i(bat[4][q]);
-      const float mxf = __int_as_float(rfl_i(bat[5][q])), myf = __int_as_float(rfl_i(bat[6][q]));
+      const int r = __builtin_amdgcn_readlane(lr, q);
+      const int c = __builtin_amdgcn_readlane(lc, q);
+      const int nrefc = __builtin_amdgcn_readlane(ln, q);
+      const int parts = min(1 << sl, (nrefc + LB_PART - 1) / LB_PART);
       const RepParams &P = s.rp[r];
       if (r != cur_r) {
         if (cur_r >= 0 && lane == 0 && acc_rows) {
-          atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
-          atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
+          atomicAdd(&cnt_of(s, cur_r, wv * 8 + xcd).nn_sum, acc_nn);
+          atomicAdd(&cnt_of(s, cur_r, wv * 8 + xcd).nn_rows, acc_rows);
         }
         cur_r = r;
         acc_nn = acc_rows = 0;
+        q_go = !rfl_i(P.halted);
         q_boff = rfl_l(P.boff);
         q_cells = rfl_i(P.use_cells);
         q_n0 = rfl_i(P.ncells[0]);
@@ -1017,32 +1018,31 @@ k_listbuild_wr(DevState s) {
         q_by = (float)rfl_d(P.box[1]);
         q_ibx = (float)rfl_d(P.one_box[0]);
         q_iby = (float)rfl_d(P.one_box[1]);
-        // a pair is near the list radius when |d^2 - rl^2| <= bandw in
-        // FP32: a superset of [rl2lo, rl2hi] (the difference of two floats
-        // this close is exact; rl2lo, rl2hi are within half an ulp of
-        // rl^2 -+ margin)
-        q_bandw = pfm * 1.0001f + 1.0e-6f * (float)q_rl2;
+        q_cx = (float)rfl_d(P.cell[0]);
+        q_cy = (float)rfl_d(P.cell[1]);
       }
+      if (!q_go) continue;
       const int64_t cbase = q_boff + (int64_t)c * q_bcap;
       int ghost = 0, ci0 = 0, ci1 = 0, ci2 = 0;
       if (q_cells) {
-        ci0 = cx0;
-        ci1 = cyz & 0xffff;
-        ci2 = cyz >> 16 & 0x7fff;
-        ghost = (uint32_t)cyz >> 31;
+        const uint32_t w0 = q_n0 + 2, w1 = q_n1 + 2, cq = (uint32_t)c / w0;
+        ci0 = (int)((uint32_t)c - cq * w0);
+        ci2 = (int)(cq / w1);
+        ci1 = (int)(cq - ci2 * w1);
+        ghost = ci0 < 1 || ci1 < 1 || ci2 < 1 || ci0 > q_n0 || ci1 > q_n1 || ci2 > q_n2;
       }
-      // the first 64 centre atoms' entries, loaded with the stencil counts
-      // (one wait for both)
-      int4 my_c = make_int4(-1, 0, 0, 0);
-      int my_ref = 0;
-      if (lane < ccnt) {
-        my_c.x = s.bucket[cbase + lane];
-        const float4 f = s.bf4[cbase + lane];
-        my_c.y = __float_as_int(f.x);
-        my_c.z = __float_as_int(f.y);
-        my_c.w = __float_as_int(f.z);
-        my_ref = (__float_as_int(f.w) >> 8 & DML_FL_REF) != 0;
+      // the image reference point: the midpoint of the centre cell
+      const float mxf = ((float)ci0 - 0.5f) * q_cx, myf = ((float)ci1 - 0.5f) * q_cy;
+      // the first 64 centre atoms' entries (entries past the cell's count
+      // are read and dropped: a cell's bucket holds them), loaded with the
+      // stencil counts (one wait for both)
+      int cs = -1;
+      float4 cf = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (lane < q_bcap) {
+        cs = s.bucket[cbase + lane];
+        cf = s.bf4[cbase + lane];
       }
+      const int ccnt = min(rfl_i(s.cell_cnt[q_coff + c]), q_bcap);
       // the 27 stencil cells: lane k holds count and first entry of cell k
       // (the first entry relative to the replica's bucket region, which
       // holds fewer than 2^31 entries)
@@ -1073,29 +1073,24 @@ k_listbuild_wr(DevState s) {
       const float rl2lo = q_lo, rl2hi = q_hi, rcf = q_rcf;
       const float bxf = q_bx, byf = q_by, ibx = q_ibx, iby = q_iby;
       const int img = q_img;
+      int rank0 = 0;  // ref atoms of the cell before a0
       for (int a0 = 0; a0 < ccnt; a0 += WAVE) {
         // centre atoms a0 .. a0+63 of this cell, one per lane
-        const int na = (ccnt - a0) < WAVE ? (ccnt - a0) : WAVE;
         const int64_t e0 = cbase + a0;
-        if (a0 > 0) {
-          // the next 64 centre atoms
-          my_c = make_int4(-1, 0, 0, 0);
-          my_ref = 0;
-          if (lane < na) {
-            my_c.x = s.bucket[e0 + lane];
-            const float4 f = s.bf4[e0 + lane];
-            my_c.y = __float_as_int(f.x);
-            my_c.z = __float_as_int(f.y);
-            my_c.w = __float_as_int(f.z);
-            my_ref = (__float_as_int(f.w) >> 8 & DML_FL_REF) != 0;
-          }
+        if (a0 > 0 && lane < ccnt - a0) {
+          cs = s.bucket[e0 + lane];
+          cf = s.bf4[e0 + lane];
         }
-        const unsigned long long refm = __ballot(my_ref);
+        const bool my_ref = lane < ccnt - a0 && (__float_as_int(cf.w) >> 8 & DML_FL_REF) != 0;
+        unsigned long long refm = __ballot(my_ref);
+        if (parts > 1) {
+          const int k = rank0 + (int)__builtin_amdgcn_mbcnt_hi(
+                                    (uint32_t)(refm >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((uint32_t)refm, 0u));
+          rank0 += __popcll(refm);
+          refm = __ballot(my_ref && (uint32_t)k % (uint32_t)parts == (uint32_t)part);
+        }
         if (!refm) continue;
-        // (read back at wave-uniform addresses by the walks below)
-        __builtin_amdgcn_wave_barrier();
-        ctr[lane] = my_c;
-        __builtin_amdgcn_wave_barrier();
         // row length (bits 0-23) and entries within rcut (24-31, saturating)
         int my_nn = 0;
         for (int s0 = 0; s0 < total; s0 += NCH * WAVE) {
@@ -1104,17 +1099,30 @@ k_listbuild_wr(DevState s) {
           const int nch = min(NCH, (total - s0 + WAVE - 1) / WAVE);
           const int last = min(total - s0, NCH * WAVE) - 1;
           // the bucket entries of stream positions s0 .. s0+last, in stream
-          // order: each stencil lane writes those of its cell (one wave's
-          // LDS slice, written and read by that wave only, in order)
+          // order: every stencil cell with entries here marks its first one,
+          // a running maximum carries the marks on (one wave's LDS slice,
+          // written and read by that wave only, in order)
+#pragma unroll
+          for (int h = 0; h < NCH; h++)
+            if (h < nch) wpos[h * WAVE + lane] = 0;
+          __builtin_amdgcn_wave_barrier();
           {
             const int lo = max(0, s0 - kpre), hi = min(kcnt, s0 + last + 1 - kpre);
-            for (int e = lo; e < hi; e++) wpos[kpre + e - s0] = kb32 + e;
+            if (lo < hi) wpos[kpre + lo - s0] = lane + 1;
           }
           __builtin_amdgcn_wave_barrier();
-          // (the slots' reads first, then the loads: no wait between chunks)
-          int slot[NCH];
+          // (the slots first, then the loads: no wait between chunks)
+          int slot[NCH], carry = 0;
 #pragma unroll
-          for (int h = 0; h < NCH; h++) slot[h] = wpos[min(h * WAVE + lane, last)];
+          for (int h = 0; h < NCH; h++) {
+            slot[h] = 0;
+            if (h < nch) {
+              const int k = max(wave_max_incl(wpos[h * WAVE + lane]), carry);
+              carry = __builtin_amdgcn_readlane(k, WAVE - 1);
+              slot[h] = __shfl(kb32 - kpre, k - 1) + s0 + min(h * WAVE + lane, last);
+              wpos[h * WAVE + lane] = slot[h];  // (for the band below)
+            }
+          }
           int cj[NCH];
           float cx[NCH], cy[NCH], cz[NCH];
 #pragma unroll
@@ -1148,7 +1156,6 @@ k_listbuild_wr(DevState s) {
           // centres with a pair near the list radius: their rows of this
           // super-chunk are written again below, the band decided in FP64
           unsigned long long redo = 0;
-          const float rl2f = (float)rl2, bandw = q_bandw;
           auto d2f = [&](auto img_c, float x, float y, float z, float xa, float ya,
                          float za) -> float {
             if (decltype(img_c)::value) {
@@ -1158,69 +1165,50 @@ k_listbuild_wr(DevState s) {
             return d2_f32(P, make_float4(x, y, z, 0.f), make_float4(xa, ya, za, 0.f), bxf, byf,
                           ibx, iby);
           };
-          // the centre loop, one form per pair-distance arithmetic
           // one centre atom's walk over the chunks: its row count, near
           // count and row address in scalar registers
-          struct Ctr {
-            int a, i, nn, nc;
-            float xa, ya, za, bmin;
-            int32_t *row;
-          };
-          auto start = [&](Ctr &c, int a) {
-            c.a = a;
-            const int4 v = ctr[a];
-            c.i = rfl_i(v.x);
-            c.xa = __int_as_float(rfl_i(v.y));
-            c.ya = __int_as_float(rfl_i(v.z));
-            c.za = __int_as_float(rfl_i(v.w));
-            const int pk = __builtin_amdgcn_readlane(my_nn, a);
-            c.nn = pk & 0xffffff;
-            c.nc = (int)((uint32_t)pk >> 24);
-            c.row = s.nbr + (int64_t)c.i * maxnn;
-            // the least |d^2 - rl^2| this lane meets (lanes past the
-            // stream's end repeat its last entry)
-            c.bmin = 3.0e38f;
-          };
-          auto step = [&](auto img_c, Ctr &c, int h) {
-            const unsigned long long vm = h == nch - 1 ? vlast : ~0ull;
-            const float df = d2f(img_c, cx[h], cy[h], cz[h], c.xa, c.ya, c.za);
-            c.bmin = fminf(c.bmin, fabsf(df - rl2f));
-            const unsigned long long lt = __builtin_amdgcn_ballot_w64(df < rl2lo);
-            const unsigned long long hm = lt & vm & __builtin_amdgcn_ballot_w64(cj[h] != c.i);
-            const int nh = __popcll(hm);
-            const uint32_t pr = __builtin_amdgcn_mbcnt_hi(
-                (uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0u));
-            const unsigned long long ok =
-                c.nn + nh <= maxnn ? hm : hm & __builtin_amdgcn_ballot_w64(c.nn + (int)pr < maxnn);
-            if (__builtin_amdgcn_inverse_ballot_w64(ok)) c.row[(uint32_t)c.nn + pr] = cj[h];
-            const unsigned long long nm = __builtin_amdgcn_ballot_w64(df <= rcf) & hm;
-            if (nm) {
-              const int qn = c.nc + (int)__builtin_amdgcn_mbcnt_hi(
-                                        (uint32_t)(nm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)nm, 0u));
-              if (__builtin_amdgcn_inverse_ballot_w64(nm) && qn < NEAR_MAX)
-                s.nearl[(int64_t)c.i * NEAR_MAX + qn] = c.nn + (int)pr;
-              const int nc2 = c.nc + __popcll(nm);
-              c.nc = nc2 < 255 ? nc2 : 255;
-            }
-            c.nn += nh;
-          };
-          auto finish = [&](Ctr &c) {
-            if (__builtin_amdgcn_ballot_w64(c.bmin <= bandw)) redo |= 1ull << c.a;
-            my_nn = lane == c.a ? (c.nn | c.nc << 24) : my_nn;
-          };
-          // the centre loop, one form per pair-distance arithmetic
           auto centres = [&](auto img_c) {
             unsigned long long m = refm;
             while (m) {
-              Ctr A;
-              start(A, __builtin_ctzll(m));
+              const int a = __builtin_ctzll(m);
               m &= m - 1;
+              const int i = __builtin_amdgcn_readlane(cs, a);
+              const float xa = rdlane_f(cf.x, a), ya = rdlane_f(cf.y, a), za = rdlane_f(cf.z, a);
+              const int pk = __builtin_amdgcn_readlane(my_nn, a);
+              int nn = pk & 0xffffff, nc = (int)((uint32_t)pk >> 24);
+              int32_t *row = s.nbr + (int64_t)i * maxnn;
+              unsigned long long band = 0;
 #pragma unroll
-              for (int h = 0; h < NCH; h++)
-                if (h < nch) step(img_c, A, h);
-              finish(A);
+              for (int h = 0; h < NCH; h++) {
+                if (h >= nch) break;
+                const unsigned long long vm = h == nch - 1 ? vlast : ~0ull;
+                const float df = d2f(img_c, cx[h], cy[h], cz[h], xa, ya, za);
+                const unsigned long long lt = __builtin_amdgcn_ballot_w64(df < rl2lo);
+                // pairs in the band (a lane past the stream's end repeats
+                // its last entry)
+                band |= __builtin_amdgcn_ballot_w64(df <= rl2hi) & ~lt;
+                const unsigned long long hm = lt & vm & __builtin_amdgcn_ballot_w64(cj[h] != i);
+                // row position of this lane's entry
+                const uint32_t at = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, (uint32_t)nn));
+                const unsigned long long ok = hm & __builtin_amdgcn_ballot_w64((int)at < maxnn);
+                if (__builtin_amdgcn_inverse_ballot_w64(ok)) row[at] = cj[h];
+                const unsigned long long nm = __builtin_amdgcn_ballot_w64(df <= rcf) & hm;
+                if (nm) {
+                  const int qn = (int)__builtin_amdgcn_mbcnt_hi(
+                      (uint32_t)(nm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)nm, (uint32_t)nc));
+                  if (__builtin_amdgcn_inverse_ballot_w64(nm) && qn < NEAR_MAX)
+                    s.nearl[(int64_t)i * NEAR_MAX + qn] = (int)at;
+                  const int nc2 = nc + __popcll(nm);
+                  nc = nc2 < 255 ? nc2 : 255;
+                }
+                nn += __popcll(hm);
+              }
+              redo |= band ? 1ull << a : 0ull;
+              my_nn = lane == a ? (nn | nc << 24) : my_nn;
             }
           };
+          // (one form per pair-distance arithmetic)
           if (img)
             centres(std::true_type());
           else
@@ -1230,10 +1218,8 @@ k_listbuild_wr(DevState s) {
           while (redo) {
             const int a = __builtin_ctzll(redo);
             redo &= redo - 1;
-            const int4 v = ctr[a];
-            const int i = rfl_i(v.x);
-            const float xa = __int_as_float(rfl_i(v.y)), ya = __int_as_float(rfl_i(v.z));
-            const float za = __int_as_float(rfl_i(v.w));
+            const int i = __builtin_amdgcn_readlane(cs, a);
+            const float xa = rdlane_f(cf.x, a), ya = rdlane_f(cf.y, a), za = rdlane_f(cf.z, a);
             const int pk = rfl_i(nn0s[a]);
             int nn = pk & 0xffffff, nc = (int)((uint32_t)pk >> 24);
             int32_t *row = s.nbr + (int64_t)i * maxnn;
@@ -1286,7 +1272,6 @@ k_listbuild_wr(DevState s) {
         my_nn &= 0xffffff;
         const bool mine = (refm >> lane) & 1ull;
         if (mine) {
-          const int my_i = ctr[lane].x;
           int nn = my_nn;
           if (nn > maxnn) {
             atomicOr(s.err, ERR_LIST);
@@ -1294,9 +1279,9 @@ k_listbuild_wr(DevState s) {
             rep_fail(s, r, ERR_LIST);
             nn = maxnn;
           }
-          s.nn[my_i] = nn;
-          s.rowflag[my_i] = (uint8_t)ghost;
-          s.ov_near[my_i] = (uint8_t)(img && my_nc <= NEAR_MAX ? my_nc : 255);
+          s.nn[cs] = nn;
+          s.rowflag[cs] = (uint8_t)ghost;
+          s.ov_near[cs] = (uint8_t)(img && my_nc <= NEAR_MAX ? my_nc : 255);
           if (ghost) s.rp[r].any_ghost = 1;
         }
         const int v = wave_scan_incl(mine ? my_nn : 0);
@@ -1306,13 +1291,13 @@ k_listbuild_wr(DevState s) {
     }
   }
   if (cur_r >= 0 && lane == 0 && acc_rows) {
-    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_sum, acc_nn);
-    atomicAdd(&cnt_of(s, cur_r, (int)wid).nn_rows, acc_rows);
+    atomicAdd(&cnt_of(s, cur_r, wv * 8 + xcd).nn_sum, acc_nn);
+    atomicAdd(&cnt_of(s, cur_r, wv * 8 + xcd).nn_rows, acc_rows);
   }
 }
 
-template __global__ void k_listbuild_wr<3, 7>(DevState s);
-template __global__ void k_listbuild_wr<2, 8>(DevState s);
+template __global__ void k_listbuild_wr<3, 7>(DevState s, int sl);
+template __global__ void k_listbuild_wr<2, 8>(DevState s, int sl);
 
 
 // bucket order by a rank sort inside one wave (cells of up to 256 atoms,
@@ -1328,7 +1313,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
   const int64_t run = (s.n_cm + nwv - 1) / nwv;
   const int64_t g_end = min(s.n_cm, (wid + 1) * run);
   for (int64_t g0 = wid * run; g0 < g_end; g0 += WAVE) {
-    int lr = 0, lc = 0, lcnt = 0;
+    int lr = 0, lc = 0, lcnt = 0, lref = 0;
     if (g0 + lane < g_end) {
       lr = s.cm_rep[g0 + lane];
       lc = s.cm_cell[g0 + lane];
@@ -1375,6 +1360,9 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
         const int kq = half ? kb : ka;
         rank += (j < mycnt) & (hdesc ? (kq > k) : (kq < k));
       }
+      const unsigned long long rm = __ballot(in && bucket_ref(f));
+      if (lane == q) lref = __popcll(rm & 0xffffffffull);
+      if (lane == q2) lref = __popcll(rm >> 32);
       if (in) {
         s.bucket[hbase + rank] = v;
         s.bx[hbase + rank] = x;
@@ -1405,10 +1393,12 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
         f = bucket_f4(s, v);
       }
       int rank = 0;
-      for (int q = 0; q < cnt; q++) {
-        const int kq = __builtin_amdgcn_readlane(k, q);  // q is wave-uniform
-        rank += desc ? (kq > k) : (kq < k);
+      for (int e = 0; e < cnt; e++) {
+        const int ke = __builtin_amdgcn_readlane(k, e);  // e is wave-uniform
+        rank += desc ? (ke > k) : (ke < k);
       }
+      const unsigned long long rm = __ballot(in && bucket_ref(f));
+      if (lane == q) lref = __popcll(rm);
       if (in) {
         b[rank] = v;
         s.bx[base + rank] = x;
@@ -1436,17 +1426,23 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
           for (int j = 0; j < SORT_W; j++) rank[j] += desc ? (kq > k[j]) : (kq < k[j]);
         }
       }
+      int nref = 0;
 #pragma unroll
       for (int j = 0; j < SORT_W; j++) {
+        bool ref = false;
         if (j * WAVE + lane < cnt) {
           const int vj = v[j], rj = rank[j];
           b[rj] = vj;
           s.bx[base + rj] = s.px[vj];
           s.by[base + rj] = s.py[vj];
           s.bz[base + rj] = s.pz[vj];
-          s.bf4[base + rj] = bucket_f4(s, vj);
+          const float4 f = bucket_f4(s, vj);
+          s.bf4[base + rj] = f;
+          ref = bucket_ref(f);
         }
+        nref += __popcll(__ballot(ref));
       }
+      if (lane == q) lref = nref;
     } else {
       if (lane == 0) {
         for (int q = 1; q < cnt; q++) {
@@ -1463,14 +1459,28 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      for (int q = lane; q < cnt; q += WAVE) {
-        int v = __hip_atomic_load(&b[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        s.bx[base + q] = s.px[v];
-        s.by[base + q] = s.py[v];
-        s.bz[base + q] = s.pz[v];
-        s.bf4[base + q] = bucket_f4(s, v);
+      int nref = 0;
+      for (int e0 = 0; e0 < cnt; e0 += WAVE) {
+        const int e = e0 + lane;
+        bool ref = false;
+        if (e < cnt) {
+          int v = __hip_atomic_load(&b[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+          s.bx[base + e] = s.px[v];
+          s.by[base + e] = s.py[v];
+          s.bz[base + e] = s.pz[v];
+          const float4 f = bucket_f4(s, v);
+          s.bf4[base + e] = f;
+          ref = bucket_ref(f);
+        }
+        nref += __popcll(__ballot(ref));
       }
+      if (lane == q) lref = nref;
     }
+    }
+    // ref atoms per cell, for the row build of the replicas that rebuild
+    if (lref > 0) {
+      const RepParams &Q = s.rp[lr];
+      if (Q.rebuild && Q.lb_kind == 3) s.cm_nref[g0 + lane] = lref;
     }
   }
 }
