@@ -84,7 +84,8 @@ struct dml_ctx {
   double last_ms = 0.0;
   int lpa = 8;
   int lpa_ov = 8;  // lanes per atom of the overlap scan (1 = thread per atom)
-  int ov_tail = 8;  // overlap rounds from this one on run in one workgroup (0: none)
+  int ov_tail = -1;  // overlap rounds from this one on run in one workgroup (0: none, -1: by size)
+  int ov_lanes_set = 0;  // lpa_ov was chosen by the caller
   // list kernel: 0 cell tiles, 1 wave per atom, 2 per replica by density
   // (0 or 1), 3 wave per cell
   int lb_mode = 4;
@@ -407,6 +408,14 @@ void wr_shape(const dml_ctx *c, int *sl, int *g) {
   *g = (int)(std::min(std::max<int64_t>(need, 8), most) + 7) / 8 * 8;
 }
 
+// slots in use in the replicas that run
+int64_t live_slots(const dml_ctx *c) {
+  int64_t n = 0;
+  for (auto &h : c->reps)
+    if (!h.p.halted) n += h.p.nslots;
+  return n;
+}
+
 void enq_listbuild(dml_ctx *c) {
   if (c->any_lb[0] && c->d.n_tm > 0)
     hipLaunchKernelGGL(k_listbuild_cells, dim3(clamp_grid(c->d.n_tm)), dim3(DML_BLOCK), 0, c->st,
@@ -465,9 +474,10 @@ void enq_cells_lists(dml_ctx *c, int gcs) {
   enq_listbuild(c);
 }
 
-void enq_test_update(dml_ctx *c, int gcs) {
+// begin_ov: the overlap rounds follow
+void enq_test_update(dml_ctx *c, int gcs, int begin_ov = 0) {
   hipLaunchKernelGGL(k_pbc_dispmax, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d);
-  hipLaunchKernelGGL(k_dispmax_final, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d);
+  hipLaunchKernelGGL(k_dispmax_final, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d, begin_ov);
   enq_cells_lists(c, gcs);
 }
 
@@ -496,71 +506,58 @@ void enq_forces(dml_ctx *c, int fuse_b, int only_ermak) {
     hipLaunchKernelGGL(k_ermak_b, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d, 1);
 }
 
-void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int rounds,
+// begun: the test_update before has started the rounds (k_dispmax_final)
+void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int rounds, int begun,
                         int err_if_pending) {
-  hipLaunchKernelGGL(k_ov_begin, dim3(1), dim3(64), 0, c->st, c->d);
-  // rounds from ov_tail on run in one workgroup, one launch (their lists
-  // are short; most of them are empty, and an empty round costs three
-  // launches otherwise)
-  const int grid_rounds = c->ov_tail > 0 && rounds > c->ov_tail ? c->ov_tail : rounds;
+  if (!begun)
+    hipLaunchKernelGGL(k_ov_begin, dim3((std::max(c->nrep, 3) + 63) / 64), dim3(64), 0, c->st,
+                       c->d);
+  // rounds from `tail` on run in one workgroup, one launch (their lists are
+  // short; most of them are empty).  Ermak moves ~0.06 A a step, its lists are
+  // short from round 3 on (100,000 particles: from 3 294 us a step, from 8
+  // 307, from 2 616); Brownian moves ~4 A and its lists shrink slowly (100,000
+  // particles: from 8 608 us, from 6 669; 12,000: from 6 308, from 3 605)
+  const int tail = c->ov_tail >= 0  ? c->ov_tail
+                   : !c->any_brown  ? (c->P <= 300000 ? 3 : 4)
+                   : c->P <= 2048   ? 3
+                   : c->P <= 24576  ? 6
+                                    : 8;
+  const int grid_rounds = tail > 0 && rounds > tail ? tail : rounds;
+  // lanes per atom.  Round 0 mostly visits the few listed entries within rcut
+  // (the tuned lanes; untuned 8, and 2 from 300,000 atoms on: 24 replicas 1,522
+  // -> 1,446 us a step).  Later rounds scan whole rows: few atoms wait on
+  // their rows' loads, so many lanes (rounds 1 and 2 at 32, 16 and 8: Brownian
+  // 4,000 particles 272, 277, 286 us, Ermak 100,000 292, 295, 306), but 8
+  // where a Brownian system keeps tens of thousands in the list (100,000: 656,
+  // 638, 608); from round 4 on 64 (Brownian 100,000 608 -> 582, 12,000 314 -> 297)
+  const int lanes0 = c->ov_lanes_set || live_slots(c) < 300000 ? c->lpa_ov : 2;
+  const int lanes12 = !c->any_brown || c->P <= 32768 ? 32 : 8;
   for (int q = 0; q < grid_rounds; q++) {
-    // round 0 mostly visits the few listed entries within rcut (the tuned
-    // lanes, often 1); later rounds scan whole rows, with at least 2 lanes,
-    // and from round 3 on, whose few atoms wait on their rows' loads, at
-    // least 4 (C3 +1.6 %; 8 gained nothing)
-    const int lpa = q == 0 ? c->lpa_ov : std::max(c->lpa_ov, q >= 3 ? 4 : 2);
-    // round 0 covers every ref position; later rounds walk their work lists
-    // (grid-stride, a bounded grid)
-    unsigned gs = (unsigned)(c->P * lpa / DML_BLOCK);
-    const unsigned chunk = DML_BLOCK * OVA_PER;
-    unsigned ga = (unsigned)((c->P + chunk - 1) / chunk);
-    unsigned gr = (unsigned)(c->P / DML_BLOCK);
-    if (q > 0) {
-      gs = std::min(gs, 4096u * (unsigned)lpa);
-      ga = std::min(ga, 2048u);
-      gr = std::min(gr, 4096u);
-    }
+    const int lpa = q == 0 ? lanes0 : std::max(c->lpa_ov, q <= 2 ? lanes12 : q == 3 ? 16 : 64);
+    // a bounded grid: each workgroup appends to the next list with one atomic
+    const unsigned g = (unsigned)std::min<int64_t>(c->P * lpa / DML_BLOCK, 2048);
     switch (lpa) {
-      case 1:
-        hipLaunchKernelGGL(k_ov_scan_l<1>, dim3(gs), dim3(DML_BLOCK), 0, c->st, c->d, u_round,
-                           stride, q, c->P);
-        break;
-      case 2:
-        hipLaunchKernelGGL(k_ov_scan_l<2>, dim3(gs), dim3(DML_BLOCK), 0, c->st, c->d, u_round,
-                           stride, q, c->P);
-        break;
-      case 4:
-        hipLaunchKernelGGL(k_ov_scan_l<4>, dim3(gs), dim3(DML_BLOCK), 0, c->st, c->d, u_round,
-                           stride, q, c->P);
-        break;
-      case 16:
-        hipLaunchKernelGGL(k_ov_scan_l<16>, dim3(gs), dim3(DML_BLOCK), 0, c->st, c->d, u_round,
-                           stride, q, c->P);
-        break;
-      default:
-        hipLaunchKernelGGL(k_ov_scan_l<8>, dim3(gs), dim3(DML_BLOCK), 0, c->st, c->d, u_round,
-                           stride, q, c->P);
-        break;
+#define DML_OV_CASE(L)                                                                          \
+  hipLaunchKernelGGL(k_ov_round<L>, dim3(g), dim3(DML_BLOCK), 0, c->st, c->d, u_round, stride, q, \
+                     c->P);                                                                     \
+  break;
+      case 1: DML_OV_CASE(1)
+      case 2: DML_OV_CASE(2)
+      case 4: DML_OV_CASE(4)
+      case 16: DML_OV_CASE(16)
+      case 32: DML_OV_CASE(32)
+      case 64: DML_OV_CASE(64)
+      default: DML_OV_CASE(8)
+#undef DML_OV_CASE
     }
-    hipLaunchKernelGGL(k_ov_apply, dim3(ga), dim3(DML_BLOCK), 0, c->st, c->d, q, c->P);
-    hipLaunchKernelGGL(k_ov_apply_r, dim3(q == 0 ? std::min(gr, 64u) : gr), dim3(DML_BLOCK), 0,
-                       c->st, c->d, q);
   }
   if (grid_rounds < rounds) {
-    const int lpa = std::max(c->lpa_ov, 4);
-    if (lpa >= 16)
-      hipLaunchKernelGGL(k_ov_tail<16>, dim3(1), dim3(DML_BLOCK), 0, c->st, c->d, u_round, stride,
-                         grid_rounds, rounds, c->P);
-    else if (lpa == 8)
-      hipLaunchKernelGGL(k_ov_tail<8>, dim3(1), dim3(DML_BLOCK), 0, c->st, c->d, u_round, stride,
-                         grid_rounds, rounds, c->P);
-    else
-      hipLaunchKernelGGL(k_ov_tail<4>, dim3(1), dim3(DML_BLOCK), 0, c->st, c->d, u_round, stride,
-                         grid_rounds, rounds, c->P);
+    hipLaunchKernelGGL(k_ov_tail<64>, dim3(1), dim3(OVT_BLOCK), 0, c->st, c->d, u_round, stride,
+                       grid_rounds, rounds, c->P);
   }
-  hipLaunchKernelGGL(k_ov_end, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d, rounds,
-                     err_if_pending);
-  hipLaunchKernelGGL(k_ov_close, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d, rounds);
+  hipLaunchKernelGGL(k_ov_finish, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d, rounds);
+  if (err_if_pending)
+    hipLaunchKernelGGL(k_ov_end, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d, rounds);
 }
 
 // the reference's order: the entries each atom can meet, then the walk
@@ -574,7 +571,7 @@ void enq_overlap_exact(dml_ctx *c, const double *u, int64_t n_u, int max_passes)
 
 void enq_overlap(dml_ctx *c) {
   if (c->any_exact) enq_overlap_exact(c, nullptr, 0, 100000);
-  if (c->any_rounds) enq_overlap_rounds(c, nullptr, 0, c->rounds, 0);
+  if (c->any_rounds) enq_overlap_rounds(c, nullptr, 0, c->rounds, 1, 0);
 }
 
 // gcmc_run (dana.F90:590-713) of one replica (rep_only >= 0, with act and
@@ -665,7 +662,7 @@ void enq_step(dml_ctx *c) {
                        (const double *)nullptr, (const double *)nullptr);
   // the cells of a GCMC replica are needed by its trials, after the second
   // test_update; the first re-sorts them only when it rebuilds the lists
-  enq_test_update(c, 0);
+  enq_test_update(c, 0, c->any_rounds);
   enq_overlap(c);
   enq_test_update(c, 1);
   enq_f2cg(c);
@@ -929,8 +926,8 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   e |= dalloc(&d.ref_pos, P);
   e |= dalloc(&d.nn, P);
   e |= dalloc(&d.nbr, P * (int64_t)maxnn);
-  e |= dalloc(&d.ov_rev, P);
-  e |= dalloc(&d.ov_st, P);
+  e |= dalloc(&d.ovq[0], P);
+  e |= dalloc(&d.ovq[1], P);
   e |= dalloc(&d.ov_near, P);
   e |= dalloc(&d.nearl, P * (int64_t)NEAR_MAX);
   e |= dalloc(&d.part_d, 2 * (P / DML_BLOCK));
@@ -950,9 +947,7 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   e |= dalloc(&d.wl_cnt, 4);
   e |= dalloc(&d.ovw[0], P);
   e |= dalloc(&d.ovw[1], P);
-  e |= dalloc(&d.ovr[0], P);
-  e |= dalloc(&d.ovr[1], P);
-  e |= dalloc(&d.ov_more, 3 * nrep);
+  e |= dalloc(&d.ov_last, nrep);
   e |= dalloc(&d.pf4, P);
   e |= dalloc(&d.gc_order, P);
   e |= dalloc(&d.b2slot, P);
@@ -998,8 +993,8 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   hipMemsetAsync(d.flags, 0, P, c->st);
   hipMemsetAsync(d.rowflag, 0, P, c->st);
   hipMemsetAsync(d.nn, 0, sizeof(int32_t) * P, c->st);
-  hipMemsetAsync(d.ov_rev, 0, sizeof(int32_t) * P, c->st);
-  hipMemsetAsync(d.ov_st, 0, P, c->st);
+  hipMemsetAsync(d.ovq[0], 0, sizeof(int32_t) * P, c->st);
+  hipMemsetAsync(d.ovq[1], 0, sizeof(int32_t) * P, c->st);
   hipMemsetAsync(d.ov_near, 0xff, P, c->st);  // 255: no entries listed
   hipMemsetAsync(d.wl_cnt, 0, sizeof(int32_t) * 4, c->st);
   hipMemsetAsync(d.pf4, 0, sizeof(float4) * P, c->st);
@@ -1024,7 +1019,10 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   if (const char *ev = getenv("DML_OV_TAIL")) c->ov_tail = std::max(0, atoi(ev));
   if (const char *ev = getenv("DML_OVERLAP_LPA")) {
     const int v = atoi(ev);
-    if (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) c->lpa_ov = v;
+    if (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) {
+      c->lpa_ov = v;
+      c->ov_lanes_set = 1;
+    }
   }
 
   refresh_modes(c);
@@ -1045,9 +1043,9 @@ int dml_destroy(dml_ctx *c) {
   void *ptrs[] = {d.px, d.py, d.pz, d.vx, d.vy, d.vz, d.ax, d.ay, d.az, d.fx, d.fy, d.fz,
                   d.epot, d.ox, d.oy, d.oz, d.cx, d.cy, d.cz, d.rvx, d.rvy, d.rvz,
                   d.species, d.flags, d.rowflag, d.bkey, d.pid, d.ref_order, d.ref_tmp,
-                  d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ov_rev,
-                  d.ov_st, d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
-                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ovr[0], d.ovr[1], d.ov_more, d.ovx_n, d.ovx_l, d.ovx_m, d.pf4, d.bf4, d.gc_order,
+                  d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ovq[0],
+                  d.ovq[1], d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
+                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ov_last, d.ovx_n, d.ovx_l, d.ovx_m, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
                   d.cm_rep, d.cm_cell, d.cm_nref, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
                   d.gb_pt, d.gb_u, d.gb_du, d.gb_g, d.gb_kind, d.gb_cell, d.gb_nblk, d.gb_blk,
@@ -1124,8 +1122,7 @@ int dml_set_state(dml_ctx *c, int32_t rep, int32_t n, const double *pos, const d
   HIPCHECK(hipMemset(c->d.nn + o, 0, sizeof(int32_t) * p.pcap));
   // a reused replica (serving) starts like a fresh one: no overlap stamps,
   // no flags beyond n, zero forces
-  HIPCHECK(hipMemset(c->d.ov_rev + o, 0, sizeof(int32_t) * p.pcap));
-  HIPCHECK(hipMemset(c->d.ov_st + o, 0, p.pcap));
+  for (int32_t *q : c->d.ovq) HIPCHECK(hipMemset(q + o, 0, sizeof(int32_t) * p.pcap));
   HIPCHECK(hipMemset(c->d.rowflag + o, 0, p.pcap));
   if (p.pcap > n) HIPCHECK(hipMemset(c->d.flags + o + n, 0, p.pcap - n));
   {
@@ -1478,7 +1475,7 @@ int dml_overlap_moveback(dml_ctx *c, const double *u_contact, int64_t n_u, int32
 int dml_overlap_rounds(dml_ctx *c, const double *u_round, int32_t max_rounds) {
   if (!c || max_rounds <= 0 || max_rounds > kMaxRounds) return DML_E_ARG;
   double *du = u_round ? upload_tmp(c, u_round, (int64_t)max_rounds * c->P) : nullptr;
-  enq_overlap_rounds(c, du, c->P, max_rounds, 1);
+  enq_overlap_rounds(c, du, c->P, max_rounds, 0, 1);
   int rc = finish(c);
   hipFree(du);
   return rc;
@@ -1839,7 +1836,8 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
                         c->any_exact << 3 | c->any_piston << 4 | c->any_gcmc << 5 |
                         (int64_t)c->any_chunks << 31 |
                         (int64_t)c->rounds << 6 | (int64_t)c->lpa << 12 |
-                        (int64_t)c->lpa_ov << 19 | (int64_t)c->lb_mode << 26 |
+                        (int64_t)c->lpa_ov << 19 | (int64_t)c->ov_lanes_set << 52 |
+                        (int64_t)(live_slots(c) < 300000) << 53 | (int64_t)c->lb_mode << 26 |
                         (int64_t)c->any_lb[0] << 32 | (int64_t)c->any_lb[1] << 33 |
                         (int64_t)c->any_lb[2] << 34 | (int64_t)c->any_lb[3] << 35;
   // a captured step holds the device state by value: any reallocation or
@@ -1937,7 +1935,10 @@ int dml_set_tuning(dml_ctx *c, int32_t lanes_per_atom, int32_t overlap_rounds,
     return DML_E_ARG;
   if (lanes_per_atom) c->lpa = lanes_per_atom;
   if (overlap_rounds) c->rounds = overlap_rounds;
-  if (overlap_lanes) c->lpa_ov = overlap_lanes;
+  if (overlap_lanes) {
+    c->lpa_ov = overlap_lanes;
+    c->ov_lanes_set = 1;
+  }
   if (list_kernel) {
     c->lb_mode = list_kernel - 1;
     int rc = fetch_params(c);

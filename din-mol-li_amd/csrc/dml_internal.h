@@ -16,7 +16,9 @@
 #include "../../include/dml.h"
 
 #define DML_BLOCK 256
-#define OVA_PER 8  // items per thread of one k_ov_apply block pass
+#define OV_STAMPS 40  // work-list stamps per overlap call (more than its rounds)
+#define OVB_MAX 2048  // list entries a workgroup of an overlap round collects in LDS
+#define OVT_BLOCK 512 // threads of the overlap tail
 #define OVX_MAX 16  // row entries listed per atom for the reference-order overlap pass
 #define OVX_BLOCK 1024
 #define NEAR_MAX 4  // row positions within rcut listed per atom by the row build
@@ -299,18 +301,16 @@ struct DevState {
   int32_t *bucket;        // slots, bucket-ordered
   double *bx, *by, *bz;   // positions, bucket-ordered
   // overlap rounds
-  int32_t *ov_rev;        // round stamp of a revert
-  uint8_t *ov_st;         // bit0 active bit1 dominated bit2 deposit bit3 self-revert
+  int32_t *ovq[2];        // stamp of the (even, odd) round an atom was last listed for
   uint8_t *ov_near;       // row entries within rcut (FP32, with margin) listed in
                           // nearl by fuerza or the row build (255: not listed)
   int32_t *nearl;         // NEAR_MAX row positions per atom
-  int32_t *wl[2];         // overlap worklists (global ref positions), by round parity
+  int32_t *wl[2];         // per-slot scratch (compactions, a GCMC call's working list)
   // overlap rounds after the first visit only their work lists: ovw[q % 2]
-  // the ref positions still unresolved (skip = 0) for round q, ovr[q % 2]
-  // the atoms reverted in round q; wl_cnt = [|ovw0|, |ovw1|, |ovr0|, |ovr1|]
+  // the ref positions to look at in round q, wl_cnt[q % 3] their number
   int32_t *wl_cnt;
-  int32_t *ovw[2], *ovr[2];
-  int32_t *ov_more;       // [3][nrep]: the replica reverted or deferred in a round
+  int32_t *ovw[2];
+  int32_t *ov_last;       // [nrep]: last round in which the replica reverted or deferred
   // reference-order overlap pass (only with such a replica): per ref position
   // the row entries it can meet (count, 255 = more than listed), and the
   // masks of positions to visit of replicas too large for LDS

@@ -3,7 +3,7 @@
 #include "dml_internal.h"
 
 __global__ void k_pbc_dispmax(DevState s);
-__global__ void k_dispmax_final(DevState s);
+__global__ void k_dispmax_final(DevState s, int begin);
 __global__ void k_init_pf4(DevState s, int64_t n);
 __global__ void k_force_rebuild(DevState s);
 __global__ void k_zero_cells(DevState s, int gcs);
@@ -12,8 +12,8 @@ __global__ void k_cell_sort(DevState s, int gcs);
 __global__ void k_cell_sort_w(DevState s, int gcs);
 __global__ void k_listbuild_cells(DevState s);
 template <int LPA>
-__global__ void k_ov_scan_l(DevState s, const double *u_round, int64_t u_stride, int round,
-                            int64_t ptotal);
+__global__ void k_ov_round(DevState s, const double *u_round, int64_t u_stride, int round,
+                           int64_t ptotal);
 template <int WPB>
 __global__ void k_listbuild(DevState s);
 template <int LPA, int FUSEB>
@@ -26,13 +26,11 @@ template <int LPA>
 __global__ void k_ov_contacts(DevState s);
 __global__ void k_ov_exact(DevState s, const double *u, int64_t n_u, int max_passes);
 __global__ void k_ov_begin(DevState s);
-__global__ void k_ov_apply_r(DevState s, int round);
-__global__ void k_ov_apply(DevState s, int round, int64_t ptotal);
 template <int LPA>
 __global__ void k_ov_tail(DevState s, const double *u_round, int64_t u_stride, int r0, int r1,
                           int64_t ptotal);
-__global__ void k_ov_end(DevState s, int rounds, int err_if_pending);
-__global__ void k_ov_close(DevState s, int rounds);
+__global__ void k_ov_finish(DevState s, int rounds);
+__global__ void k_ov_end(DevState s, int rounds);
 __global__ void k_zero_i32(int32_t *a, int64_t n);
 __global__ void k_f2cg_mark(DevState s);
 __global__ void k_f2cg_scan(DevState s);

@@ -127,12 +127,23 @@ __global__ void __launch_bounds__(DML_BLOCK) k_pbc_dispmax(DevState s) {
   }
 }
 
+// before the first overlap round: stamps past every earlier call's, no round with progress
+__device__ inline void ov_begin_rep(const DevState &s, int r) {
+  s.rp[r].ov_round += OV_STAMPS;
+  s.ov_last[r] = -1;
+}
+
 // one block per replica merges the block partials (a kernel boundary orders
 // them; no device-scope fences, which on this part write back per-XCD L2)
-__global__ void __launch_bounds__(DML_BLOCK) k_dispmax_final(DevState s) {
+// begin: also start the overlap rounds that follow (k_ov_begin)
+__global__ void __launch_bounds__(DML_BLOCK) k_dispmax_final(DevState s, int begin) {
   __shared__ double sh[2 * DML_BLOCK / WAVE];
   const int r = blockIdx.x;
   RepParams *Pw = s.rp + r;
+  if (begin && threadIdx.x == 0) {
+    ov_begin_rep(s, r);
+    if (r == 0) s.wl_cnt[0] = s.wl_cnt[1] = s.wl_cnt[2] = 0;
+  }
   if (Pw->halted) return;
   const int b0 = Pw->poff / DML_BLOCK, nb = Pw->pcap / DML_BLOCK;
   double a1 = -1.0, a2 = -1.0;
@@ -2121,40 +2132,72 @@ __global__ void __launch_bounds__(OVX_BLOCK) k_ov_exact(DevState s, const double
 }
 
 // deterministic parallel rounds (this build's schedule; orc.c
-// orc_overlap_rounds is its specification).  Round 0 covers every ref
-// position; round r > 0 covers the worklist of atoms left with skip = 0 by
-// round r-1, plus the atoms reverted in round r.  Worklist entries are global
-// ref positions, deduplicated by a per-slot round stamp.
-__device__ inline int ov_stamp(const RepParams &P, int round) { return P.ov_round + round + 1; }
+// orc_overlap_rounds is its specification), one launch a round.  Round 0
+// covers every ref position; a later round the atoms the round before left
+// unresolved or reverted, each once (ovq stamps), from a work list.
+//
+// A round sees the positions and marks of its start, and nothing it finds is
+// applied before the last round: an atom has only two positions in a call,
+// the current one and old_cg, and pf4's species word says from which round on
+// it is at the second (bits 8-15: the round after the first revert; bit 16:
+// reverted by a neighbour, which also stops it; 0 outside the call).  Whether
+// an atom is unresolved in a round is its stamp for that round.  px, vx and
+// the flags stay as they are until k_ov_finish writes them, once per atom.
+// (With an apply pass over the lists after every scan a round took three
+// launches: 283 us of a 100,000-particle Ermak step and 575 us of a Brownian
+// one, an apply pass of the first round alone 32 us.)
+#define OVW_AT(w) ((w) >> 8 & 0xff)
+#define OVW_HIT 0x10000
+__device__ inline bool ov_moved(int w, int round) { return OVW_AT(w) != 0 && OVW_AT(w) <= round; }
 
 __global__ void k_ov_begin(DevState s) {
-  int q = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int k = q; k < 3 * s.nrep; k += gridDim.x * blockDim.x) s.ov_more[k] = 0;
-  if (q == 0) s.wl_cnt[2] = 0;  // round 0's list of reverted atoms outside ref
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < s.nrep) ov_begin_rep(s, q);
+  if (q < 3) s.wl_cnt[q] = 0;
 }
 
-// one round's scan as workgroup bid of nbk (k_ov_scan_l: the whole grid;
-// k_ov_tail: one workgroup)
+// one round as workgroup bid of nbk (k_ov_round: the whole grid; k_ov_tail:
+// one workgroup)
 template <int LPA>
-__device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_round,
-                                             int64_t u_stride, int round, int64_t ptotal,
-                                             int bid, int nbk) {
-  // progress flags rotate over three buffers: this round writes round % 3,
-  // is gated by (round - 1) % 3, and clears (round + 1) % 3 for the next one
-  const int cur = round % 3, prv = (round + 2) % 3, nxt = (round + 1) % 3;
-  if (bid == 0) {
-    for (int q = threadIdx.x; q < s.nrep; q += DML_BLOCK) s.ov_more[nxt * s.nrep + q] = 0;
-    if (threadIdx.x == 0) s.wl_cnt[(round + 1) % 2] = 0;  // the next round's list
-  }
-  // round 0: every ref position; later rounds: the positions left unresolved
-  // (lists hold at most ptotal entries, each a position below ptotal)
-  const int64_t nitems =
-      round == 0 ? ptotal : min((int64_t)s.wl_cnt[round % 2], ptotal);
+__device__ __forceinline__ void ov_round_body(const DevState &s, const double *u_round,
+                                              int64_t u_stride, int round, int64_t ptotal,
+                                              int bid, int nbk) {
+  // this workgroup's entries of the next round's list, appended at its end
+  // with one atomic (atomics on the list's counter are done one by one
+  // across the chip)
+  __shared__ int32_t buf[OVB_MAX];
+  __shared__ int buf_n, buf_at;
+  const int nt = (int)blockDim.x;
+  if (threadIdx.x == 0) buf_n = 0;
+  // lists alternate, their counters take three turns: read, appended to,
+  // cleared for the round after next
+  if (bid == 0 && threadIdx.x == 0) s.wl_cnt[(round + 2) % 3] = 0;
+  __syncthreads();
+  const int64_t nitems = round == 0 ? ptotal : min((int64_t)s.wl_cnt[round % 3], ptotal);
   const int32_t *wl = s.ovw[round % 2];
-  const int gtid = bid * DML_BLOCK + threadIdx.x;
+  int32_t *next = s.ovw[(round + 1) % 2];
+  int32_t *now_q = s.ovq[round % 2], *next_q = s.ovq[(round + 1) % 2];
+  const int gtid = bid * nt + threadIdx.x;
   const int sub = gtid % LPA;
-  const int64_t stride = (int64_t)nbk * (DML_BLOCK / LPA);
+  const int64_t stride = (int64_t)nbk * (nt / LPA);
   const int wv = gtid / WAVE;  // counter shard
+  // atom j (ref position t) is to be looked at in the next round
+  auto queue = [&](const RepParams &P, int j, int t) {
+    const int stamp = P.ov_round + round + 1;
+    if (atomicExch(&next_q[j], stamp) == stamp) return;  // it is listed
+    const int q = atomicAdd(&buf_n, 1);
+    if (q < OVB_MAX) {
+      buf[q] = t;
+    } else {
+      const int g = atomicAdd(&s.wl_cnt[(round + 1) % 3], 1);
+      if (g < ptotal) next[g] = t;
+    }
+  };
+  // atom j sits at old_cg from the next round on
+  auto put_back = [&](int j, int w, int hit) {
+    const int bits = hit | (OVW_AT(w) ? 0 : (round + 1) << 8);
+    if ((w & bits) != bits) atomicOr(reinterpret_cast<int *>(&s.pf4[j]) + 3, bits);
+  };
   // one ref position: its verdict, and what it adds to its replica's
   // counters (k_r = the replica, -1 when the position is not scanned)
   auto scan_one = [&](int64_t item, int &k_try, int &k_ch, int &k_ch3, int &k_more, int &k_r) {
@@ -2164,42 +2207,53 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
     const RepParams &P = s.rp[r];
     if (P.halted || P.overlap_mode != DML_OVERLAP_ROUNDS) return;
     // the sequential pass recurses only after a revert or a deferred atom
-    if (round > 0 && !s.ov_more[prv * s.nrep + r]) return;
+    if (round > 0 && s.ov_last[r] < round - 1) return;
     const int local = t - P.poff;
     if (local >= P.nref) return;
     const int i = s.ref_order[t];
-    if (s.flags[i] & DML_FL_SKIP) {
-      if (sub == 0) s.ov_st[i] = 0;
-      return;
-    }
+    if (round == 0 && (s.flags[i] & DML_FL_SKIP)) return;
     // fuerza or the row build of this step, at these same positions and on
     // this same row, listed the row positions of the entries within rcut
     // (FP32 with margin): every other entry lies beyond rcut.  None listed:
     // no contact, no neighbour to revert and no earlier atom to wait for
     int nlist = round == 0 && P.ovn_stamp == P.step + 1 ? s.ov_near[i] : 255;
-    if (nlist == 0) {
-      if (sub == 0) s.ov_st[i] = 1;
-      return;
+    if (nlist == 0) return;
+    float4 fi = s.pf4[i];
+    const int wi = __float_as_int(fi.w);
+    const bool back_i = ov_moved(wi, round);
+    const double xi = back_i ? s.cx[i] : s.px[i], yi = back_i ? s.cy[i] : s.py[i],
+                 zi = back_i ? s.cz[i] : s.pz[i];
+    if (back_i) {
+      fi.x = (float)xi;
+      fi.y = (float)yi;
+      fi.z = (float)zi;
     }
-    const double xi = s.px[i], yi = s.py[i], zi = s.pz[i];
-    const float4 fi = s.pf4[i];
     const float bxf = (float)P.box[0], byf = (float)P.box[1];
     const float ibx = (float)P.one_box[0], iby = (float)P.one_box[1];
     const float rcf = (float)P.rcut2 + P.pf_margin;
+    const int now = P.ov_round + round;  // the stamp of the atoms of this round
     const int nn = s.nn[i];
     const int32_t *row = s.nbr + (int64_t)i * s.maxnn;
     // up to four non-CG hits per lane kept in registers (named, so that no
     // private array is needed), more fall back to a second pass
     int hj0 = 0, hj1 = 0, hj2 = 0, hj3 = 0, he0 = 0, he1 = 0, he2 = 0, he3 = 0;
     int nh = 0, over = 0, dom = 0, firstcg = 0x7fffffff;
-    // row entry e (neighbour j) within rcut in FP64
-    auto visit = [&](int e, int j) {
+    // within rcut of neighbour j (its species word w) in FP64
+    auto near = [&](int j, int w) -> bool {
+      double dx, dy, dz;
+      if (ov_moved(w, round))
+        vdist_mic(P, xi, yi, zi, s.cx[j], s.cy[j], s.cz[j], &dx, &dy, &dz);
+      else
+        vdist_mic(P, xi, yi, zi, s.px[j], s.py[j], s.pz[j], &dx, &dy, &dz);
+      return !(dot3(dx, dy, dz) > P.rcut2);
+    };
+    // row entry e (neighbour j)
+    auto visit = [&](int e, int j, int w) {
       uint8_t fj = s.flags[j];
       if (fj & DML_FL_LIMBO) return;
-      double dx, dy, dz;
-      vdist_mic(P, xi, yi, zi, s.px[j], s.py[j], s.pz[j], &dx, &dy, &dz);
-      if (dot3(dx, dy, dz) > P.rcut2) return;
-      if ((fj & DML_FL_REF) && !(fj & DML_FL_SKIP)) {
+      if (!near(j, w)) return;
+      if ((fj & DML_FL_REF) &&
+          (round == 0 ? !(fj & DML_FL_SKIP) : now_q[j] == now)) {
         const int pj = s.ref_pos[j];
         if (pj >= 0 && pj < local) dom = 1;
       }
@@ -2229,13 +2283,20 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
     if (nlist <= NEAR_MAX) {
       for (int k = sub; k < nlist; k += LPA) {
         const int e = nl[k];
-        visit(e, row[e]);
+        visit(e, row[e], 0);  // (round 0: every atom at its current position)
       }
     } else {
       for (int e = sub; e < nn; e += LPA) {
-        int j = row[e];
-        if (d2_f32(P, fi, s.pf4[j], bxf, byf, ibx, iby) > rcf) continue;  // surely no hit
-        visit(e, j);
+        const int j = row[e];
+        float4 fj = s.pf4[j];
+        const int w = __float_as_int(fj.w);
+        if (ov_moved(w, round)) {
+          fj.x = (float)s.cx[j];
+          fj.y = (float)s.cy[j];
+          fj.z = (float)s.cz[j];
+        }
+        if (d2_f32(P, fi, fj, bxf, byf, ibx, iby) > rcf) continue;  // surely no hit
+        visit(e, j, w);
       }
     }
     for (int off = LPA / 2; off > 0; off >>= 1) {
@@ -2245,25 +2306,16 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
       firstcg = o < firstcg ? o : firstcg;
     }
     int n_ch = 0, n_ch3 = 0;  // reverts of this atom: at most its row length
-    const int stamp = ov_stamp(P, round);
+    const bool same_i = back_i || same_pos(s, i);
     // a revert of neighbour j (or, piston, the "unsolvable" count when
     // both sit where they were, dana.F90:920-927); returns 1 for the latter.
     // Counted by the callers with arithmetic, keeping the counters in registers
     auto revert = [&](int j) -> int {
-      if (P.piston && same_pos(s, j) && same_pos(s, i)) return 1;
-      if (round == 0 && (s.flags[j] & DML_FL_REF) && s.ref_pos[j] >= 0) {
-        s.ov_rev[j] = stamp;  // k_ov_apply walks every ref position in round 0
-      } else if (atomicExch(&s.ov_rev[j], stamp) != stamp) {
-        // first to revert j in this round: it is applied from the list
-        // (one atomic for the lanes that are here together)
-        const unsigned long long m = __ballot(1);
-        const int lead = __builtin_ctzll(m);
-        int q = 0;
-        if ((int)(threadIdx.x % WAVE) == lead) q = atomicAdd(&s.wl_cnt[2 + round % 2], __popcll(m));
-        q = __shfl(q, lead) + (int)__builtin_amdgcn_mbcnt_hi(
-                                  (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        if (q < ptotal) s.ovr[round % 2][q] = j;
-      }
+      const int w = __float_as_int(s.pf4[j].w);
+      if (P.piston && same_i && (ov_moved(w, round) || same_pos(s, j))) return 1;
+      put_back(j, w, OVW_HIT);
+      const int tj = s.ref_pos[j];
+      if ((s.flags[j] & DML_FL_REF) && tj >= 0) queue(P, j, P.poff + tj);
       return 0;
     };
     if (!dom) {
@@ -2276,9 +2328,7 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
         for (int e = sub; e < nn && e < firstcg; e += LPA) {
           int j = row[e];
           if (s.flags[j] & DML_FL_LIMBO) continue;
-          double dx, dy, dz;
-          vdist_mic(P, xi, yi, zi, s.px[j], s.py[j], s.pz[j], &dx, &dy, &dz);
-          if (dot3(dx, dy, dz) > P.rcut2 || s.species[j] == SP_CG) continue;
+          if (!near(j, __float_as_int(s.pf4[j].w)) || s.species[j] == SP_CG) continue;
           const int c3 = revert(j);
           n_ch3 += c3;
           n_ch += 1 - c3;
@@ -2290,22 +2340,30 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
       n_ch3 += lpa_xor<LPA>(n_ch3, off);
     }
     if (sub == 0) {
-      uint8_t st = 1;
       if (dom) {
-        st |= 2;
+        queue(P, i, t);
       } else if (firstcg != 0x7fffffff) {
         k_try = 1;
         double ne;
         if (u_round) {
           ne = u_round[(int64_t)round * u_stride + i];
         } else {
-          u32x4 wv = dml_philox(P.seed, s.pid[i], (uint32_t)P.step, RS_CONTACT,
-                                (uint32_t)(1000 + round));
-          ne = u01_from(wv.x, wv.y);
+          u32x4 wv4 = dml_philox(P.seed, s.pid[i], (uint32_t)P.step, RS_CONTACT,
+                                 (uint32_t)(1000 + round));
+          ne = u01_from(wv4.x, wv4.y);
         }
-        st |= (ne < P.prob) ? 4 : 8;
+        if (ne < P.prob) {
+          // (Li and F only: neither is the CG that a neighbour looks for)
+          atomicAdd(&cnt_of(s, r, wv).depo, 1ull);
+          s.species[i] = SP_F;
+          atomicOr(reinterpret_cast<int *>(&s.pf4[i]) + 3, SP_F);
+          s.rp[r].any_f = 1;
+          if (zi > P.z0) rep_fail(s, r, ERR_DEPZ0);
+        } else {
+          put_back(i, wi, 0);
+          queue(P, i, t);
+        }
       }
-      s.ov_st[i] = st;
       k_ch = n_ch;
       k_ch3 = n_ch3;
       // a revert or a dominated atom: the sequential pass would recurse
@@ -2317,10 +2375,8 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
   // can be summed over the wave: one atomic per wave and counter when the
   // wave's items belong to one replica (always in round 0, whose items are
   // consecutive positions of one 256-slot block; mostly later, the work
-  // lists being appended block by block), one per atom otherwise.  The
-  // counters of a replica are single addresses, which serialise across the
-  // chip when every atom adds to them.
-  for (int64_t it0 = (int64_t)bid * (DML_BLOCK / LPA); it0 < nitems; it0 += stride) {
+  // lists being appended block by block), one per atom otherwise.
+  for (int64_t it0 = (int64_t)bid * (nt / LPA); it0 < nitems; it0 += stride) {
     const int64_t item = it0 + threadIdx.x / LPA;
     int k_try = 0, k_ch = 0, k_ch3 = 0, k_more = 0, k_r = -1;
     if (item < nitems) scan_one(item, k_try, k_ch, k_ch3, k_more, k_r);
@@ -2337,199 +2393,98 @@ __device__ __forceinline__ void ov_scan_body(const DevState &s, const double *u_
         if (t_try) atomicAdd(&cnt_of(s, r0, wv).try_, (unsigned long long)(uint32_t)t_try);
         if (t_ch) atomicAdd(&cnt_of(s, r0, wv).choques, (unsigned long long)(uint32_t)t_ch);
         if (t_ch3) atomicAdd(&cnt_of(s, r0, wv).choques3, (unsigned long long)(uint32_t)t_ch3);
-        if (more) s.ov_more[cur * s.nrep + r0] = 1;
+        if (more) s.ov_last[r0] = round;
       }
     } else if (k_r >= 0) {
       if (k_try) atomicAdd(&cnt_of(s, k_r, wv).try_, (unsigned long long)(uint32_t)k_try);
       if (k_ch) atomicAdd(&cnt_of(s, k_r, wv).choques, (unsigned long long)(uint32_t)k_ch);
       if (k_ch3) atomicAdd(&cnt_of(s, k_r, wv).choques3, (unsigned long long)(uint32_t)k_ch3);
-      if (k_more) s.ov_more[cur * s.nrep + k_r] = 1;
+      if (k_more) s.ov_last[k_r] = round;
     }
   }
+  __syncthreads();
+  const int n = min(buf_n, OVB_MAX);
+  if (threadIdx.x == 0) buf_at = n ? atomicAdd(&s.wl_cnt[(round + 1) % 3], n) : 0;
+  __syncthreads();
+  for (int q = threadIdx.x; q < n; q += nt)
+    if (buf_at + q < ptotal) next[buf_at + q] = buf[q];
 }
 
 template <int LPA>
 __global__ void __launch_bounds__(DML_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
-k_ov_scan_l(DevState s, const double *u_round, int64_t u_stride, int round, int64_t ptotal) {
-  ov_scan_body<LPA>(s, u_round, u_stride, round, ptotal, blockIdx.x, gridDim.x);
+k_ov_round(DevState s, const double *u_round, int64_t u_stride, int round, int64_t ptotal) {
+  ov_round_body<LPA>(s, u_round, u_stride, round, ptotal, blockIdx.x, gridDim.x);
 }
-template __global__ void k_ov_scan_l<1>(DevState, const double *, int64_t, int, int64_t);
-template __global__ void k_ov_scan_l<2>(DevState, const double *, int64_t, int, int64_t);
-template __global__ void k_ov_scan_l<4>(DevState, const double *, int64_t, int, int64_t);
-template __global__ void k_ov_scan_l<8>(DevState, const double *, int64_t, int, int64_t);
-template __global__ void k_ov_scan_l<16>(DevState, const double *, int64_t, int, int64_t);
+#define INST_OV(L) \
+  template __global__ void k_ov_round<L>(DevState, const double *, int64_t, int, int64_t);
+INST_OV(1)
+INST_OV(2)
+INST_OV(4)
+INST_OV(8)
+INST_OV(16)
+INST_OV(32)
+INST_OV(64)
 
-// one atom's outcome of a round (its own verdict st, a revert by a
-// neighbour); returns 1 when the atom belongs in the next round's list
-__device__ inline int ov_apply_one(const DevState &s, int r, const RepParams &P, int i, int t,
-                                   int round) {
-  const uint8_t st = s.ov_st[i];
-  uint8_t f = s.flags[i];
-  int moved = 0;
-  if ((st & 1) && !(st & 2)) f |= DML_FL_SKIP;
-  if (st & 4) {
-    atomicAdd(&cnt_of(s, r, i / WAVE).depo, 1ull);
-    s.species[i] = SP_F;
-    s.rp[r].any_f = 1;
-    moved = 1;
-    if (s.pz[i] > P.z0) rep_fail(s, r, ERR_DEPZ0);
-  }
-  if (st & 8) {
-    s.px[i] = s.cx[i]; s.py[i] = s.cy[i]; s.pz[i] = s.cz[i];
-    f &= (uint8_t)~DML_FL_SKIP;
-    moved = 1;
-  }
-  if (s.ov_rev[i] == ov_stamp(P, round)) {
-    s.ov_rev[i] = 0;  // applied (stamps are positive)
-    s.px[i] = s.cx[i]; s.py[i] = s.cy[i]; s.pz[i] = s.cz[i];
-    s.vx[i] = 0.0; s.vy[i] = 0.0; s.vz[i] = 0.0;
-    s.ax[i] = 0.0; s.ay[i] = 0.0; s.az[i] = 0.0;
-    f &= (uint8_t)~DML_FL_SKIP;
-    moved = 1;
-  }
-  if (st || moved) {
-    s.flags[i] = f;
-    s.ov_st[i] = 0;
-  }
-  if (moved) put_pf4(s, i, s.px[i], s.py[i], s.pz[i], s.species[i]);
-  // the scan of the next round visits this atom when it is unresolved and
-  // its replica goes on (its scan reverted or deferred something)
-  return !(f & DML_FL_SKIP) && t >= P.poff && s.ov_more[(round % 3) * s.nrep + r];
-}
-
-// round 0: every ref position; later rounds: the positions scanned in it.
-// A block takes OVA_PER * DML_BLOCK consecutive items at a time and appends
-// the unresolved ones to the next round's list with one atomic (a per-item
-// or per-wave atomic on the single list counter serialises across the chip);
-// the list order is free, every round's outcome depends on its start state only
-__device__ __forceinline__ void ov_apply_body(const DevState &s, int round, int64_t ptotal,
-                                              int bid, int nbk) {
-  __shared__ int32_t buf[DML_BLOCK * OVA_PER];
-  __shared__ int wcnt[DML_BLOCK / WAVE];
-  __shared__ int64_t base_sh;
-  const int prv = (round + 2) % 3;
-  const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
-  if (bid == 0 && threadIdx.x == 0) s.wl_cnt[2 + (round + 1) % 2] = 0;  // next reverts
-  const int64_t nitems =
-      round == 0 ? ptotal : min((int64_t)s.wl_cnt[round % 2], ptotal);
-  const int32_t *wl = s.ovw[round % 2];
-  int32_t *next = s.ovw[(round + 1) % 2];
-  int32_t *wb = buf + w * WAVE * OVA_PER;
-  const int64_t chunk = (int64_t)DML_BLOCK * OVA_PER;
-  for (int64_t b0 = bid * chunk; b0 < nitems; b0 += (int64_t)nbk * chunk) {
-    int n = 0;  // this wave's appends so far (wave-uniform)
-    for (int k = 0; k < OVA_PER; k++) {
-      const int64_t item = b0 + (int64_t)k * DML_BLOCK + threadIdx.x;
-      int push = 0, t = 0;
-      if (item < nitems) t = round == 0 ? (int)item : wl[item];
-      if (item < nitems && (uint32_t)t < (uint64_t)ptotal) {
-        const int r = s.blk2rep[t / DML_BLOCK];
-        const RepParams &P = s.rp[r];
-        if (!P.halted && P.overlap_mode == DML_OVERLAP_ROUNDS) {
-          if (round == 0 && t == P.poff) s.rp[r].ovn_stamp = 0;  // reverts move atoms
-          // round > 0 and a replica whose scan stopped: nothing to apply
-          if ((round == 0 || s.ov_more[prv * s.nrep + r]) && t - P.poff < P.nref)
-            push = ov_apply_one(s, r, P, s.ref_order[t], t, round);
-        }
-      }
-      const unsigned long long m = __ballot(push);
-      if (push) wb[n + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = t;
-      n += __popcll(m);
-    }
-    if (lane == 0) wcnt[w] = n;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int tot = 0;
-      for (int q = 0; q < DML_BLOCK / WAVE; q++) tot += wcnt[q];
-      base_sh = tot ? (int64_t)atomicAdd(&s.wl_cnt[(round + 1) % 2], tot) : 0;
-    }
-    __syncthreads();
-    int64_t off = base_sh;
-    for (int q = 0; q < w; q++) off += wcnt[q];
-    for (int q = lane; q < n; q += WAVE)
-      if (off + q < ptotal) next[off + q] = wb[q];
-    __syncthreads();  // buf, wcnt and base_sh are reused
-  }
-}
-__global__ void __launch_bounds__(DML_BLOCK) k_ov_apply(DevState s, int round, int64_t ptotal) {
-  ov_apply_body(s, round, ptotal, blockIdx.x, gridDim.x);
-}
-
-// the atoms reverted in a round that k_ov_apply does not reach: in round 0
-// those outside the ref list (it walks every ref position), later the ones
-// the round did not scan (those that were are applied, and their stamp
-// cleared, by k_ov_apply)
-__device__ __forceinline__ void ov_apply_r_body(const DevState &s, int round, int bid, int nbk) {
-  const int64_t cap = (int64_t)s.nblocks * DML_BLOCK;
-  const int64_t nitems = min((int64_t)s.wl_cnt[2 + round % 2], cap);
-  const int32_t *rl = s.ovr[round % 2];
-  const int64_t stride = (int64_t)nbk * DML_BLOCK;
-  for (int64_t item = (int64_t)bid * DML_BLOCK + threadIdx.x; item < nitems; item += stride) {
-    const int j = rl[item];
-    if ((uint32_t)j >= (uint64_t)cap) continue;
-    const int r = s.blk2rep[j / DML_BLOCK];
-    const RepParams &P = s.rp[r];
-    if (P.halted || s.ov_rev[j] != ov_stamp(P, round)) continue;
-    const int t = P.poff + s.ref_pos[j];  // ref_pos is replica-local
-    const int push = ov_apply_one(s, r, P, j, t, round);
-    // one atomic per wave for its appends (the active lanes of this pass)
-    const unsigned long long m = __ballot(push);
-    if (m) {
-      const int lead = __builtin_ctzll(m);
-      int base = 0;
-      if ((int)(threadIdx.x % WAVE) == lead) base = atomicAdd(&s.wl_cnt[(round + 1) % 2], __popcll(m));
-      base = __shfl(base, lead);
-      const int q = base + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-      if (push && q < cap) s.ovw[(round + 1) % 2][q] = t;
-    }
-  }
-}
-__global__ void __launch_bounds__(DML_BLOCK) k_ov_apply_r(DevState s, int round) {
-  ov_apply_r_body(s, round, blockIdx.x, gridDim.x);
-}
-
-// the last rounds, whose work lists are short, in one workgroup: the three
-// phases of each round (scan, apply, apply of the other reverted atoms)
-// separated by the workgroup's barriers instead of kernel boundaries, one
-// launch for all of them instead of three per round.  The same code per
-// phase as the grid-wide kernels, so the same result.
+// the last rounds, whose work lists are short, in one workgroup: a barrier
+// between two rounds instead of a launch; the same code, so the same result
 template <int LPA>
-__global__ void __launch_bounds__(DML_BLOCK) k_ov_tail(DevState s, const double *u_round, int64_t u_stride, int r0, int r1, int64_t ptotal) {
+__global__ void __launch_bounds__(OVT_BLOCK) k_ov_tail(DevState s, const double *u_round,
+                                                       int64_t u_stride, int r0, int r1,
+                                                       int64_t ptotal) {
   for (int q = r0; q < r1; q++) {
-    ov_scan_body<LPA>(s, u_round, u_stride, q, ptotal, 0, 1);
-    __syncthreads();
-    ov_apply_body(s, q, ptotal, 0, 1);
-    __syncthreads();
-    ov_apply_r_body(s, q, 0, 1);
+    ov_round_body<LPA>(s, u_round, u_stride, q, ptotal, 0, 1);
     __syncthreads();
   }
 }
-template __global__ void k_ov_tail<4>(DevState, const double *, int64_t, int, int, int64_t);
-template __global__ void k_ov_tail<8>(DevState, const double *, int64_t, int, int, int64_t);
-template __global__ void k_ov_tail<16>(DevState, const double *, int64_t, int, int, int64_t);
+template __global__ void k_ov_tail<64>(DevState, const double *, int64_t, int, int, int64_t);
 
-// after the rounds: a replica whose last round still made progress would
-// need more rounds
-__global__ void k_ov_end(DevState s, int rounds, int err_if_pending) {
+// after the rounds: positions, velocities and marks of every atom
+__global__ void __launch_bounds__(DML_BLOCK) k_ov_finish(DevState s, int rounds) {
+  const int i = blockIdx.x * DML_BLOCK + threadIdx.x;
+  int r;
+  const RepParams &P = rep_of_block(s, blockIdx.x, &r);
+  if (P.overlap_mode != DML_OVERLAP_ROUNDS) return;
+  const int last = s.ov_last[r];
+  if (i == P.poff) {
+    atomicAdd(&cnt_of(s, r, 0).passes, 1ull);
+    if (!P.halted) {
+      s.rp[r].ovn_stamp = 0;  // reverts move atoms
+      // the last round still made progress: more would be needed
+      if (last == rounds - 1) atomicAdd(&cnt_of(s, r, 0).ov_unfinished, 1ull);
+    }
+  }
+  if (i - P.poff >= P.nslots) return;
+  const int w = __float_as_int(s.pf4[i].w);
+  if (OVW_AT(w)) {
+    const double x = s.cx[i], y = s.cy[i], z = s.cz[i];
+    s.px[i] = x; s.py[i] = y; s.pz[i] = z;
+    if (w & OVW_HIT) {
+      s.vx[i] = 0.0; s.vy[i] = 0.0; s.vz[i] = 0.0;
+      s.ax[i] = 0.0; s.ay[i] = 0.0; s.az[i] = 0.0;
+    }
+    put_pf4(s, i, x, y, z, s.species[i]);
+  }
+  if (P.halted) return;
+  const uint8_t f = s.flags[i];
+  const int at = max(s.ovq[0][i], s.ovq[1][i]) - P.ov_round;  // the last round it was listed for
+  uint8_t g = f;
+  if (at > 0) {
+    // resolved there if that round came to it
+    g = at < rounds && last >= at - 1 ? f | DML_FL_SKIP : f & (uint8_t)~DML_FL_SKIP;
+  } else if (f & DML_FL_REF) {
+    g = f | DML_FL_SKIP;  // resolved in round 0
+  } else if (w & OVW_HIT) {
+    g = f & (uint8_t)~DML_FL_SKIP;
+  }
+  if (g != f) s.flags[i] = g;
+}
+
+// atoms still overlapping after the last round are an error of the call
+__global__ void k_ov_end(DevState s, int rounds) {
   int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= s.nrep) return;
   if (s.rp[r].overlap_mode != DML_OVERLAP_ROUNDS || s.rp[r].halted) return;
-  if (s.ov_more[((rounds - 1) % 3) * s.nrep + r]) {
-    if (err_if_pending) rep_fail(s, r, ERR_OVERLAP);
-    atomicAdd(&cnt_of(s, r, 0).ov_unfinished, 1ull);
-  }
-}
-
-// advance every replica's stamp base past this call's rounds
-__global__ void k_ov_close(DevState s, int rounds) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= s.nrep) return;
-  RepParams *Pw = s.rp + r;
-  if (Pw->overlap_mode != DML_OVERLAP_ROUNDS) return;
-  Pw->ov_round += rounds + 2;
-  atomicAdd(&cnt_of(s, r, 0).passes, 1ull);
+  if (s.ov_last[r] == rounds - 1) rep_fail(s, r, ERR_OVERLAP);
 }
 
 __global__ void k_init_pf4(DevState s, int64_t n) {
