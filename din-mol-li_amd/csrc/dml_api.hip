@@ -775,14 +775,17 @@ int ensure_exact(dml_ctx *c) {
   for (auto &h : c->reps) any |= h.p.overlap_mode == DML_OVERLAP_EXACT;
   if (!any) return DML_OK;
   uint8_t *n = nullptr;
-  int32_t *l = nullptr;
-  unsigned long long *m = nullptr;
-  if (dalloc(&n, c->P) || dalloc(&l, c->P * (int64_t)OVX_MAX) || dalloc(&m, c->P / 64)) {
+  uint32_t *b = nullptr;
+  unsigned long long *l = nullptr, *m = nullptr;
+  if (dalloc(&n, c->P) || dalloc(&l, c->P * (int64_t)OVX_MAX) || dalloc(&m, c->P / 64) ||
+      dalloc(&b, 2 * (c->P / 32))) {
     hipFree(n);
     hipFree(l);
     hipFree(m);
+    hipFree(b);
     return DML_E_NOMEM;
   }
+  c->d.ovx_b = b;
   c->d.ovx_n = n;
   c->d.ovx_l = l;
   c->d.ovx_m = m;
@@ -1045,7 +1048,7 @@ int dml_destroy(dml_ctx *c) {
                   d.species, d.flags, d.rowflag, d.bkey, d.pid, d.ref_order, d.ref_tmp,
                   d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ovq[0],
                   d.ovq[1], d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
-                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ov_last, d.ovx_n, d.ovx_l, d.ovx_m, d.pf4, d.bf4, d.gc_order,
+                  d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ov_last, d.ovx_n, d.ovx_l, d.ovx_m, d.ovx_b, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
                   d.cm_rep, d.cm_cell, d.cm_nref, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
                   d.gb_pt, d.gb_u, d.gb_du, d.gb_g, d.gb_kind, d.gb_cell, d.gb_nblk, d.gb_blk,

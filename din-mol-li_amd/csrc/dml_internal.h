@@ -312,11 +312,13 @@ struct DevState {
   int32_t *ovw[2];
   int32_t *ov_last;       // [nrep]: last round in which the replica reverted or deferred
   // reference-order overlap pass (only with such a replica): per ref position
-  // the row entries it can meet (count, 255 = more than listed), and the
-  // masks of positions to visit of replicas too large for LDS
+  // the row entries it can meet (count, 255 = more than listed), and, of
+  // replicas too large for LDS, the masks of positions to visit and the
+  // slots' position bits
   uint8_t *ovx_n;
-  int32_t *ovx_l;         // OVX_MAX per ref position
+  unsigned long long *ovx_l;  // OVX_MAX per ref position
   unsigned long long *ovx_m;
+  uint32_t *ovx_b;
   int32_t *gc_order;      // gcmc group in list order (global slots)
   int32_t *b2slot;        // hs%b index -> global slot, -1 when free
   int32_t *seq;           // creation number: the order of sys%alist

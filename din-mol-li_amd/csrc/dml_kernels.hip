@@ -1859,18 +1859,58 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ermak_a(DevState s, const double 
 // An atom holds one of two positions during the call: the current one or,
 // once reverted, old_cg.  k_ov_contacts lists, in parallel and in row order,
 // the row entries that come within rcut of an atom at some combination of
-// the two atoms' positions (FP64, the expressions of the walk): no other
-// entry can be met, whatever the reverts.  k_ov_exact then walks the atoms
-// that have such entries; a visit to any other atom only marks it.  The walk
+// the two atoms' positions (FP64, the reference's expressions), with the
+// verdict of each combination: no other entry can be met, whatever the
+// reverts, and the walk needs no positions.  k_ov_exact then walks the atoms
+// that have such entries, a visit to any other atom only marks it.  The walk
 // is one wave: it takes the 64 atoms of a mask word at a time, every lane
-// testing its own atom's few entries at the current positions, and visits
-// the first atom with a contact exactly as the sequential pass does; after a
-// visit that moved something the lanes behind it test again.
+// testing its own atom's few entries for the positions the atoms hold now
+// (a bit each, in LDS), and visits the first atom with a contact exactly as
+// the sequential pass does; after a visit that moved something the lanes
+// behind it test again.  The workgroup writes positions, velocities and marks
+// at the end, once per atom.
 //
-// The walk is bound by its chain of dependent loads.  Visiting every atom's
+// The walk is bound by its chain of dependent steps.  Visiting every atom's
 // whole row one after the other (four dependent loads an atom) took 0.50 ms
 // a call for 600 ions, 0.99 ms for 1,204 and 2.46 ms for the 1,505 to 3,009
-// ions of a chunks run with ~120 reverts a call.
+// ions of a chunks run with ~120 reverts a call; with the lists alone, the
+// positions read from memory at every test, 57, 60 and 573 us; now 18, 12 and
+// 162 us.
+//
+// an entry: replica-local slot (29 bits), ref position + 1 (0: not in ref; 29
+// bits), then in bits 58-61 "within rcut" with (this atom, the entry) at
+// (current, current), (current, old), (old, current), (old, old), bit 62: an
+// electrode atom, bit 63: its two positions are the same
+#define OVX_J(e) ((int)((e) & 0x1fffffffull))
+#define OVX_T(e) ((int)((e) >> 29 & 0x1fffffffull) - 1)
+#define OVX_NEAR(e, io, jo) ((int)((e) >> (58 + 2 * (io) + (jo))) & 1)
+#define OVX_CG (1ull << 62)
+#define OVX_SAME (1ull << 63)
+__device__ inline int within2(const RepParams &P, double ax, double ay, double az, double bx,
+                              double by, double bz) {
+  double dx, dy, dz;
+  vdist_mic(P, ax, ay, az, bx, by, bz, &dx, &dy, &dz);
+  return !(dot3(dx, dy, dz) > P.rcut2);
+}
+// the entry for row neighbour j of the atom at (xi, yi, zi), old_cg (ui, vi, wi)
+__device__ inline unsigned long long ovx_entry(const DevState &s, const RepParams &P, int j,
+                                               double xi, double yi, double zi, double ui,
+                                               double vi, double wi) {
+  const double x = s.px[j], y = s.py[j], z = s.pz[j];
+  const double u = s.cx[j], v = s.cy[j], w = s.cz[j];
+  const int cg = s.species[j] == SP_CG;  // stays where it is
+  unsigned long long e = (unsigned long long)(within2(P, xi, yi, zi, x, y, z) |
+                                              within2(P, ui, vi, wi, x, y, z) << 2)
+                         << 58;
+  if (!cg)
+    e |= (unsigned long long)(within2(P, xi, yi, zi, u, v, w) << 1 |
+                              within2(P, ui, vi, wi, u, v, w) << 3)
+         << 58;
+  const int t = (s.flags[j] & DML_FL_REF) ? s.ref_pos[j] + 1 : 0;
+  return e | (unsigned long long)(uint32_t)(j - P.poff) | (unsigned long long)(uint32_t)t << 29 |
+         (cg ? OVX_CG : 0ull) | (x == u && y == v && z == w ? OVX_SAME : 0ull);
+}
+
 template <int LPA>
 __global__ void __launch_bounds__(DML_BLOCK) k_ov_contacts(DevState s) {
   const int gid = blockIdx.x * DML_BLOCK + threadIdx.x;
@@ -1885,32 +1925,17 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ov_contacts(DevState s) {
   const int nn = s.nn[i];
   const int32_t *row = s.nbr + (int64_t)i * s.maxnn;
   const int g0 = (threadIdx.x % WAVE) & ~(LPA - 1);  // first lane of this atom
-  const double rcut2 = P.rcut2;
   int n = 0;
   for (int e0 = 0; e0 < nn; e0 += LPA) {
-    const int e = e0 + sub;
-    int j = -1, hit = 0;
-    if (e < nn) {
-      j = row[e];
-      if (!(s.flags[j] & DML_FL_LIMBO)) {
-        const double x = s.px[j], y = s.py[j], z = s.pz[j];
-        const double u = s.cx[j], v = s.cy[j], w = s.cz[j];
-        double dx, dy, dz;
-        vdist_mic(P, xi, yi, zi, x, y, z, &dx, &dy, &dz);
-        hit = !(dot3(dx, dy, dz) > rcut2);
-        vdist_mic(P, ui, vi, wi, x, y, z, &dx, &dy, &dz);
-        hit |= !(dot3(dx, dy, dz) > rcut2);
-        if (s.species[j] != SP_CG) {  // an electrode atom stays where it is
-          vdist_mic(P, xi, yi, zi, u, v, w, &dx, &dy, &dz);
-          hit |= !(dot3(dx, dy, dz) > rcut2);
-          vdist_mic(P, ui, vi, wi, u, v, w, &dx, &dy, &dz);
-          hit |= !(dot3(dx, dy, dz) > rcut2);
-        }
-      }
+    unsigned long long ent = 0;
+    if (e0 + sub < nn) {
+      const int j = row[e0 + sub];
+      if (!(s.flags[j] & DML_FL_LIMBO)) ent = ovx_entry(s, P, j, xi, yi, zi, ui, vi, wi);
     }
+    const int hit = (ent >> 58 & 15) != 0;
     const uint32_t m = (uint32_t)(__ballot(hit) >> g0) & ((1u << LPA) - 1u);
     const int q = n + __popc(m & ((1u << sub) - 1u));
-    if (hit && q < OVX_MAX) s.ovx_l[(int64_t)t * OVX_MAX + q] = j;
+    if (hit && q < OVX_MAX) s.ovx_l[(int64_t)t * OVX_MAX + q] = ent;
     n += __popc(m);
   }
   if (sub == 0) s.ovx_n[t] = (uint8_t)(n <= OVX_MAX ? n : 255);
@@ -1918,217 +1943,261 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ov_contacts(DevState s) {
 template __global__ void k_ov_contacts<8>(DevState s);
 
 #define OVX_WORDS 2048  // mask words kept in LDS (131,072 ref atoms); more: in HBM
-__global__ void __launch_bounds__(OVX_BLOCK) k_ov_exact(DevState s, const double *u, int64_t n_u,
-                                                        int max_passes) {
-  __shared__ unsigned long long sh_m[OVX_WORDS];
-  const int r = blockIdx.x;
+#define OVX_BITS 8192   // words of 32 slots' position bits kept in LDS (262,144 slots)
+__device__ __forceinline__ int ovx_bit(const uint32_t *b, int k) {
+  return (int)(b[k >> 5] >> (k & 31)) & 1;
+}
+// word w's atoms (slot, number of entries, the first four of them), one per
+// lane (w < 0: nothing); the next word's are loaded while one is walked
+#define OVX_FETCH(w)                                                            \
+  if ((w) >= 0) {                                                               \
+    const int ft = (w) * WAVE + lane;                                           \
+    f_w = (w);                                                                  \
+    f_n = 0;                                                                    \
+    f_i = poff;                                                                 \
+    if (ft < nref) {                                                            \
+      f_i = s.ref_order[poff + ft];                                             \
+      f_n = s.ovx_n[poff + ft];                                                 \
+      const unsigned long long *l = s.ovx_l + (int64_t)(poff + ft) * OVX_MAX;   \
+      f_0 = l[0];                                                               \
+      f_1 = l[1];                                                               \
+      f_2 = l[2];                                                               \
+      f_3 = l[3];                                                               \
+    }                                                                           \
+  }
+
+// M: bit t % 64 of word t / 64: ref position t is to be visited and has
+// entries to look at; H: it has entries at all.  old_b, hit_b, per slot: the
+// atom is at old_cg; a neighbour put it there.  L: the lists of the word the
+// walk is at, entry-major (lanes on their own banks).  One instance for LDS
+// and one for HBM: a pointer that could be either would make every access
+// wait for both kinds
+template <bool LDS>
+__device__ __forceinline__ void ov_exact_body(const DevState &s, const double *u, int64_t n_u,
+                                              int max_passes, int r, unsigned long long *M,
+                                              unsigned long long *H, uint32_t *old_b,
+                                              uint32_t *hit_b, unsigned long long (*L)[WAVE]) {
   const RepParams &P = s.rp[r];
-  if (P.halted || P.overlap_mode != DML_OVERLAP_EXACT) return;
   const int lane = threadIdx.x % WAVE;
-  const int poff = P.poff, nref = P.nref;
-  const int nw = (nref + WAVE - 1) / WAVE;
-  // bit t % 64 of word t / 64: ref position t is to be visited and has
-  // entries to look at
-  unsigned long long *M = nw <= OVX_WORDS ? sh_m : s.ovx_m + poff / WAVE;
+  const int poff = P.poff, nref = P.nref, nslots = P.nslots;
+  const int nw = (nref + WAVE - 1) / WAVE, nbw = (nslots + 31) / 32;
+  for (int q = threadIdx.x; q < nbw; q += OVX_BLOCK) old_b[q] = hit_b[q] = 0u;
   for (int w = threadIdx.x / WAVE; w < nw; w += OVX_BLOCK / WAVE) {
     const int t = w * WAVE + lane;
-    int go = 0;
-    if (t < nref) {
-      const int i = s.ref_order[poff + t];
-      const uint8_t f = s.flags[i];
-      if (!(f & DML_FL_SKIP)) {
-        go = s.ovx_n[poff + t] != 0;
-        if (!go) s.flags[i] = f | DML_FL_SKIP;
-      }
+    const int has = t < nref && s.ovx_n[poff + t] != 0;
+    const int go = has && !(s.flags[s.ref_order[poff + t]] & DML_FL_SKIP);
+    const unsigned long long m = __ballot(go), h = __ballot(has);
+    if (lane == 0) {
+      M[w] = m;
+      if (LDS) H[w] = h;  // positions that have entries at all
     }
-    const unsigned long long m = __ballot(go);
-    if (lane == 0) M[w] = m;
   }
   __syncthreads();
-  if (threadIdx.x >= WAVE) return;
-  const double *ur = u ? u + (int64_t)r * n_u : nullptr;
-  int64_t ucount = 0;
-  unsigned long long n_try = 0, n_depo = 0, n_ch = 0, n_ch3 = 0, n_pass = 0;
-  const double rcut2 = P.rcut2;
-  int again = 1;
-  for (int pass = 0; again; pass++) {
-    if (pass >= max_passes) {
-      if (lane == 0) rep_fail(s, r, ERR_OVERLAP);
-      break;
-    }
-    again = 0;
-    n_pass++;
-    for (int w0 = 0; w0 < nw; w0 += WAVE) {
-      // 64 mask words, one per lane
-      unsigned long long word = w0 + lane < nw ? M[w0 + lane] : 0ull;
-      unsigned long long nz = __ballot(word != 0ull);
-      while (nz) {
-        const int wq = __builtin_ctzll(nz);
-        nz &= nz - 1ull;
-        // the atoms of this word still to visit in this pass, and those a
-        // visit puts back behind it (next pass)
-        unsigned long long cur =
-            (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)word, wq) |
-            (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), wq) << 32;
-        unsigned long long nxt = 0ull;
-        const int wi = w0 + wq;
-        const int t = poff + wi * WAVE + lane;  // this lane's ref position
-        const bool in = wi * WAVE + lane < nref;
-        const int i = in ? s.ref_order[t] : poff;
-        const int n = in ? s.ovx_n[t] : 0;
-        // the list, four entries at a time (entry 0 where there is none: the
-        // loads below then need no branch around each)
-        const int have = n <= OVX_MAX ? n : 0;
-        int l[OVX_MAX];
-#pragma unroll
-        for (int k = 0; k < OVX_MAX; k += 4) {
-          int4 v = make_int4(i, i, i, i);
-          if (k < have) v = *(const int4 *)(s.ovx_l + (int64_t)t * OVX_MAX + k);
-          l[k] = v.x;
-          l[k + 1] = k + 1 < have ? v.y : i;
-          l[k + 2] = k + 2 < have ? v.z : i;
-          l[k + 3] = k + 3 < have ? v.w : i;
-        }
-        unsigned long long met = 0ull;
-        bool stale = true;  // positions moved since `met` was found
-        while (cur) {
-          if (stale) {
-            int hit = n > OVX_MAX;
-            const double xi = s.px[i], yi = s.py[i], zi = s.pz[i];
-#pragma unroll
-            for (int k0 = 0; k0 < OVX_MAX; k0 += 4) {
-              if (!__ballot(k0 < have)) break;
-              double x[4], y[4], z[4];
-#pragma unroll
-              for (int k = 0; k < 4; k++) {
-                x[k] = s.px[l[k0 + k]];
-                y[k] = s.py[l[k0 + k]];
-                z[k] = s.pz[l[k0 + k]];
-              }
-#pragma unroll
-              for (int k = 0; k < 4; k++) {
-                double dx, dy, dz;
-                vdist_mic(P, xi, yi, zi, x[k], y[k], z[k], &dx, &dy, &dz);
-                hit |= (k0 + k < have) & !(dot3(dx, dy, dz) > rcut2);
-              }
+  if (threadIdx.x < WAVE) {
+    const double *ur = u ? u + (int64_t)r * n_u : nullptr;
+    int64_t ucount = 0;
+    unsigned long long n_try = 0, n_depo = 0, n_ch = 0, n_ch3 = 0, n_pass = 0;
+    const int piston = P.piston;
+    // a word's atoms (slot, entries, the first four of them), one per lane;
+    // the next word's are loaded while this one is walked
+    int f_w = -1, f_i = 0, f_n = 0;
+    unsigned long long f_0 = 0ull, f_1 = 0ull, f_2 = 0ull, f_3 = 0ull;
+    int again = 1;
+    for (int pass = 0; again; pass++) {
+      if (pass >= max_passes) {
+        if (lane == 0) rep_fail(s, r, ERR_OVERLAP);
+        break;
+      }
+      again = 0;
+      n_pass++;
+      for (int w0 = 0; w0 < nw; w0 += WAVE) {
+        // 64 mask words, one per lane
+        unsigned long long word = w0 + lane < nw ? M[w0 + lane] : 0ull;
+        unsigned long long nz = __ballot(word != 0ull);
+        while (nz) {
+          const int wq = __builtin_ctzll(nz);
+          nz &= nz - 1ull;
+          // the atoms of this word still to visit in this pass, and those a
+          // visit puts back behind it (next pass)
+          unsigned long long cur =
+              (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)word, wq) |
+              (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), wq) << 32;
+          unsigned long long nxt = 0ull;
+          const int wi = w0 + wq;
+          const int t = poff + wi * WAVE + lane;  // this lane's ref position
+          int get = f_w != wi ? wi : -1;
+          OVX_FETCH(get)
+          const int i = f_i - poff, n = f_n;
+          const int have = n <= OVX_MAX ? n : 0;
+          // the lists; all 64 atoms' (a visit may put one back that is not
+          // in `cur` yet)
+          __builtin_amdgcn_wave_barrier();
+          L[0][lane] = f_0;
+          L[1][lane] = f_1;
+          L[2][lane] = f_2;
+          L[3][lane] = f_3;
+          for (int k = 4; __ballot(k < have); k += 2) {
+            if (k < have) {
+              const unsigned long long *l = s.ovx_l + (int64_t)t * OVX_MAX + k;
+              const unsigned long long l0 = l[0], l1 = l[1];
+              L[k][lane] = l0;
+              L[k + 1][lane] = l1;
             }
-            met = __ballot(hit);
-            stale = false;
           }
-          const unsigned long long first = met & cur;
-          const int q = first ? __builtin_ctzll(first) : WAVE - 1;
-          // the atoms up to and including q are visited
-          const unsigned long long upto = q == WAVE - 1 ? ~0ull : (1ull << (q + 1)) - 1ull;
-          if (cur & upto & 1ull << lane) s.flags[i] |= DML_FL_SKIP;
-          cur &= ~upto;
-          if (!first) break;
-          // the visit of the reference's pass
-          const int ii = __builtin_amdgcn_readlane(i, q);
-          const int nq = __builtin_amdgcn_readlane(n, q);
-          const int nn = nq > OVX_MAX ? s.nn[ii] : nq;
-          const int32_t *row = nq > OVX_MAX ? s.nbr + (int64_t)ii * s.maxnn
-                                            : s.ovx_l + (int64_t)(poff + wi * WAVE + q) * OVX_MAX;
-          const double xi = s.px[ii], yi = s.py[ii], zi = s.pz[ii];
-          // reverted atom (replica-local ref position tj) back into the masks
-          auto back = [&](int tj) {
-            const int wj = tj >> 6;
-            const unsigned long long bit = 1ull << (tj & 63);
-            if (wj == wi) {
-              if ((tj & 63) > q) cur |= bit; else nxt |= bit;
-              return;
+          get = nz ? w0 + __builtin_ctzll(nz) : -1;
+          OVX_FETCH(get)
+          __builtin_amdgcn_wave_barrier();
+          unsigned long long met = 0ull;
+          bool stale = true;  // atoms moved since `met` was found
+          while (cur) {
+            if (stale) {
+              int hit = n > OVX_MAX;
+              const int io = ovx_bit(old_b, i);
+              for (int k = 0; __ballot(k < have); k++) {
+                if (k < have) {
+                  const unsigned long long e = L[k][lane];
+                  hit |= OVX_NEAR(e, io, ovx_bit(old_b, OVX_J(e)));
+                }
+              }
+              met = __ballot(hit);
+              stale = false;
             }
-            if (lane == 0) M[wj] |= bit;
-            if (wj > wi && wj < w0 + WAVE) {
-              if (lane == wj - w0) word |= bit;
-              nz |= 1ull << (wj - w0);
-            }
-          };
-          int done = 0;
-          for (int e0 = 0; e0 < nn && !done; e0 += WAVE) {
-            const int e = e0 + lane;
-            const int j = e < nn ? row[e] : -1;
-            int hit = 0;
-            if (j >= 0 && !(s.flags[j] & DML_FL_LIMBO)) {
-              double dx, dy, dz;
-              vdist_mic(P, xi, yi, zi, s.px[j], s.py[j], s.pz[j], &dx, &dy, &dz);
-              hit = !(dot3(dx, dy, dz) > rcut2);
-            }
-            unsigned long long hm = __ballot(hit);
-            while (hm) {
-              const int q2 = __builtin_ctzll(hm);
-              hm &= hm - 1ull;
-              const int jj = __builtin_amdgcn_readlane(j, q2);
-              double dx, dy, dz;
-              vdist_mic(P, xi, yi, zi, s.px[jj], s.py[jj], s.pz[jj], &dx, &dy, &dz);
+            const unsigned long long first = met & cur;
+            if (!first) break;  // the rest of the word has no contact
+            const int q = __builtin_ctzll(first);
+            cur &= q == WAVE - 1 ? 0ull : ~0ull << (q + 1);
+            // the visit of the reference's pass
+            const int ii = __builtin_amdgcn_readlane(i, q);
+            const int nq = __builtin_amdgcn_readlane(n, q);
+            const int gi = poff + ii;
+            const int nn = nq > OVX_MAX ? s.nn[gi] : nq;
+            const int io = ovx_bit(old_b, ii);
+            for (int k = 0; k < nn; k++) {
+              unsigned long long e;
+              if (nq <= OVX_MAX) {
+                e = L[k][q];
+              } else {
+                // more entries than the list holds: the whole row
+                const int j = s.nbr[(int64_t)gi * s.maxnn + k];
+                if (s.flags[j] & DML_FL_LIMBO) continue;
+                e = ovx_entry(s, P, j, s.px[gi], s.py[gi], s.pz[gi], s.cx[gi], s.cy[gi],
+                              s.cz[gi]);
+              }
               // every lane takes the same decisions from the same reads, then
-              // writes the same values: the reads come before any write
-              const bool near = !(dot3(dx, dy, dz) > rcut2);
-              const bool cg = near && s.species[jj] == SP_CG;
-              const bool stay = near && !cg && P.piston && same_pos(s, jj) && same_pos(s, ii);
-              const uint8_t fj = s.flags[jj];
-              const int tj = s.ref_pos[jj];
+              // one writes: the reads come before any write
+              const int jj = OVX_J(e), jo = ovx_bit(old_b, jj);
               __builtin_amdgcn_wave_barrier();
-              if (!near) continue;
-              if (cg) {
+              if (!OVX_NEAR(e, io, jo)) continue;
+              if (e & OVX_CG) {
                 n_try++;
                 double ne;
                 if (ur) {
                   ne = ucount < n_u ? ur[ucount] : 0.5;
                   if (ucount >= n_u && lane == 0) rep_fail(s, r, ERR_OVERLAP);
                 } else {
-                  u32x4 w = dml_philox(P.seed, s.pid[ii], (uint32_t)P.step, RS_CONTACT,
+                  u32x4 w = dml_philox(P.seed, s.pid[gi], (uint32_t)P.step, RS_CONTACT,
                                        (uint32_t)ucount);
                   ne = u01_from(w.x, w.y);
                 }
                 ucount++;
                 if (ne < P.prob) {
                   n_depo++;
-                  s.species[ii] = SP_F;
-                  put_pf4_sp(s, ii, SP_F);
-                  if (lane == 0) s.rp[r].any_f = 1;
-                  if (zi > P.z0 && lane == 0) rep_fail(s, r, ERR_DEPZ0);
+                  if (lane == 0) {
+                    s.species[gi] = SP_F;
+                    put_pf4_sp(s, gi, SP_F);
+                    s.rp[r].any_f = 1;
+                    if ((io ? s.cz[gi] : s.pz[gi]) > P.z0) rep_fail(s, r, ERR_DEPZ0);
+                  }
                 } else {
-                  s.px[ii] = s.cx[ii]; s.py[ii] = s.cy[ii]; s.pz[ii] = s.cz[ii];
-                  put_pf4(s, ii, s.cx[ii], s.cy[ii], s.cz[ii], s.species[ii]);
-                  s.flags[ii] &= (uint8_t)~DML_FL_SKIP;
+                  if (lane == 0) old_b[ii >> 5] |= 1u << (ii & 31);
                   nxt |= 1ull << q;
                   stale = true;
                 }
-                done = 1;
                 break;
               }
-              if (stay) {
+              // dana.F90:920-927: both sit where they were
+              if (piston && (jo || (e & OVX_SAME)) && (io || same_pos(s, gi))) {
                 n_ch3++;
                 continue;
               }
-              s.px[jj] = s.cx[jj]; s.py[jj] = s.cy[jj]; s.pz[jj] = s.cz[jj];
-              put_pf4(s, jj, s.cx[jj], s.cy[jj], s.cz[jj], s.species[jj]);
-              s.vx[jj] = 0.0; s.vy[jj] = 0.0; s.vz[jj] = 0.0;
-              s.ax[jj] = 0.0; s.ay[jj] = 0.0; s.az[jj] = 0.0;
+              if (lane == 0) {
+                old_b[jj >> 5] |= 1u << (jj & 31);
+                hit_b[jj >> 5] |= 1u << (jj & 31);
+              }
               // a ref atom that has nothing to meet is visited again to no
               // effect but its mark
-              const bool ref = (fj & DML_FL_REF) && tj >= 0 && tj < nref;
-              const bool more = ref && s.ovx_n[poff + tj] != 0;
-              if (more) back(tj);
-              s.flags[jj] = (uint8_t)(ref && !more ? fj | DML_FL_SKIP : fj & ~DML_FL_SKIP);
+              const int tj = OVX_T(e);
+              if (tj >= 0 && tj < nref &&
+                  (LDS ? (int)(H[tj >> 6] >> (tj & 63) & 1ull) : s.ovx_n[poff + tj] != 0)) {
+                // back into the masks
+                const int wj = tj >> 6;
+                const unsigned long long bit = 1ull << (tj & 63);
+                if (wj == wi) {
+                  if ((tj & 63) > q) cur |= bit; else nxt |= bit;
+                } else {
+                  if (lane == 0) M[wj] |= bit;
+                  if (wj > wi && wj < w0 + WAVE) {
+                    word |= lane == wj - w0 ? bit : 0ull;
+                    nz |= 1ull << (wj - w0);
+                  }
+                }
+              }
               n_ch++;
               again = 1;
               stale = true;
             }
+            __builtin_amdgcn_wave_barrier();
           }
+          if (lane == 0) M[wi] = nxt;
+          __builtin_amdgcn_wave_barrier();
         }
-        if (lane == 0) M[wi] = nxt;
-        __builtin_amdgcn_wave_barrier();
       }
     }
+    if (lane == 0) {
+      atomicAdd(&cnt_of(s, r, 0).try_, n_try);
+      atomicAdd(&cnt_of(s, r, 0).depo, n_depo);
+      atomicAdd(&cnt_of(s, r, 0).choques, n_ch);
+      atomicAdd(&cnt_of(s, r, 0).choques3, n_ch3);
+      atomicAdd(&cnt_of(s, r, 0).passes, n_pass);
+    }
   }
-  if (lane == 0) {
-    atomicAdd(&cnt_of(s, r, 0).try_, n_try);
-    atomicAdd(&cnt_of(s, r, 0).depo, n_depo);
-    atomicAdd(&cnt_of(s, r, 0).choques, n_ch);
-    atomicAdd(&cnt_of(s, r, 0).choques3, n_ch3);
-    atomicAdd(&cnt_of(s, r, 0).passes, n_pass);
+  __syncthreads();
+  for (int q = threadIdx.x; q < nslots; q += OVX_BLOCK) {
+    const uint32_t bit = 1u << (q & 31);
+    if (!(old_b[q >> 5] & bit)) continue;
+    const int i = poff + q;
+    const double x = s.cx[i], y = s.cy[i], z = s.cz[i];
+    s.px[i] = x; s.py[i] = y; s.pz[i] = z;
+    put_pf4(s, i, x, y, z, s.species[i]);
+    if (hit_b[q >> 5] & bit) {
+      s.vx[i] = 0.0; s.vy[i] = 0.0; s.vz[i] = 0.0;
+      s.ax[i] = 0.0; s.ay[i] = 0.0; s.az[i] = 0.0;
+      if (!(s.flags[i] & DML_FL_REF)) s.flags[i] &= (uint8_t)~DML_FL_SKIP;
+    }
   }
+  // every ref atom is resolved but those whose failed contact trial ended
+  // the last pass
+  for (int t = threadIdx.x; t < nref; t += OVX_BLOCK) {
+    const int i = s.ref_order[poff + t];
+    const uint8_t f = s.flags[i];
+    s.flags[i] = M[t >> 6] >> (t & 63) & 1ull ? f & (uint8_t)~DML_FL_SKIP : f | DML_FL_SKIP;
+  }
+}
+#undef OVX_FETCH
+
+__global__ void __launch_bounds__(OVX_BLOCK) k_ov_exact(DevState s, const double *u, int64_t n_u,
+                                                        int max_passes) {
+  __shared__ unsigned long long sh_m[OVX_WORDS], sh_h[OVX_WORDS], sh_l[OVX_MAX][WAVE];
+  __shared__ uint32_t sh_b[2][OVX_BITS];
+  const int r = blockIdx.x;
+  const RepParams &P = s.rp[r];
+  if (P.halted || P.overlap_mode != DML_OVERLAP_EXACT) return;
+  if (P.nref <= OVX_WORDS * WAVE && P.nslots <= OVX_BITS * 32)
+    ov_exact_body<true>(s, u, n_u, max_passes, r, sh_m, sh_h, sh_b[0], sh_b[1], sh_l);
+  else
+    ov_exact_body<false>(s, u, n_u, max_passes, r, s.ovx_m + P.poff / WAVE, sh_h,
+                         s.ovx_b + P.poff / 32,
+                         s.ovx_b + s.nblocks * (DML_BLOCK / 32) + P.poff / 32, sh_l);
 }
 
 // deterministic parallel rounds (this build's schedule; orc.c
