@@ -105,6 +105,15 @@ struct dml_ctx {
   uint64_t graph_dsig = 0;   // device-state bytes the captured step was built with
   int64_t gb_total = 0;      // batched-GCMC trial pool (sum of the replicas' capacities)
   int dev = 0;               // the GPU current at creation
+  // the host mirror (reps[].p) holds what the device table does: set by every
+  // fetch and upload, cleared by whatever may change the table
+  int fresh = 0;
+  int err_seen = 0;          // error bits of the last fetch
+  unsigned char *h_rp = nullptr;    // pinned: the table and the error word
+  unsigned char *h_pin = nullptr;   // pinned staging of small transfers, kept
+  size_t h_cap = 0;
+  unsigned char *d_stage = nullptr; // device staging, kept
+  size_t d_cap = 0;
   unsigned char *scratch = nullptr;  // that GPU's copy of `scratch`
 };
 
@@ -240,17 +249,61 @@ int dalloc(T **p, int64_t n) {
   return DML_OK;
 }
 
-int read_err(dml_ctx *c, int reset) {
-  int e = 0;
-  if (hipMemcpyAsync(&e, c->d.err, sizeof(int), hipMemcpyDeviceToHost, c->st) != hipSuccess)
-    return -1;
-  if (hipStreamSynchronize(c->st) != hipSuccess) return -1;
-  if (reset && e) {
-    int z = 0;
-    hipMemcpyAsync(c->d.err, &z, sizeof(int), hipMemcpyHostToDevice, c->st);
-    hipStreamSynchronize(c->st);
+// The replica table and the error word lie together on the device: one copy
+// into pinned memory and one wait bring both.  (A call that read the word, then
+// the table, each through pageable memory, waited twice: about 35 us of the
+// 68 us that a routine of a 1,204-ion system took.)
+size_t table_bytes(const dml_ctx *c) { return sizeof(RepParams) * (size_t)c->nrep; }
+
+void copy_table(dml_ctx *c) {
+  hipMemcpyAsync(c->h_rp, c->d.rp, table_bytes(c) + sizeof(int32_t), hipMemcpyDeviceToHost, c->st);
+}
+
+// after copy_table: wait for the stream and take the table over
+int take_table(dml_ctx *c) {
+  if (hipStreamSynchronize(c->st) != hipSuccess) return DML_E_HIP;
+  for (int r = 0; r < c->nrep; r++)
+    memcpy(&c->reps[r].p, c->h_rp + sizeof(RepParams) * (size_t)r, sizeof(RepParams));
+  int32_t e;
+  memcpy(&e, c->h_rp + table_bytes(c), sizeof(e));
+  c->err_seen = e;
+  c->fresh = 1;
+  return DML_OK;
+}
+
+// pinned staging of at least n bytes, null when it would be too large to keep
+constexpr size_t kPinMost = 4u << 20;
+unsigned char *pinned(dml_ctx *c, size_t n) {
+  if (n > kPinMost) return nullptr;
+  if (n > c->h_cap) {
+    if (c->h_pin) hipHostFree(c->h_pin);
+    c->h_pin = nullptr;
+    c->h_cap = 0;
+    size_t cap = 64u << 10;
+    while (cap < n) cap *= 2;
+    if (hipHostMalloc((void **)&c->h_pin, cap, hipHostMallocDefault) != hipSuccess) {
+      c->h_pin = nullptr;
+      return nullptr;
+    }
+    c->h_cap = cap;
   }
-  return e;
+  return c->h_pin;
+}
+
+// device staging of at least n bytes (the stream is idle: the old one may go)
+unsigned char *staging(dml_ctx *c, size_t n) {
+  if (n > c->d_cap) {
+    hipFree(c->d_stage);
+    c->d_stage = nullptr;
+    c->d_cap = 0;
+    const size_t cap = std::max<size_t>(n, 64u << 10);
+    if (hipMalloc((void **)&c->d_stage, cap) != hipSuccess) {
+      c->d_stage = nullptr;
+      return nullptr;
+    }
+    c->d_cap = cap;
+  }
+  return c->d_stage;
 }
 
 void assign_list_kernels(dml_ctx *c);
@@ -319,17 +372,15 @@ int upload_params(dml_ctx *c) {
   for (int r = 0; r < c->nrep; r++) v[r] = c->reps[r].p;
   HIPCHECK(hipMemcpyAsync(c->d.rp, v.data(), sizeof(RepParams) * c->nrep, hipMemcpyHostToDevice,
                           c->st));
+  c->fresh = 1;
   return DML_OK;
 }
 
 // the mutable device fields are authoritative: fetch them into the mirror
 int fetch_params(dml_ctx *c) {
-  std::vector<RepParams> v(c->nrep);
-  HIPCHECK(hipMemcpyAsync(v.data(), c->d.rp, sizeof(RepParams) * c->nrep, hipMemcpyDeviceToHost,
-                          c->st));
-  HIPCHECK(hipStreamSynchronize(c->st));
-  for (int r = 0; r < c->nrep; r++) c->reps[r].p = v[r];
-  return DML_OK;
+  if (c->fresh) return DML_OK;
+  copy_table(c);
+  return take_table(c);
 }
 
 int alloc_cells(dml_ctx *c) {
@@ -465,6 +516,7 @@ void assign_list_kernels(dml_ctx *c) {
 // gcs = 1: also re-sort the cells of the GCMC replicas (their trials read
 // them before the next test_update)
 void enq_cells_lists(dml_ctx *c, int gcs) {
+  c->fresh = 0;
   dim3 gc(clamp_grid((c->d.n_cm + DML_BLOCK - 1) / DML_BLOCK));
   dim3 gw(clamp_grid((c->d.n_cm + 3) / 4));
   int nb = c->d.nblocks;
@@ -476,6 +528,7 @@ void enq_cells_lists(dml_ctx *c, int gcs) {
 
 // begin_ov: the overlap rounds follow
 void enq_test_update(dml_ctx *c, int gcs, int begin_ov = 0) {
+  c->fresh = 0;
   hipLaunchKernelGGL(k_pbc_dispmax, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_dispmax_final, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d, begin_ov);
   enq_cells_lists(c, gcs);
@@ -496,6 +549,7 @@ void launch_force_lpa(dml_ctx *c, int lpa, int only_ermak) {
 }
 
 void enq_forces(dml_ctx *c, int fuse_b, int only_ermak) {
+  c->fresh = 0;
   if (fuse_b)
     launch_force_lpa<1>(c, c->lpa, only_ermak);
   else
@@ -509,6 +563,7 @@ void enq_forces(dml_ctx *c, int fuse_b, int only_ermak) {
 // begun: the test_update before has started the rounds (k_dispmax_final)
 void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int rounds, int begun,
                         int err_if_pending) {
+  c->fresh = 0;
   if (!begun)
     hipLaunchKernelGGL(k_ov_begin, dim3((std::max(c->nrep, 3) + 63) / 64), dim3(64), 0, c->st,
                        c->d);
@@ -562,6 +617,7 @@ void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int r
 
 // the reference's order: the entries each atom can meet, then the walk
 void enq_overlap_exact(dml_ctx *c, const double *u, int64_t n_u, int max_passes) {
+  c->fresh = 0;
   if (!c->d.ovx_n) return;  // no replica in this mode
   hipLaunchKernelGGL(k_ov_contacts<8>, dim3((unsigned)(c->P * 8 / DML_BLOCK)), dim3(DML_BLOCK), 0,
                      c->st, c->d);
@@ -607,6 +663,7 @@ static void enq_gcmc_batch(dml_ctx *c, int r, const double *u, const double *g) 
 
 static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g, double act,
                      int nadj) {
+  c->fresh = 0;
   const int nb = c->d.nblocks;
   for (int stage = 0; stage < 2; stage++) {
     if (stage == 1) {
@@ -633,6 +690,7 @@ static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g,
 }
 
 void enq_f2cg(dml_ctx *c) {
+  c->fresh = 0;
   int nb = c->d.nblocks;
   hipLaunchKernelGGL(k_f2cg_mark, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_f2cg_scan, dim3(c->nrep), dim3(1024), 0, c->st, c->d);
@@ -643,6 +701,7 @@ void enq_f2cg(dml_ctx *c) {
 
 // bloques, then test_update of the replicas that added a block (dana.F90:771)
 void enq_bloques(dml_ctx *c) {
+  c->fresh = 0;
   const int rb = (c->nrep + 63) / 64;
   hipLaunchKernelGGL(k_chunk_run, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_mask_fired, dim3(rb), dim3(64), 0, c->st, c->d, 1);
@@ -651,6 +710,7 @@ void enq_bloques(dml_ctx *c) {
 }
 
 void enq_step(dml_ctx *c) {
+  c->fresh = 0;
   int nb = c->d.nblocks;
   if (c->any_ermak) {
     hipLaunchKernelGGL(k_ermak_a, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d,
@@ -726,11 +786,12 @@ int handle_overflow(dml_ctx *c, int e, int resume) {
       }
       HIPCHECK(hipMemcpy(c->d.rp, v.data(), sizeof(RepParams) * c->nrep, hipMemcpyHostToDevice));
     }
+    c->fresh = 0;
     int z = 0;
     HIPCHECK(hipMemcpyAsync(c->d.err, &z, sizeof(int), hipMemcpyHostToDevice, c->st));
     enq_cells_lists(c, 1);
-    e = read_err(c, 0);
-    if (e < 0) return DML_E_HIP;
+    if (fetch_params(c)) return DML_E_HIP;
+    e = c->err_seen;
   }
   return DML_OK;
 }
@@ -738,24 +799,24 @@ int handle_overflow(dml_ctx *c, int e, int resume) {
 // replica_fatal: report a replica's halt as the call's status (per-routine
 // entry points); dml_run leaves halted replicas to dml_replica_status()
 int finish(dml_ctx *c, int replica_fatal = 1, int resume = 1) {
-  int e = read_err(c, 0);
-  if (e < 0) return DML_E_HIP;
+  c->fresh = 0;
+  if (fetch_params(c)) return DML_E_HIP;
+  int e = c->err_seen;
   if (e & (ERR_LIST | ERR_BUCKET)) {
     int rc = handle_overflow(c, e, resume);
     if (rc) return rc;
-    e = read_err(c, 0);
+    c->fresh = 0;
+    if (fetch_params(c)) return DML_E_HIP;
+    e = c->err_seen;
   }
   if (e) {
     int z = 0;
     hipMemcpy(c->d.err, &z, sizeof(int), hipMemcpyHostToDevice);
     return status_from_err(e);
   }
-  if (replica_fatal) {
-    int rc = fetch_params(c);
-    if (rc) return rc;
+  if (replica_fatal)
     for (auto &h : c->reps)
       if (h.p.err_bits) return status_from_err(h.p.err_bits);
-  }
   return DML_OK;
 }
 
@@ -937,14 +998,22 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   e |= dalloc(&d.obs, 4 * (P / DML_BLOCK) + 4 * (int64_t)nrep);
   e |= dalloc(&d.part_i, 2 * (P / DML_BLOCK));
   e |= dalloc(&d.blk2rep, P / DML_BLOCK);
-  e |= dalloc(&d.rp, nrep);
+  {
+    unsigned char *q = nullptr;  // the table, then the error word
+    e |= dalloc(&q, (int64_t)table_bytes(c) + 64);
+    d.rp = (RepParams *)q;
+    d.err = q ? (int32_t *)(q + table_bytes(c)) : nullptr;
+  }
+  if (hipHostMalloc((void **)&c->h_rp, table_bytes(c) + 64, hipHostMallocDefault) != hipSuccess) {
+    c->h_rp = nullptr;
+    e |= 1;
+  }
   // a few thousand shards in all: a single large system needs the most (its
   // row build adds from some ten thousand waves), the replicas of an ensemble
   // are each other's shards
   d.ncsh = 512;
   while (d.ncsh > 8 && (int64_t)d.ncsh * nrep > 4096) d.ncsh /= 2;
   e |= dalloc(&d.cnt, (int64_t)nrep * d.ncsh);
-  e |= dalloc(&d.err, 1);
   e |= dalloc(&d.wl[0], P);
   e |= dalloc(&d.wl[1], P);
   e |= dalloc(&d.wl_cnt, 4);
@@ -1047,7 +1116,7 @@ int dml_destroy(dml_ctx *c) {
                   d.epot, d.ox, d.oy, d.oz, d.cx, d.cy, d.cz, d.rvx, d.rvy, d.rvz,
                   d.species, d.flags, d.rowflag, d.bkey, d.pid, d.ref_order, d.ref_tmp,
                   d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ovq[0],
-                  d.ovq[1], d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.err, d.wl[0],
+                  d.ovq[1], d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.wl[0],
                   d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ov_last, d.ovx_n, d.ovx_l, d.ovx_m, d.ovx_b, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
                   d.cm_rep, d.cm_cell, d.cm_nref, d.tm_rep, d.tm_cell, d.wm_blk, d.obs,
@@ -1059,6 +1128,9 @@ int dml_destroy(dml_ctx *c) {
                   d.gb_chead, d.gb_ccnt, d.gb_claim};
   for (void *q : ptrs)
     if (q) hipFree(q);
+  if (c->d_stage) hipFree(c->d_stage);
+  if (c->h_rp) hipHostFree(c->h_rp);
+  if (c->h_pin) hipHostFree(c->h_pin);
   if (c->e0) hipEventDestroy(c->e0);
   if (c->e1) hipEventDestroy(c->e1);
   if (c->st) hipStreamDestroy(c->st);
@@ -1079,100 +1151,79 @@ int dml_set_state(dml_ctx *c, int32_t rep, int32_t n, const double *pos, const d
   if (rc) return rc;
   RepParams &p = c->reps[rep].p;
   if (n > p.pcap) return DML_E_NOMEM;
-  int64_t o = p.poff;
-  std::vector<double> tmp(std::max(n, 1));
-  auto put = [&](double *dst, const double *src, int k, double dflt) -> int {
-    for (int i = 0; i < n; i++) tmp[i] = src ? src[(int64_t)k * n + i] : dflt;
-    HIPCHECK(hipMemcpy(dst + o, tmp.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-    return DML_OK;
-  };
-  double *P3[3] = {c->d.px, c->d.py, c->d.pz};
-  double *V3[3] = {c->d.vx, c->d.vy, c->d.vz};
-  double *A3[3] = {c->d.ax, c->d.ay, c->d.az};
-  double *O3[3] = {c->d.ox, c->d.oy, c->d.oz};
-  double *G3[3] = {c->d.cx, c->d.cy, c->d.cz};
-  for (int k = 0; k < 3; k++) {
-    if ((rc = put(P3[k], pos, k, 0.0))) return rc;
-    if ((rc = put(V3[k], vel, k, 0.0))) return rc;
-    if ((rc = put(A3[k], acel, k, 0.0))) return rc;
-    if ((rc = put(O3[k], pos_old ? pos_old : pos, k, 0.0))) return rc;
-    if ((rc = put(G3[k], old_cg, k, 1e8))) return rc;
+  const int64_t o = p.poff;
+  // one block of everything that the caller gave or that is listed here, one
+  // copy, one kernel (k_load_state) that also resets what a reused replica
+  // still holds: 15 copies and 12 fills of ~10 us each before.  Layout: pos
+  // and the given of vel, acel, pos_old, old_cg (24 n each); ref_pos, ref_order,
+  // gc_order (4 n each); species, flags (n each)
+  const size_t m = (size_t)n;
+  const double *given[5] = {pos, vel, acel, pos_old, old_cg};
+  int have = 0;
+  size_t bytes = 0;
+  for (int k = 0; k < 5; k++)
+    if (given[k]) {
+      have |= 1 << k;
+      bytes += 24 * m;
+    }
+  const size_t ints = bytes;
+  bytes += 12 * m + 2 * m;
+  unsigned char *dev = staging(c, std::max<size_t>(bytes, 16));
+  if (!dev) return DML_E_NOMEM;
+  std::vector<unsigned char> big;
+  unsigned char *h = pinned(c, bytes);
+  if (!h) {
+    big.resize(bytes + 1);
+    h = big.data();
   }
-  std::vector<int8_t> sp(std::max(n, 1));
-  std::vector<uint8_t> fl(std::max(n, 1));
-  std::vector<int32_t> bk(std::max(n, 1)), rord, rpos(std::max(n, 1), -1);
-  std::vector<uint32_t> pid(std::max(n, 1));
+  {
+    size_t at = 0;
+    for (int k = 0; k < 5; k++)
+      if (given[k]) {
+        memcpy(h + at, given[k], 24 * m);
+        at += 24 * m;
+      }
+  }
+  int32_t *rpos = (int32_t *)(h + ints), *rord = rpos + m, *gco = rord + m;
+  int8_t *sp = (int8_t *)(gco + m);
+  uint8_t *fl = (uint8_t *)(sp + m);
+  int nref = 0, ngc = 0, nat = 0;
   for (int i = 0; i < n; i++) {
     sp[i] = species ? species[i] : (int8_t)SP_LI;
     fl[i] = flags ? flags[i]
                   : (uint8_t)(DML_FL_ALIVE | (sp[i] != SP_CG ? DML_FL_REF : 0) |
                               ((p.reservoir == DML_GCMC && sp[i] == SP_LI) ? DML_FL_GCMC : 0));
-    bk[i] = i;
-    pid[i] = (uint32_t)i;
+    rpos[i] = -1;
     if (fl[i] & DML_FL_REF) {
-      rpos[i] = (int32_t)rord.size();
-      rord.push_back((int32_t)(o + i));
+      rpos[i] = nref;
+      rord[nref++] = (int32_t)(o + i);
     }
+    // the gcmc group in sys order (dana.F90:505-513)
+    if (fl[i] & DML_FL_GCMC) gco[ngc++] = (int32_t)(o + i);
+    nat += fl[i] & DML_FL_ALIVE;
   }
-  HIPCHECK(hipMemcpy(c->d.species + o, sp.data(), n, hipMemcpyHostToDevice));
-  HIPCHECK(hipMemcpy(c->d.flags + o, fl.data(), n, hipMemcpyHostToDevice));
-  HIPCHECK(hipMemcpy(c->d.bkey + o, bk.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-  HIPCHECK(hipMemcpy(c->d.pid + o, pid.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice));
-  HIPCHECK(hipMemcpy(c->d.ref_pos + o, rpos.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-  if (!rord.empty())
-    HIPCHECK(hipMemcpy(c->d.ref_order + o, rord.data(), sizeof(int32_t) * rord.size(),
-                       hipMemcpyHostToDevice));
-  HIPCHECK(hipMemset(c->d.nn + o, 0, sizeof(int32_t) * p.pcap));
-  // a reused replica (serving) starts like a fresh one: no overlap stamps,
-  // no flags beyond n, zero forces
-  for (int32_t *q : c->d.ovq) HIPCHECK(hipMemset(q + o, 0, sizeof(int32_t) * p.pcap));
-  HIPCHECK(hipMemset(c->d.rowflag + o, 0, p.pcap));
-  if (p.pcap > n) HIPCHECK(hipMemset(c->d.flags + o + n, 0, p.pcap - n));
-  {
-    double *z8[] = {c->d.fx, c->d.fy, c->d.fz, c->d.epot, c->d.rvx, c->d.rvy, c->d.rvz};
-    for (double *q : z8) HIPCHECK(hipMemset(q + o, 0, sizeof(double) * p.pcap));
-  }
+  if (n > 0) HIPCHECK(hipMemcpyAsync(dev, h, bytes, hipMemcpyHostToDevice, c->st));
+  hipLaunchKernelGGL(k_load_state, dim3((unsigned)(p.pcap / DML_BLOCK)), dim3(DML_BLOCK), 0, c->st,
+                     c->d, p.poff, n, nref, ngc, have, (const unsigned char *)dev);
   p.ov_round = 0;
   p.ov_pending = 0;
   p.rho_count = 0;
   p.any_ghost = 0;
   p.lohi = 0.0;
   p.d1 = p.d2 = 0.0;
-  // hs%b index table, the gcmc group in sys order (dana.F90:505-513) and
-  // the creation numbers
-  {
-    std::vector<int32_t> b2s(p.pcap, -1), gco, sq(std::max(n, 1));
-    int nat = 0;
-    for (int i = 0; i < n; i++) {
-      sq[i] = i;
-      if (fl[i] & DML_FL_ALIVE) {
-        nat++;
-        b2s[i] = (int32_t)(o + i);
-      }
-      if (fl[i] & DML_FL_GCMC) gco.push_back((int32_t)(o + i));
-    }
-    HIPCHECK(hipMemcpy(c->d.b2slot + o, b2s.data(), sizeof(int32_t) * p.pcap, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->d.seq + o, sq.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    if (!gco.empty())
-      HIPCHECK(hipMemcpy(c->d.gc_order + o, gco.data(), sizeof(int32_t) * gco.size(),
-                         hipMemcpyHostToDevice));
-    p.nat = nat;
-    p.nlimbo = 0;
-    p.b_amax = n;
-    p.b_nat = nat;
-    p.ngc = (int32_t)gco.size();
-    p.pid_next = (uint32_t)n;
-    p.seq_next = n;
-    p.gcmc_calls = 0;
-  }
+  p.nat = nat;
+  p.nlimbo = 0;
+  p.b_amax = n;
+  p.b_nat = nat;
+  p.ngc = ngc;
+  p.pid_next = (uint32_t)n;
+  p.seq_next = n;
+  p.gcmc_calls = 0;
   p.free_lo = 0;
   p.bfree_lo = 0;
-  p.ovn_stamp = 0;
-  // no entries-within-rcut lists for the new atoms until fuerza or a row
-  // build writes them
-  HIPCHECK(hipMemsetAsync(c->d.ov_near + o, 0xff, (size_t)p.pcap, c->st));
+  p.ovn_stamp = 0;  // no entries-within-rcut lists for the new atoms yet
   p.nslots = n;
-  p.nref = (int32_t)rord.size();
+  p.nref = nref;
   p.listed = 0;
   p.rebuild = 0;
   p.any_f = 0;
@@ -1189,11 +1240,8 @@ int dml_set_state(dml_ctx *c, int32_t rep, int32_t n, const double *pos, const d
     p.rho0 = (double)g / (p.box[0] * p.box[1] * (p.zmax - p.z0));
   }
   rc = upload_params(c);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_init_pf4, dim3((unsigned)((c->P + DML_BLOCK - 1) / DML_BLOCK)),
-                     dim3(DML_BLOCK), 0, c->st, c->d, c->P);
-  HIPCHECK(hipStreamSynchronize(c->st));
-  return DML_OK;
+  HIPCHECK(hipStreamSynchronize(c->st));  // the staging is free again
+  return rc;
 }
 
 int dml_set_order(dml_ctx *c, int32_t rep, int32_t nref, const int32_t *ref_order,
@@ -1249,29 +1297,41 @@ int dml_get_state(dml_ctx *c, int32_t rep, int32_t n, double *pos, double *vel, 
                   double *force, double *epot, double *pos_old, double *old_cg, int8_t *species,
                   uint8_t *flags) {
   if (!c || rep < 0 || rep >= c->nrep || n < 0) return DML_E_ARG;
-  HIPCHECK(hipStreamSynchronize(c->st));
   const RepParams &p = c->reps[rep].p;
   if (n > p.pcap) return DML_E_ARG;
-  int64_t o = p.poff;
-  auto get3 = [&](double *dst, double *const *src) -> int {
-    if (!dst) return DML_OK;
-    for (int k = 0; k < 3; k++)
-      HIPCHECK(hipMemcpy(dst + (int64_t)k * n, src[k] + o, sizeof(double) * n, hipMemcpyDeviceToHost));
+  if (n == 0) {
+    HIPCHECK(hipStreamSynchronize(c->st));
     return DML_OK;
-  };
-  double *P3[3] = {c->d.px, c->d.py, c->d.pz};
-  double *V3[3] = {c->d.vx, c->d.vy, c->d.vz};
-  double *A3[3] = {c->d.ax, c->d.ay, c->d.az};
-  double *F3[3] = {c->d.fx, c->d.fy, c->d.fz};
-  double *O3[3] = {c->d.ox, c->d.oy, c->d.oz};
-  double *G3[3] = {c->d.cx, c->d.cy, c->d.cz};
-  int rc;
-  if ((rc = get3(pos, P3)) || (rc = get3(vel, V3)) || (rc = get3(acel, A3)) ||
-      (rc = get3(force, F3)) || (rc = get3(pos_old, O3)) || (rc = get3(old_cg, G3)))
-    return rc;
-  if (epot) HIPCHECK(hipMemcpy(epot, c->d.epot + o, sizeof(double) * n, hipMemcpyDeviceToHost));
-  if (species) HIPCHECK(hipMemcpy(species, c->d.species + o, n, hipMemcpyDeviceToHost));
-  if (flags) HIPCHECK(hipMemcpy(flags, c->d.flags + o, n, hipMemcpyDeviceToHost));
+  }
+  // the asked-for arrays packed by one kernel; in one copy through pinned
+  // memory when they are small (a copy per component, 21 of ~10 us, before), in
+  // one copy an array otherwise
+  void *dst[9] = {pos, vel, acel, force, pos_old, old_cg, epot, species, flags};
+  const size_t m = (size_t)n, size[9] = {24 * m, 24 * m, 24 * m, 24 * m, 24 * m, 24 * m,
+                                         8 * m,  m,      m};
+  int want = 0;
+  size_t bytes = 0;
+  for (int k = 0; k < 9; k++)
+    if (dst[k]) {
+      want |= 1 << k;
+      bytes += size[k];
+    }
+  HIPCHECK(hipStreamSynchronize(c->st));
+  if (!want) return DML_OK;
+  unsigned char *dev = staging(c, bytes);
+  if (!dev) return DML_E_NOMEM;
+  hipLaunchKernelGGL(k_pack_state, dim3((unsigned)((n + DML_BLOCK - 1) / DML_BLOCK)),
+                     dim3(DML_BLOCK), 0, c->st, c->d, p.poff, n, want, dev);
+  unsigned char *h = pinned(c, bytes);
+  if (h) HIPCHECK(hipMemcpyAsync(h, dev, bytes, hipMemcpyDeviceToHost, c->st));
+  HIPCHECK(hipStreamSynchronize(c->st));
+  size_t at = 0;
+  for (int k = 0; k < 9; k++)
+    if (dst[k]) {
+      if (h) memcpy(dst[k], h + at, size[k]);
+      else HIPCHECK(hipMemcpy(dst[k], dev + at, size[k], hipMemcpyDeviceToHost));
+      at += size[k];
+    }
   return DML_OK;
 }
 
@@ -1329,12 +1389,7 @@ int dml_set_box(dml_ctx *c, int32_t rep, const double box[3]) {
   } else {
     p.ccap = oldcap;
   }
-  if (c->gexec) {
-    hipGraphExecDestroy(c->gexec);
-    hipGraphDestroy(c->graph);
-    c->gexec = nullptr;
-    c->graph = nullptr;
-  }
+  // (a captured step is taken again when a buffer it holds has moved)
   return upload_params(c);
 }
 
@@ -1537,11 +1592,13 @@ int dml_observables(dml_ctx *c, double *out) {
   hipLaunchKernelGGL(k_observe_part, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_observe_final, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d);
   std::vector<double> o(4 * (size_t)c->nrep);
-  if (hipMemcpyAsync(o.data(), c->d.obs + 4 * (int64_t)c->d.nblocks, o.size() * sizeof(double),
-                     hipMemcpyDeviceToHost, c->st) != hipSuccess)
+  unsigned char *h = pinned(c, o.size() * sizeof(double));
+  if (hipMemcpyAsync(h ? (void *)h : (void *)o.data(), c->d.obs + 4 * (int64_t)c->d.nblocks,
+                     o.size() * sizeof(double), hipMemcpyDeviceToHost, c->st) != hipSuccess)
     return DML_E_HIP;
   int rc = finish(c);
   if (rc) return rc;
+  if (h) memcpy(o.data(), h, o.size() * sizeof(double));
   // kB_ui of dana.F90:22-24, the constant kion divides by
   const double kB_eVK = 8.617330350e-5, kJm_ui = 100.0, eV_kJm = 96.485;
   const double kB_ui = kB_eVK * (eV_kJm * kJm_ui);
@@ -1735,33 +1792,36 @@ int dml_gcmc_trial_energy(dml_ctx *c, int32_t rep, int32_t ntrial, const double 
     }
     if (exclude && (exclude[t] < (pos3 ? -1 : 0) || exclude[t] >= p.nslots)) return DML_E_ARG;
   }
-  double *dp = nullptr, *de = nullptr;
-  int32_t *dx = nullptr, *dh = nullptr;
-  rc = DML_E_NOMEM;
-  if ((!pos3 || !dalloc(&dp, 3 * (int64_t)ntrial)) && !dalloc(&de, ntrial) &&
-      !dalloc(&dh, ntrial) && (!exclude || !dalloc(&dx, ntrial))) {
-    rc = DML_OK;
-    if ((pos3 && hipMemcpyAsync(dp, pos3, sizeof(double) * 3 * (size_t)ntrial,
-                                hipMemcpyHostToDevice, c->st) != hipSuccess) ||
-        (exclude && hipMemcpyAsync(dx, exclude, sizeof(int32_t) * (size_t)ntrial,
-                                   hipMemcpyHostToDevice, c->st) != hipSuccess))
-      rc = DML_E_HIP;
+  // one staging block each way, kept between calls: points | exclude up,
+  // energies | hard-core flags (and the replica table) down.  Allocated and
+  // freed per call, with a copy per array, 96 trials took 278 us and 8,192
+  // trials 490
+  const size_t n = (size_t)ntrial, np = pos3 ? 24 * n : 0, nx = exclude ? 4 * n : 0;
+  const size_t up = np + nx, off = (up + 15) / 16 * 16, down = 12 * n;
+  unsigned char *d = staging(c, off + down);
+  if (!d) return DML_E_NOMEM;
+  std::vector<unsigned char> big;
+  unsigned char *h = pinned(c, std::max(up, down));
+  if (!h) {
+    big.resize(std::max(up, down));
+    h = big.data();
   }
-  if (!rc) {
-    int64_t threads = (int64_t)ntrial * 64;
-    hipLaunchKernelGGL(k_gcmc_energy, dim3((unsigned)((threads + DML_BLOCK - 1) / DML_BLOCK)),
-                       dim3(DML_BLOCK), 0, c->st, c->d, rep, ntrial, (const double *)dp,
-                       (const int32_t *)dx, de, dh);
-    rc = finish(c);
-  }
-  if (!rc && (hipMemcpy(du, de, sizeof(double) * ntrial, hipMemcpyDeviceToHost) != hipSuccess ||
-              hipMemcpy(hard, dh, sizeof(int32_t) * ntrial, hipMemcpyDeviceToHost) != hipSuccess))
-    rc = DML_E_HIP;
-  hipFree(dp);
-  hipFree(de);
-  hipFree(dh);
-  hipFree(dx);
-  return rc;
+  if (pos3) memcpy(h, pos3, np);
+  if (exclude) memcpy(h + np, exclude, nx);
+  double *de = (double *)(d + off);
+  int32_t *dh = (int32_t *)(d + off + 8 * n);
+  HIPCHECK(hipMemcpyAsync(d, h, up, hipMemcpyHostToDevice, c->st));
+  const int64_t threads = (int64_t)ntrial * 64;
+  hipLaunchKernelGGL(k_gcmc_energy, dim3((unsigned)((threads + DML_BLOCK - 1) / DML_BLOCK)),
+                     dim3(DML_BLOCK), 0, c->st, c->d, rep, ntrial,
+                     (const double *)(pos3 ? d : nullptr),
+                     (const int32_t *)(exclude ? d + np : nullptr), de, dh);
+  HIPCHECK(hipMemcpyAsync(h, de, down, hipMemcpyDeviceToHost, c->st));
+  rc = finish(c);
+  if (rc) return rc;
+  memcpy(du, h, 8 * n);
+  memcpy(hard, h + 8 * n, 4 * n);
+  return DML_OK;
 }
 
 int dml_gcmc_trial_energy_noalloc(dml_ctx *c, int32_t rep, int32_t ntrial, const double *pos3,
@@ -1864,6 +1924,7 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     c->graph_modes = modes;
     c->graph_dsig = dsig;
   }
+  c->fresh = 0;
   HIPCHECK(hipEventRecord(c->e0, c->st));
   for (int q = 0; q < nsteps; q++) {
     if (use_graph)

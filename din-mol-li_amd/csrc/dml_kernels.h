@@ -4,7 +4,9 @@
 
 __global__ void k_pbc_dispmax(DevState s);
 __global__ void k_dispmax_final(DevState s, int begin);
-__global__ void k_init_pf4(DevState s, int64_t n);
+__global__ void k_load_state(DevState s, int poff, int n, int nref, int ngc, int have,
+                             const unsigned char *in);
+__global__ void k_pack_state(DevState s, int poff, int n, int want, unsigned char *out);
 __global__ void k_force_rebuild(DevState s);
 __global__ void k_zero_cells(DevState s, int gcs);
 __global__ void k_cell_key(DevState s, int gcs);

@@ -2556,9 +2556,95 @@ __global__ void k_ov_end(DevState s, int rounds) {
   if (s.ov_last[r] == rounds - 1) rep_fail(s, r, ERR_OVERLAP);
 }
 
-__global__ void k_init_pf4(DevState s, int64_t n) {
-  int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q < n) put_pf4(s, (int)q, s.px[q], s.py[q], s.pz[q], s.species[q]);
+// dml_set_state: n atoms from one block (pos, then the given of vel, acel,
+// pos_old, old_cg: bits 0-4 of `have`, 3 n doubles each; ref_pos, ref_order,
+// gc_order; species; flags) into the replica at poff, with the defaults of
+// atom_allocate / config_inic, and the slots beyond n emptied
+__global__ void __launch_bounds__(DML_BLOCK) k_load_state(DevState s, int poff, int n, int nref,
+                                                          int ngc, int have,
+                                                          const unsigned char *in) {
+  const int k = blockIdx.x * DML_BLOCK + threadIdx.x;  // (a block per 256 slots of the replica)
+  const int i = poff + k;
+  s.nn[i] = 0;
+  s.ovq[0][i] = s.ovq[1][i] = 0;
+  s.rowflag[i] = 0;
+  s.fx[i] = s.fy[i] = s.fz[i] = s.epot[i] = 0.0;
+  s.rvx[i] = s.rvy[i] = s.rvz[i] = 0.0;
+  s.ov_near[i] = 255;
+  if (k >= n) {
+    s.flags[i] = 0;
+    s.b2slot[i] = -1;
+    put_pf4(s, i, s.px[i], s.py[i], s.pz[i], s.species[i]);
+    return;
+  }
+  const double *d = reinterpret_cast<const double *>(in);
+  const double x = d[k], y = d[n + k], z = d[2 * (int64_t)n + k];
+  d += 3 * (int64_t)n;
+  auto next = [&](int bit, double &a, double &b, double &c) {
+    if (!(have >> bit & 1)) return;
+    a = d[k];
+    b = d[n + k];
+    c = d[2 * (int64_t)n + k];
+    d += 3 * (int64_t)n;
+  };
+  double vx = 0.0, vy = 0.0, vz = 0.0, ax = 0.0, ay = 0.0, az = 0.0;
+  double ox = x, oy = y, oz = z, cx = 1e8, cy = 1e8, cz = 1e8;
+  next(1, vx, vy, vz);
+  next(2, ax, ay, az);
+  next(3, ox, oy, oz);
+  next(4, cx, cy, cz);
+  const int32_t *q = reinterpret_cast<const int32_t *>(d);
+  const int8_t *sp = reinterpret_cast<const int8_t *>(q + 3 * (int64_t)n);
+  const uint8_t fl = reinterpret_cast<const uint8_t *>(sp + n)[k];
+  s.px[i] = x; s.py[i] = y; s.pz[i] = z;
+  s.vx[i] = vx; s.vy[i] = vy; s.vz[i] = vz;
+  s.ax[i] = ax; s.ay[i] = ay; s.az[i] = az;
+  s.ox[i] = ox; s.oy[i] = oy; s.oz[i] = oz;
+  s.cx[i] = cx; s.cy[i] = cy; s.cz[i] = cz;
+  s.species[i] = sp[k];
+  s.flags[i] = fl;
+  s.bkey[i] = k;
+  s.pid[i] = (uint32_t)k;
+  s.seq[i] = k;
+  s.b2slot[i] = (fl & DML_FL_ALIVE) ? i : -1;
+  s.ref_pos[i] = q[k];
+  if (k < nref) s.ref_order[i] = q[n + k];
+  if (k < ngc) s.gc_order[i] = q[2 * (int64_t)n + k];
+  put_pf4(s, i, x, y, z, sp[k]);
+}
+
+// dml_get_state: the first n slots' asked-for arrays (bits of `want`: pos, vel,
+// acel, force, pos_old, old_cg of 3 n doubles, epot of n, species and flags of
+// n bytes), one after the other
+__global__ void __launch_bounds__(DML_BLOCK) k_pack_state(DevState s, int poff, int n, int want,
+                                                          unsigned char *out) {
+  const int k = blockIdx.x * DML_BLOCK + threadIdx.x;
+  if (k >= n) return;
+  const int i = poff + k;
+  double *d = reinterpret_cast<double *>(out);
+  auto put = [&](int bit, const double *a, const double *b, const double *c) {
+    if (!(want >> bit & 1)) return;
+    d[k] = a[i];
+    d[n + k] = b[i];
+    d[2 * (int64_t)n + k] = c[i];
+    d += 3 * (int64_t)n;
+  };
+  put(0, s.px, s.py, s.pz);
+  put(1, s.vx, s.vy, s.vz);
+  put(2, s.ax, s.ay, s.az);
+  put(3, s.fx, s.fy, s.fz);
+  put(4, s.ox, s.oy, s.oz);
+  put(5, s.cx, s.cy, s.cz);
+  if (want >> 6 & 1) {
+    d[k] = s.epot[i];
+    d += n;
+  }
+  uint8_t *b = reinterpret_cast<uint8_t *>(d);
+  if (want >> 7 & 1) {
+    b[k] = (uint8_t)s.species[i];
+    b += n;
+  }
+  if (want >> 8 & 1) b[k] = s.flags[i];
 }
 
 __global__ void k_zero_i32(int32_t *a, int64_t n) {
