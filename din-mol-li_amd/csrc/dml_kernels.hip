@@ -3843,9 +3843,10 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
 // So every trial's point, its hard-core neighbours among the atoms present
 // at the call's start and the earlier trial points within rcut can be found
 // in parallel (k_gb_trials, k_gb_conflicts).  What stays sequential is the
-// count n of the control volume and which atoms are present: one wave walks
-// the trials (k_gb_decide) with the in-volume list in LDS as a bitmap
-// (deletions take the m-th present entry, insertions append), and a second
+// count n of the control volume and which atoms are present: one wave decides
+// the trials in order, 64 at a time (k_gb_decide), with the in-volume list in
+// LDS as a bitmap (deletions take the m-th present entry, insertions append),
+// and a second
 // wave walks the accepted moves (k_gb_commit) for the hs%b indices (lowest
 // free first, indices freed in this call included), the template and the
 // list tail that the reference's insertion reads, and the ordered stores of
@@ -4196,19 +4197,35 @@ __global__ void __launch_bounds__(DML_BLOCK) k_gb_conflicts(DevState s, int r) {
 }
 
 
-// the decisions, one wave walking the trials in order (dana.F90:621-710):
-// n, the Metropolis tests, the hard-core test against the neighbours still
-// present and the earlier points accepted and still present, and for a
-// deletion the m-th present entry of the in-volume list (list order, the
-// call's insertions appended).  The list is a bitmap in LDS with per-chunk
-// counts (1024 entries a chunk, 16 chunks a lane, lane totals in registers).
-// Nothing of the replica's state is written here.
+// the decisions (dana.F90:621-710): n, the Metropolis tests, the hard-core
+// test against the neighbours still present and the earlier points accepted
+// and still present, and for a deletion the m-th present entry of the
+// in-volume list (list order, the call's insertions appended).  The list is a
+// bitmap in LDS with per-chunk counts (1024 entries a chunk, 16 chunks a lane,
+// lane totals in registers).  Nothing of the replica's state is written here.
+//
+// One wave decides 64 trials at a time, a lane each, exactly as one after the
+// other would.  With the neighbours of the batch's start, which trials pass
+// depends on the earlier ones only through n: repeating "count the accepted
+// before me, test again" settles at least one more trial a time (mostly all of
+// them in two).  An accepted deletion takes rank m-1 of the list as it is then;
+// undoing the batch's earlier deletions from the last to the first (one that
+// took rank q moves ranks >= q up by one) gives its rank in the list of the
+// batch's start, which each lane looks up by itself.  A batch with points
+// within rcut of each other, or whose deletions free a point that was taken,
+// is walked trial by trial instead.
+// What bounds it: one wave's LDS latency, a few thousand cycles a batch: 0.60
+// ms a call of 8,192 trials over 10^6 entries (trial by trial 4.27 ms).
+struct GbBatch {  // one trial per lane
+  int kind, nblk, ncf, thr;
+  double u2;
+  int4 blk[GB_NB / 4], cf[GB_NC / 4];
+};
 __global__ void __launch_bounds__(WAVE) k_gb_decide(DevState s, int r) {
-  __shared__ uint32_t vb[GB_VWORDS];
-  __shared__ int32_t ccnt[WAVE * 16];
+  __shared__ __align__(16) uint32_t vb[GB_VWORDS];
+  __shared__ __align__(16) int32_t ccnt[WAVE * 16];
+  __shared__ int32_t gpre[WAVE];  // entries present before a lane's chunks
   __shared__ int32_t res[DML_GCMC_BATCH_MAX];
-  // the neighbour lists of 64 trials, double-buffered: [buffer][trial][entry]
-  __shared__ int32_t lblk[2][WAVE][GB_NB], lcf[2][WAVE][GB_NC];
   RepParams *Pw = s.rp + r;
   if (!gb_on(*Pw)) return;
   const int lane = threadIdx.x;
@@ -4225,161 +4242,305 @@ __global__ void __launch_bounds__(WAVE) k_gb_decide(DevState s, int r) {
     ccnt[c] = v;
     tot += v;
   }
-  // and in the chunks of lanes 0 .. lane (kept up to date, not rescanned)
-  int pre = wave_scan_incl(tot);
-  // each trial's result (insertion rank, in-volume position, -1): the walk
-  // writes it to LDS only; the per-trial and per-move records in memory are
-  // written from it after the walk, 64 trials at a time
-  for (int q = lane; q < T; q += WAVE) res[q] = -1;
-  // per-trial data of a 64-trial chunk and its lists, loaded into
-  // registers one chunk ahead and staged into LDS at the chunk's start, so
-  // that the walk reads LDS and never waits on memory (a load result kept
-  // in a register across the loop would make every iteration wait for the
-  // iteration's own stores too); the walk is one wave, whose LDS accesses
-  // execute in program order
-  __shared__ int32_t lkind[2][WAVE], lnblk[2][WAVE], lncf[2][WAVE];
-  __shared__ double lu1[2][WAVE], lu2[2][WAVE];
-  int p_kind = 0, p_nblk = 0, p_ncf = 0;
-  double p_u1 = 0.0, p_u2 = 0.0;
-  int pb[GB_NB], pc[GB_NC];
-  auto load_chunk = [&](int t0) {
+  int pre = wave_scan_incl(tot);  // and in the chunks of lanes 0 .. lane
+  gpre[lane] = pre - tot;
+  auto present = [&](int vp) -> int { return (int)(vb[vp >> 5] >> (vp & 31)) & 1; };
+  // the trials of the batch at t0, loaded one batch ahead
+  GbBatch B, N;
+  auto load = [&](GbBatch &X, int t0) {
     const int q = t0 + lane;
+    X.kind = 3;  // (past the end: nothing)
+    X.nblk = X.ncf = X.thr = 0;
+    X.u2 = 0.0;
     if (q < T) {
-      p_kind = s.gb_kind[off + q];
-      p_nblk = s.gb_nblk[off + q];
-      p_ncf = s.gb_ncf[off + q];
-      p_u1 = s.gb_u[2 * (off + q)];
-      p_u2 = s.gb_u[2 * (off + q) + 1];
-    }
-    // the lists of the chunk's 64 trials, 16 entries each: coalesced
+      X.kind = s.gb_kind[off + q];
+      X.nblk = s.gb_nblk[off + q];
+      X.ncf = s.gb_ncf[off + q];
+      X.thr = (int)s.gb_u[2 * (off + q)];  // the Metropolis threshold on n
+      X.u2 = s.gb_u[2 * (off + q) + 1];
 #pragma unroll
-    for (int j = 0; j < GB_NB; j++) {
-      const int64_t e = (int64_t)(off + t0) * GB_NB + j * WAVE + lane;
-      pb[j] = t0 + (j * WAVE + lane) / GB_NB < T ? s.gb_blk[e] : 0;
-    }
+      for (int k = 0; k < GB_NB / 4; k++)
+        X.blk[k] = *(const int4 *)(s.gb_blk + (int64_t)(off + q) * GB_NB + 4 * k);
 #pragma unroll
-    for (int j = 0; j < GB_NC; j++) {
-      const int64_t e = (int64_t)(off + t0) * GB_NC + j * WAVE + lane;
-      pc[j] = t0 + (j * WAVE + lane) / GB_NC < T ? s.gb_cf[e] : 0;
+      for (int k = 0; k < GB_NC / 4; k++)
+        X.cf[k] = *(const int4 *)(s.gb_cf + (int64_t)(off + q) * GB_NC + 4 * k);
     }
   };
-  auto stage_chunk = [&](int buf) {
-    lkind[buf][lane] = p_kind;
-    lnblk[buf][lane] = p_nblk;
-    lncf[buf][lane] = p_ncf;
-    lu1[buf][lane] = p_u1;
-    lu2[buf][lane] = p_u2;
-#pragma unroll
-    for (int j = 0; j < GB_NB; j++) {
-      const int e = j * WAVE + lane;
-      lblk[buf][e / GB_NB][e % GB_NB] = pb[j];
-    }
-#pragma unroll
-    for (int j = 0; j < GB_NC; j++) {
-      const int e = j * WAVE + lane;
-      lcf[buf][e / GB_NC][e % GB_NC] = pc[j];
-    }
-  };
-  load_chunk(0);
+  load(N, 0);
   __syncthreads();
   int n = ilen, nins = 0, ndel = 0;
   int fail = 0;
-  for (int t = 0; t < T && !fail; t++) {
-    const int a = t & (WAVE - 1);
-    const int buf = (t / WAVE) & 1;
-    if (a == 0) {
-      stage_chunk(buf);
-      if (t + WAVE < T) load_chunk(t + WAVE);
-      __builtin_amdgcn_wave_barrier();
-    }
-    const int kind = lkind[buf][a];
-    const int nblk = lnblk[buf][a];
-    const int ncf = lncf[buf][a];
-    const int thr = (int)lu1[buf][a];  // the Metropolis threshold on n
-    const double u2 = lu2[buf][a];
-    int out = -1;
-    if (kind == 2) {
+  for (int t0 = 0; t0 < T && !fail; t0 += WAVE) {
+    B = N;
+    if (t0 + WAVE < T) load(N, t0 + WAVE);
+    __builtin_amdgcn_wave_barrier();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (__ballot(B.kind == 2)) {
       fail = 1;  // a point outside the cells: the sequential kernel's error path
-    } else if (kind == 0) {
-      if (n <= thr && nblk >= 0) {
-        if (nblk > GB_NB || ncf > GB_NC) {
-          fail = 1;
-        } else {
-          int here = 0;
-          if (lane < nblk) {
-            const int vp = lblk[buf][a][lane];
-            here = (vb[vp >> 5] >> (vp & 31)) & 1;
-          } else if (lane >= GB_NB && lane < GB_NB + ncf) {
-            const int k = res[lcf[buf][a][lane - GB_NB]];  // an earlier insertion: accepted, still present?
-            if (k >= 0) {
-              const int vp = ilen + k;
-              here = (vb[vp >> 5] >> (vp & 31)) & 1;
-            }
-          }
-          if (!__ballot(here)) {
-            const int k = nins++;
-            const int vp = ilen + k;
-            if (lane == 0) {
-              vb[vp >> 5] |= 1u << (vp & 31);
-              ccnt[vp >> 10]++;
-            }
-            if (lane == (vp >> 14)) tot++;
-            if (lane >= (vp >> 14)) pre++;
-            n++;
-            out = k;
+      break;
+    }
+    const bool ins = B.kind == 0 && B.nblk >= 0;
+    const bool big = B.nblk > GB_NB || B.ncf > GB_NC;
+    // is a neighbour of this lane's point, or an earlier point, there now?
+    // (same: an earlier point of this batch, whose trial is not decided yet)
+    auto taken = [&](int &same) -> int {
+      int here = 0;
+      same = 0;
+#pragma unroll
+      for (int k = 0; k < GB_NB; k++) {
+        if (!__ballot(ins && !big && k < B.nblk)) break;
+        const int4 v = B.blk[k / 4];
+        const int vp = k % 4 == 0 ? v.x : k % 4 == 1 ? v.y : k % 4 == 2 ? v.z : v.w;
+        if (ins && !big && k < B.nblk) here |= present(vp);
+      }
+#pragma unroll
+      for (int k = 0; k < GB_NC; k++) {
+        if (!__ballot(ins && !big && k < B.ncf)) break;
+        const int4 v = B.cf[k / 4];
+        const int tp = k % 4 == 0 ? v.x : k % 4 == 1 ? v.y : k % 4 == 2 ? v.z : v.w;
+        if (ins && !big && k < B.ncf) {
+          if (tp >= t0) {
+            same = 1;
+          } else {
+            const int j = res[tp];  // an earlier insertion: accepted, still present?
+            if (j >= 0) here |= present(ilen + j);
           }
         }
       }
-    } else {
-      if (n >= thr) {
-        int m = (int)floor(u2 * n) + 1;
-        if (m > n) m = n;
-        if (m < 1) {
-          fail = 1;  // nothing to delete: the sequential kernel reports it
+      return here;
+    };
+    int same;
+    const int here = taken(same);
+    bool slow = __ballot(ins && !here && same) != 0;
+    int out = -1;
+    if (!slow) {
+      const bool can = ins && !here && !big;
+      unsigned long long ai = 0, ad = 0;
+      int nt = n;
+      for (;;) {
+        nt = n + __popcll(ai & below) - __popcll(ad & below);
+        const unsigned long long bi = __ballot(can && nt <= B.thr);
+        const unsigned long long bd = __ballot(B.kind == 1 && nt >= B.thr);
+        if (bi == ai && bd == ad) break;
+        ai = bi;
+        ad = bd;
+      }
+      const bool is_i = ai >> lane & 1ull, is_d = ad >> lane & 1ull;
+      int m = (int)floor(B.u2 * nt) + 1;
+      if (m > nt) m = nt;
+      // more neighbours than listed, or nothing to delete: the sequential
+      // kernel decides or reports it
+      if (__ballot((ins && big && nt <= B.thr) || (is_d && m < 1))) {
+        fail = 1;
+        break;
+      }
+      const int rem = m - 1;
+      int y = rem;  // -> rank among the entries of the batch's start, then its insertions
+      for (unsigned long long w = ad; w;) {
+        const int q = 63 - __builtin_clzll(w);
+        w &= ~(1ull << q);
+        const int rq = __builtin_amdgcn_readlane(rem, q);
+        if (lane > q) y += y >= rq;
+      }
+      const int ki = nins + __popcll(ai & below);  // rank of this lane's insertion
+      int p = -1;
+      if (is_d) {
+        if (y >= n) {
+          p = ilen + nins + (y - n);
         } else {
-          // the (m-1)-th present entry: lane, chunk, word, bit (each level's
-          // ballot is non-empty while the counts agree with the bitmap)
-          int rem = m - 1;
-          const unsigned long long b1 = __ballot(pre > rem);
-          const int L = b1 ? __builtin_ctzll(b1) : 0;
-          rem -= __builtin_amdgcn_readlane(pre - tot, L);
-          const int c16 = lane < 16 ? ccnt[16 * L + lane] : 0;
-          const int incl2 = row_scan16(c16);
-          const unsigned long long b2 = __ballot(lane < 16 && incl2 > rem);
-          const int j = b2 ? __builtin_ctzll(b2) : 0;
-          rem -= __builtin_amdgcn_readlane(incl2 - c16, j);
-          const int chunk = 16 * L + j;
-          const uint32_t wv = lane < 32 ? vb[32 * chunk + lane] : 0u;
-          const int pc1 = __popc(wv);
-          const int incl3 = half_scan32(pc1);
-          const unsigned long long b3 = __ballot(lane < 32 && incl3 > rem);
-          const int k = b3 ? __builtin_ctzll(b3) : 0;
-          rem -= __builtin_amdgcn_readlane(incl3 - pc1, k);
-          const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)wv, k);
-          const unsigned long long b4 = __ballot(
-              lane < 32 && ((word >> (lane & 31)) & 1u) &&
-              __popc(word & ((1u << (lane & 31)) - 1u)) == rem);
-          const int bit = b4 ? __builtin_ctzll(b4) : 0;
-          if (!b1 || !b2 || !b3 || !b4 || chunk >= GB_CHUNKS) {
-            fail = 1;  // cannot happen; leave the call to the sequential kernel
-            break;
+          // the y-th present entry: lane group, chunk, word, bit
+          int L = 0;
+#pragma unroll
+          for (int st = WAVE / 2; st > 0; st >>= 1)
+            if (gpre[L + st] <= y) L += st;
+          int x = y - gpre[L], acc = 0, base = 0, c = 0;
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            const int4 v = *(const int4 *)(ccnt + 16 * L + 4 * k);
+            const int e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              acc += e[j];
+              const int ge = x >= acc;
+              c += ge;
+              base = ge ? acc : base;
+            }
           }
-          const int p = chunk * 1024 + k * 32 + bit;
-          if (lane == 0) {
-            vb[32 * chunk + k] = word & ~(1u << bit);
-            ccnt[chunk]--;
+          x -= base;
+          const int chunk = 16 * L + c;
+          uint32_t word = 0;
+          int kw = 0;
+          acc = base = 0;
+          if (chunk < GB_CHUNKS) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+              const uint4 v = *(const uint4 *)(vb + 32 * chunk + 4 * k);
+              const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+              for (int j = 0; j < 4; j++) {
+                const int before = acc;
+                acc += __popc(e[j]);
+                const bool hit = x >= before && x < acc;
+                word = hit ? e[j] : word;
+                kw = hit ? 4 * k + j : kw;
+                base = hit ? before : base;
+              }
+            }
+            x -= base;
+            int bit = 0;
+#pragma unroll
+            for (int st = 16; st > 0; st >>= 1) {
+              const int cl = __popc(word >> bit & ((1u << st) - 1u));
+              const int ge = x >= cl;
+              x -= ge ? cl : 0;
+              bit += ge ? st : 0;
+            }
+            if (word >> bit & 1u) p = chunk * 1024 + kw * 32 + bit;
           }
-          if (lane == L) tot--;
-          if (lane >= L) pre--;
-          ndel++;
-          n--;
-          out = p;
         }
+      }
+      if (__ballot(is_d && p < 0)) {
+        fail = 1;  // cannot happen; leave the call to the sequential kernel
+        break;
+      }
+      const int vi = ilen + ki;
+      auto flip = [&](bool mine, int vp, int on) {
+        if (mine) {
+          if (on) atomicOr(&vb[vp >> 5], 1u << (vp & 31));
+          else atomicAnd(&vb[vp >> 5], ~(1u << (vp & 31)));
+          atomicAdd(&ccnt[vp >> 10], on ? 1 : -1);
+        }
+        __builtin_amdgcn_wave_barrier();
+      };
+      __builtin_amdgcn_wave_barrier();
+      flip(is_i, vi, 1);
+      flip(is_d, p, 0);
+      // a point taken at the batch's start and free after its deletions: the
+      // order inside the batch matters
+      int again;
+      const int here2 = taken(again);
+      slow = __ballot(ins && !big && here && !here2) != 0;
+      if (slow) {
+        flip(is_d, p, 1);
+        flip(is_i, vi, 0);
+      } else {
+        out = is_i ? ki : is_d ? p : -1;
+        if (t0 + lane < T) res[t0 + lane] = out;
+        nins += __popcll(ai);
+        ndel += __popcll(ad);
+        n += __popcll(ai) - __popcll(ad);
+        tot = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int4 v = *(const int4 *)(ccnt + 16 * lane + 4 * k);
+          tot += v.x + v.y + v.z + v.w;
+        }
+        pre = wave_scan_incl(tot);
+        gpre[lane] = pre - tot;
       }
     }
-    if (lane == 0) res[t] = out;
+    if (slow) {
+      // trial by trial
+      for (int a = 0; a < WAVE && t0 + a < T && !fail; a++) {
+        const int kind = __builtin_amdgcn_readlane(B.kind, a);
+        const int thr = __builtin_amdgcn_readlane(B.thr, a);
+        out = -1;
+        if (kind == 0) {
+          const int nblk = __builtin_amdgcn_readlane(B.nblk, a);
+          const int ncf = __builtin_amdgcn_readlane(B.ncf, a);
+          if (n <= thr && nblk >= 0) {
+            if (nblk > GB_NB || ncf > GB_NC) {
+              fail = 1;
+              break;
+            }
+            int there = 0;
+            if (lane == a) {
+#pragma unroll
+              for (int k = 0; k < GB_NB; k++) {
+                const int4 v = B.blk[k / 4];
+                const int vp = k % 4 == 0 ? v.x : k % 4 == 1 ? v.y : k % 4 == 2 ? v.z : v.w;
+                if (k < nblk) there |= present(vp);
+              }
+#pragma unroll
+              for (int k = 0; k < GB_NC; k++) {
+                const int4 v = B.cf[k / 4];
+                const int tp = k % 4 == 0 ? v.x : k % 4 == 1 ? v.y : k % 4 == 2 ? v.z : v.w;
+                if (k < ncf) {
+                  const int j = res[tp];
+                  if (j >= 0) there |= present(ilen + j);
+                }
+              }
+            }
+            if (!__ballot(there)) {
+              const int k = nins++;
+              const int vp = ilen + k;
+              if (lane == 0) {
+                vb[vp >> 5] |= 1u << (vp & 31);
+                ccnt[vp >> 10]++;
+              }
+              if (lane == (vp >> 14)) tot++;
+              if (lane >= (vp >> 14)) pre++;
+              n++;
+              out = k;
+            }
+          }
+        } else {
+          if (n >= thr) {
+            int m = (int)floor(rdlane_d(B.u2, a) * n) + 1;
+            if (m > n) m = n;
+            if (m < 1) {
+              fail = 1;  // nothing to delete: the sequential kernel reports it
+              break;
+            }
+            // the (m-1)-th present entry: lane, chunk, word, bit (each level's
+            // ballot is non-empty while the counts agree with the bitmap)
+            int rem = m - 1;
+            const unsigned long long b1 = __ballot(pre > rem);
+            const int L = b1 ? __builtin_ctzll(b1) : 0;
+            rem -= __builtin_amdgcn_readlane(pre - tot, L);
+            const int c16 = lane < 16 ? ccnt[16 * L + lane] : 0;
+            const int incl2 = row_scan16(c16);
+            const unsigned long long b2 = __ballot(lane < 16 && incl2 > rem);
+            const int j = b2 ? __builtin_ctzll(b2) : 0;
+            rem -= __builtin_amdgcn_readlane(incl2 - c16, j);
+            const int chunk = 16 * L + j;
+            const uint32_t wv = lane < 32 && chunk < GB_CHUNKS ? vb[32 * chunk + lane] : 0u;
+            const int pc1 = __popc(wv);
+            const int incl3 = half_scan32(pc1);
+            const unsigned long long b3 = __ballot(lane < 32 && incl3 > rem);
+            const int k = b3 ? __builtin_ctzll(b3) : 0;
+            rem -= __builtin_amdgcn_readlane(incl3 - pc1, k);
+            const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)wv, k);
+            const unsigned long long b4 = __ballot(
+                lane < 32 && ((word >> (lane & 31)) & 1u) &&
+                __popc(word & ((1u << (lane & 31)) - 1u)) == rem);
+            const int bit = b4 ? __builtin_ctzll(b4) : 0;
+            if (!b1 || !b2 || !b3 || !b4) {
+              fail = 1;  // cannot happen; leave the call to the sequential kernel
+              break;
+            }
+            if (lane == 0) {
+              vb[32 * chunk + k] = word & ~(1u << bit);
+              ccnt[chunk]--;
+            }
+            if (lane == L) tot--;
+            if (lane >= L) pre--;
+            ndel++;
+            n--;
+            out = chunk * 1024 + k * 32 + bit;
+          }
+        }
+        if (lane == 0) res[t0 + a] = out;
+        __builtin_amdgcn_wave_barrier();
+      }
+      gpre[lane] = pre - tot;
+    }
     __builtin_amdgcn_wave_barrier();
   }
+  // (a call that falls back leaves no results to read)
+  if (fail)
+    for (int q = lane; q < T; q += WAVE) res[q] = -1;
+  __syncthreads();
   // the records of the walk, in trial order: every trial's result, each
   // insertion's trial (its rank is its result), each deletion's trial and
   // position in deletion order; then, once those are written, the trial

@@ -181,6 +181,12 @@ inline T atomicOr(T *p, U v) {
   return o;
 }
 template <class T, class U>
+inline T atomicAnd(T *p, U v) {
+  T o = *p;
+  *p = o & (T)v;
+  return o;
+}
+template <class T, class U>
 inline T atomicMax(T *p, U v) {
   T o = *p;
   if ((T)v > o) *p = (T)v;
