@@ -467,6 +467,16 @@ int64_t live_slots(const dml_ctx *c) {
   return n;
 }
 
+// The force kernel takes the atoms of a system of FO_LEAST slots or more cell
+// by cell (list and ermak_b cost two launches): 4 steps of a dendrite of 2M
+// atoms 43.4 -> 37.3 ms, 600,000 12.7 -> 11.5, 300,000 9.7 -> 9.6, 150,000 even; 80
+// steps of 100,000 dense atoms 29.8 -> 30.5
+bool by_cell(const dml_ctx *c) {
+  for (auto &h : c->reps)
+    if (!h.p.halted && h.p.integrator == DML_ERMAK && h.p.nslots >= FO_LEAST) return true;
+  return false;
+}
+
 void enq_listbuild(dml_ctx *c) {
   if (c->any_lb[0] && c->d.n_tm > 0)
     hipLaunchKernelGGL(k_listbuild_cells, dim3(clamp_grid(c->d.n_tm)), dim3(DML_BLOCK), 0, c->st,
@@ -523,6 +533,9 @@ void enq_cells_lists(dml_ctx *c, int gcs) {
   hipLaunchKernelGGL(k_zero_cells, gc, dim3(DML_BLOCK), 0, c->st, c->d, gcs);
   hipLaunchKernelGGL(k_cell_key, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d, gcs);
   hipLaunchKernelGGL(k_cell_sort_w, gw, dim3(DML_BLOCK), 0, c->st, c->d, gcs);
+  if (by_cell(c))
+    hipLaunchKernelGGL(k_force_order, dim3(clamp_grid((c->d.n_cm + 63) / 64)), dim3(FO_BLOCK), 0,
+                       c->st, c->d);
   enq_listbuild(c);
 }
 
@@ -550,14 +563,15 @@ void launch_force_lpa(dml_ctx *c, int lpa, int only_ermak) {
 
 void enq_forces(dml_ctx *c, int fuse_b, int only_ermak) {
   c->fresh = 0;
-  if (fuse_b)
+  const int fused = fuse_b && !by_cell(c);
+  if (fused)
     launch_force_lpa<1>(c, c->lpa, only_ermak);
   else
     launch_force_lpa<0>(c, c->lpa, only_ermak);
   hipLaunchKernelGGL(k_ghost_scatter, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d,
                      only_ermak);
   if (fuse_b)
-    hipLaunchKernelGGL(k_ermak_b, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d, 1);
+    hipLaunchKernelGGL(k_ermak_b, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d, fused);
 }
 
 // begun: the test_update before has started the rounds (k_dispmax_final)
@@ -987,6 +1001,7 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
   e |= dalloc(&d.pid, P);
   e |= dalloc(&d.ref_order, P);
   e |= dalloc(&d.ref_tmp, P);
+  e |= dalloc(&d.ford, P);
   e |= dalloc(&d.ref_pos, P);
   e |= dalloc(&d.nn, P);
   e |= dalloc(&d.nbr, P * (int64_t)maxnn);
@@ -1115,7 +1130,7 @@ int dml_destroy(dml_ctx *c) {
   void *ptrs[] = {d.px, d.py, d.pz, d.vx, d.vy, d.vz, d.ax, d.ay, d.az, d.fx, d.fy, d.fz,
                   d.epot, d.ox, d.oy, d.oz, d.cx, d.cy, d.cz, d.rvx, d.rvy, d.rvz,
                   d.species, d.flags, d.rowflag, d.bkey, d.pid, d.ref_order, d.ref_tmp,
-                  d.ref_pos, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ovq[0],
+                  d.ref_pos, d.ford, d.nn, d.nbr, d.cell_cnt, d.bucket, d.bx, d.by, d.bz, d.ovq[0],
                   d.ovq[1], d.ov_near, d.nearl, d.part_d, d.part_i, d.blk2rep, d.rp, d.cnt, d.wl[0],
                   d.wl[1], d.wl_cnt, d.ovw[0], d.ovw[1], d.ov_last, d.ovx_n, d.ovx_l, d.ovx_m, d.ovx_b, d.pf4, d.bf4, d.gc_order,
                   d.b2slot, d.seq, d.chx, d.chy, d.chz, d.chox, d.choy, d.choz,
@@ -1222,6 +1237,7 @@ int dml_set_state(dml_ctx *c, int32_t rep, int32_t n, const double *pos, const d
   p.free_lo = 0;
   p.bfree_lo = 0;
   p.ovn_stamp = 0;  // no entries-within-rcut lists for the new atoms yet
+  p.fo_n = 0;
   p.nslots = n;
   p.nref = nref;
   p.listed = 0;
@@ -1290,6 +1306,7 @@ int dml_set_order(dml_ctx *c, int32_t rep, int32_t nref, const int32_t *ref_orde
     p.bfree_lo = 0;
   }
   p.ovn_stamp = 0;  // another set of ref atoms: no lists for the new ones
+  p.fo_n = 0;
   return upload_params(c);
 }
 
@@ -1900,7 +1917,7 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
                         (int64_t)c->any_chunks << 31 |
                         (int64_t)c->rounds << 6 | (int64_t)c->lpa << 12 |
                         (int64_t)c->lpa_ov << 19 | (int64_t)c->ov_lanes_set << 52 |
-                        (int64_t)(live_slots(c) < 300000) << 53 | (int64_t)c->lb_mode << 26 |
+                        (int64_t)(live_slots(c) < 300000) << 53 | (int64_t)by_cell(c) << 54 | (int64_t)c->lb_mode << 26 |
                         (int64_t)c->any_lb[0] << 32 | (int64_t)c->any_lb[1] << 33 |
                         (int64_t)c->any_lb[2] << 34 | (int64_t)c->any_lb[3] << 35;
   // a captured step holds the device state by value: any reallocation or

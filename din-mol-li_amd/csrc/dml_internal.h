@@ -21,6 +21,8 @@
 #define OVT_BLOCK 512 // threads of the overlap tail
 #define OVX_MAX 16  // row entries listed per atom for the reference-order overlap pass
 #define OVX_BLOCK 1024
+#define FO_BLOCK 512  // threads of k_force_order
+#define FO_LEAST 200000  // slots from which the force kernel takes the atoms cell by cell
 #define NEAR_MAX 4  // row positions within rcut listed per atom by the row build
 #define DML_GCMC_BLOCK 256  // one workgroup per GCMC replica
 
@@ -125,6 +127,7 @@ struct RepParams {
   int32_t gb_nins, gb_ndel, gb_nalist;
   uint32_t gb_stamp;       // gcmc_calls + 1 of this call (stamped per-cell / per-slot marks)
   double gb_act;
+  int32_t fo_n;  // entries of the force kernel's list in cell order (0: ref order)
 };
 
 // cgroup_tessellate (Cells.F90:180-265) on the replica's box: the fast path
@@ -294,6 +297,7 @@ struct DevState {
   int32_t *bkey;          // hs%b slot: cell-chain order key
   uint32_t *pid;          // stable particle id (Philox counter)
   int32_t *ref_order, *ref_tmp, *ref_pos;
+  int32_t *ford;          // ref atoms of the last rebuild cell by cell, then those inserted since
   int32_t *nn, *nbr;
   int32_t maxnn;
   // cells

@@ -8,6 +8,7 @@ __global__ void k_load_state(DevState s, int poff, int n, int nref, int ngc, int
                              const unsigned char *in);
 __global__ void k_pack_state(DevState s, int poff, int n, int want, unsigned char *out);
 __global__ void k_force_rebuild(DevState s);
+__global__ void k_force_order(DevState s);
 __global__ void k_zero_cells(DevState s, int gcs);
 __global__ void k_cell_key(DevState s, int gcs);
 __global__ void k_cell_sort(DevState s, int gcs);

@@ -203,6 +203,7 @@ __global__ void k_zero_cells(DevState s, int gcs) {
     const int c = s.cm_cell[g];
     if (P.halted || !want_cells(P, gcs) || c >= ncell_total(P)) continue;
     s.cell_cnt[P.coff + c] = 0;
+    if (c == 0 && P.rebuild) s.rp[s.cm_rep[g]].fo_n = 0;
   }
 }
 
@@ -1499,11 +1500,76 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
 
 
 // ------------------------------------------------------------------------
+// The ref atoms of the replicas that rebuild, cell by cell (s.ford, P.fo_n of
+// them), for the force kernel of a large system.  A workgroup lists 64 cells
+// of the flat cell list: the counts of k_cell_sort_w, one atomic for its
+// place in the replica's list, 8 waves copying cells.  Bound by the latency
+// of a wave's 8 cells.
+// ------------------------------------------------------------------------
+__global__ void __launch_bounds__(FO_BLOCK) k_force_order(DevState s) {
+  __shared__ int at0;
+  const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
+  for (int64_t g0 = (int64_t)blockIdx.x * WAVE; g0 < s.n_cm; g0 += (int64_t)gridDim.x * WAVE) {
+    int lr = -1, lc = 0, ln = 0;
+    if (g0 + lane < s.n_cm) {
+      ln = s.cm_nref[g0 + lane];
+      if (ln > 0) {
+        lr = s.cm_rep[g0 + lane];
+        lc = s.cm_cell[g0 + lane];
+        if (s.rp[lr].nslots < FO_LEAST || s.rp[lr].integrator != DML_ERMAK) ln = 0;
+      }
+    }
+    unsigned long long todo = __ballot(ln > 0);
+    // the cells of one replica at a time (a block of cells mostly has one)
+    while (todo) {
+      const int r = __builtin_amdgcn_readlane(lr, __builtin_ctzll(todo));
+      const unsigned long long mine = __ballot(ln > 0 && lr == r);
+      todo &= ~mine;
+      const int incl = wave_scan_incl(lr == r ? ln : 0);
+      if (threadIdx.x == 0) at0 = atomicAdd(&s.rp[r].fo_n, __builtin_amdgcn_readlane(incl, WAVE - 1));
+      __syncthreads();
+      const RepParams &P = s.rp[r];
+      int32_t *out = s.ford + P.poff + at0;
+      int k = 0;
+      for (unsigned long long m = mine; m; m &= m - 1, k++) {
+        if (k % (FO_BLOCK / WAVE) != w) continue;
+        const int q = __builtin_ctzll(m);
+        const int c = __builtin_amdgcn_readlane(lc, q);
+        const int cnt = __builtin_amdgcn_readlane(ln, q);
+        int at = __builtin_amdgcn_readlane(incl, q) - cnt;
+        const int end = at + cnt;
+        const int64_t base = P.boff + (int64_t)c * P.bcap;
+        for (int e0 = 0; at < end && e0 < P.bcap; e0 += WAVE) {
+          const int e = e0 + lane;
+          const bool in = e < P.bcap;
+          const int v = in ? s.bucket[base + e] : 0;
+          const float4 f = in ? s.bf4[base + e] : make_float4(0.f, 0.f, 0.f, 0.f);
+          const unsigned long long b = __ballot(in && bucket_ref(f));
+          const int p = at + __popcll(b & ((1ull << lane) - 1ull));
+          if (in && bucket_ref(f) && p < end) out[p] = v;
+          at += __popcll(b);
+        }
+      }
+      __syncthreads();  // at0 is rewritten
+    }
+  }
+}
+
+// ------------------------------------------------------------------------
 // fuerza (dana.F90:1055-1139) as a gather: the full list plus reaction of
 // the reference counts every ref-ref pair twice, so entry j of row i
 // weighs 2 when j is a ref atom (its row holds i) and 1 otherwise.  Rows
 // built from a ghost-layer cell are found by nobody; their reactions are
 // added by k_ghost_scatter.  Optionally fused with ermak_b (1031-1052).
+//
+// What bounds it: the gathers of the row entries' positions (16 bytes each,
+// about 100 entries an atom of a dense system, of which one or two are within
+// r0).  A lane has FU of them in flight before it looks at any.  In ref order a
+// large system's gathers miss the 4 MB L2 of an XCD (its mirror is 16 bytes a
+// slot), so there the atoms are taken cell by cell (s.ford): a 2M-atom system
+// 2,490 -> 890 us, of which FU accounts for 170, the order for the rest; 600,000
+// atoms 446 -> 249.  The atom's own fields are then scattered, so ermak_b, 9
+// arrays of them, runs on its own in ref order (fused 1,440, alone 870 + 80).
 // ------------------------------------------------------------------------
 __device__ inline double pow6d(double x) {
   double x2 = x * x, x4 = x2 * x2;
@@ -1548,6 +1614,7 @@ __device__ inline double lpa_xor_d(double v, int off) {
   return __longlong_as_double((int64_t)(uint32_t)lo | ((int64_t)hi << 32));
 }
 
+#define FU 4  // row entries a lane has in flight
 template <int LPA, int FUSEB>
 __global__ void __launch_bounds__(DML_BLOCK) k_force(DevState s, int only_ermak) {
   int gid = blockIdx.x * DML_BLOCK + threadIdx.x;
@@ -1558,22 +1625,23 @@ __global__ void __launch_bounds__(DML_BLOCK) k_force(DevState s, int only_ermak)
   if (only_ermak && P.integrator != DML_ERMAK) return;
   const int FP32 = P.precision == DML_FP32_FORCE;
   int local = t - P.poff;
-  int active = local < P.nref;
-  int i = active ? s.ref_order[t] : 0;
+  const int by_cell = P.fo_n > 0;
+  int active = local < (by_cell ? P.fo_n : P.nref);
+  int i = active ? (by_cell ? s.ford[t] : s.ref_order[t]) : 0;
+  // atoms that left the ref group since the list was made
+  if (by_cell && active && !(s.flags[i] & DML_FL_REF)) active = 0;
   double fx = 0.0, fy = 0.0, fz = 0.0, ea = 0.0;
   // entries within rcut (FP32 with margin), the ones overlap_moveback looks
   // at: their number on this lane and the row position of the last one
   int ncnt = 0, ne = 0;
   if (local == 0 && sub == 0) s.rp[r].ovn_stamp = P.step + 1;
   if (active) {
-    int k = s.species[i];
     const float rcf = (float)P.rcut2 + P.pf_margin;
-    double xi = s.px[i], yi = s.py[i], zi = s.pz[i];
     double hbx = P.box[0] * .5, hby = P.box[1] * .5;
-    int ghost = s.rowflag[i] & 1;
     int nn = s.nn[i];
     const int32_t *row = s.nbr + (int64_t)i * s.maxnn;
     const float4 fi = s.pf4[i];
+    const int k = __float_as_int(fi.w);  // its species
     const float bxf = (float)P.box[0], byf = (float)P.box[1];
     const float ibx = (float)P.one_box[0], iby = (float)P.one_box[1];
     // this atom's FP32 prefilter bound r0^2 + margin against each of the
@@ -1581,23 +1649,37 @@ __global__ void __launch_bounds__(DML_BLOCK) k_force(DevState s, int only_ermak)
     const float th1 = (float)P.r0[(k - 1) * 3 + 0] * (float)P.r0[(k - 1) * 3 + 0] + P.pf_margin;
     const float th2 = (float)P.r0[(k - 1) * 3 + 1] * (float)P.r0[(k - 1) * 3 + 1] + P.pf_margin;
     const float th3 = (float)P.r0[(k - 1) * 3 + 2] * (float)P.r0[(k - 1) * 3 + 2] + P.pf_margin;
-    for (int e = sub; e < nn; e += LPA) {
-      int j = row[e];
-      const float4 fj4 = s.pf4[j];
-      {  // surely beyond the pair's r0: no force, no energy
-        const int sj = __float_as_int(fj4.w);
+    for (int e0 = sub; e0 < nn; e0 += FU * LPA) {
+      int ju[FU];
+      float4 fu[FU];
+#pragma unroll
+      for (int u = 0; u < FU; u++) ju[u] = e0 + u * LPA < nn ? row[e0 + u * LPA] : i;
+#pragma unroll
+      for (int u = 0; u < FU; u++) fu[u] = s.pf4[ju[u]];
+      // the entries within their pair's r0 (FP32 with margin), a bit each
+      uint32_t hit = 0;
+#pragma unroll
+      for (int u = 0; u < FU; u++) {
+        const int sj = __float_as_int(fu[u].w);
         const float th = sj == 1 ? th1 : (sj == 2 ? th2 : th3);
-        const float d2f = d2_f32(P, fi, fj4, bxf, byf, ibx, iby);
-        if (d2f <= rcf) {
+        const float d2f = d2_f32(P, fi, fu[u], bxf, byf, ibx, iby);
+        const bool in = e0 + u * LPA < nn;
+        if (in && d2f <= rcf) {
           ncnt++;
-          ne = e;
+          ne = e0 + u * LPA;
         }
-        if (d2f > th) continue;
+        // (beyond it surely no force, no energy; a NaN is looked at)
+        if (in && !(d2f > th)) hit |= 1u << u;
       }
+      for (; hit; hit &= hit - 1) {
+      const int u0 = __builtin_ctz(hit);
+      int j = ju[0];
+#pragma unroll
+      for (int u = 1; u < FU; u++) j = u0 == u ? ju[u] : j;
       uint8_t fj = s.flags[j];
       if (fj & DML_FL_LIMBO) continue;
       int m = s.species[j];
-      double vx = xi - s.px[j], vy = yi - s.py[j], vz = zi - s.pz[j];
+      double vx = s.px[i] - s.px[j], vy = s.py[i] - s.py[j], vz = s.pz[i] - s.pz[j];
       if (vx > hbx) vx = vx - P.box[0];
       else if (vx < -hbx) vx = vx + P.box[0];
       if (vy > hby) vy = vy - P.box[1];
@@ -1608,6 +1690,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_force(DevState s, int only_ermak)
       double r0 = P.r0[km];
       if (dr2 > r0 * r0) continue;
       double eps = P.eps[km];
+      const int ghost = s.rowflag[i] & 1;
       double w = ((fj & DML_FL_REF) && !ghost) ? 2.0 : 1.0;
       if (FP32) {
         // FP32 pair arithmetic without cancellation: r0^2 - r^2 comes from
@@ -1637,6 +1720,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_force(DevState s, int only_ermak)
         double u = eps * b * (b - 2);
         u = u + eps;
         ea += w * (u * .5);
+      }
       }
     }
   }
@@ -3390,6 +3474,9 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
   int idel = 0;  // in-volume entries deleted so far (tombstones in invl)
   int nslots = P.nslots, nat = P.nat, nlimbo = P.nlimbo, b_amax = P.b_amax, b_nat = P.b_nat;
   int rlen = P.nref;  // ref list length with tombstones
+  // an inserted atom joins the force kernel's list (no slot is in it twice:
+  // with lists a slot comes back only after a rebuild, which lists anew)
+  int fo_n = listed ? P.fo_n : 0;
   int head = 0, tail = glen - 1;  // first / last live gcmc entry
   uint32_t pid_next = P.pid_next;
   int seq_next = P.seq_next;
@@ -3566,6 +3653,7 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
         s.nn[i] = 0;
         rord[rlen] = i;
         s.ref_pos[i] = rlen;
+        if (fo_n > 0) s.ford[poff + fo_n] = i;
         put_pf4(s, i, rx, ry, rz, s.species[tmpl]);
       }
       {
@@ -3596,6 +3684,7 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
       nat++;
       b_nat++;
       rlen++;
+      if (fo_n > 0) fo_n++;
       if (listed) {
         const int ghost = P.use_cells && (ci2 == 0 || ci2 == P.ncells[2] + 1 || ci0 == 0 ||
                                           ci0 == P.ncells[0] + 1 || ci1 == 0 ||
@@ -3819,6 +3908,7 @@ __global__ void __launch_bounds__(GC_BLOCK) k_gcmc_run(DevState s, int rep_only,
     Pw->gc_pending = 2;
     if (n_ins || n_del) Pw->ovn_stamp = 0;  // atoms added or removed
     Pw->free_lo = hs_scan;
+    Pw->fo_n = fo_n;
     Pw->bfree_lo = nfreed_b ? min(b_scan, sh_freed_b[0]) : b_scan;
     Pw->nslots = nslots;
     Pw->nat = nat;
@@ -5053,6 +5143,7 @@ __global__ void __launch_bounds__(WAVE) k_gb_commit(DevState s, int r, const dou
     Pw->b_nat = b_nat;
     Pw->pid_next = P.pid_next + (uint32_t)nins;
     Pw->seq_next = P.seq_next + nins;
+    if (P.fo_n > 0) Pw->fo_n = P.fo_n + nins;  // (their entries: k_gb_fields)
     Pw->gc_len = glen + nins;
     Pw->ref_len = P.gb_rlen + nins;
     Pw->gc_pending = 2;
@@ -5084,6 +5175,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_gb_fields(DevState s, int r) {
   s.pid[i] = P.pid_next - (uint32_t)P.gb_nins + (uint32_t)k;
   s.seq[i] = P.seq_next - P.gb_nins + k;
   s.rowflag[i] = 0;
+  if (P.fo_n > 0) s.ford[P.poff + P.fo_n - P.gb_nins + k] = i;
   put_pf4(s, i, rx, ry, rz, s.species[i]);
   // the row built at insertion (kept even when the atom leaves later in the
   // call) marks a ghost-layer cell
@@ -5471,6 +5563,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_chunk_run(DevState s) {
     Pw->seq_next = P.seq_next + nch;
     Pw->listed = 0;  // hs%listed = .false.: the next test_update rebuilds
     Pw->chunk_fired = 1;
+    Pw->fo_n = 0;
     Pw->ovn_stamp = 0;  // atoms added
   }
 }
