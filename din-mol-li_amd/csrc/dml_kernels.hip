@@ -4920,17 +4920,30 @@ __global__ void __launch_bounds__(DML_BLOCK) k_gb_brank(DevState s, int r) {
 // the accepted moves in trial order, one wave: hs%b indices (the lowest
 // free one, indices freed earlier in the call included, Groups.F90:1094-
 // 1100), the template (first live gcmc atom) and list tail whose velocity
-// the insertion sets (dana.F90:620-668), and the ordered stores: flags,
-// hs%b maps, ref and gcmc list entries, limbo (Groups.F90:433-467).  The
-// universe of free hs%b indices is a bitmap in LDS searched from a lower
-// bound of the lowest free rank, their values in LDS too.
+// the insertion sets (dana.F90:620-668), and the stores: flags, hs%b maps,
+// ref and gcmc list entries, limbo (Groups.F90:433-467).
+//
+// 64 trials at a time, a lane each.  Only the ranks in the universe of free
+// hs%b indices go one move after the other, in scalar registers: the lowest
+// free ranks of the batch's start (a list, from a bitmap in LDS) against the
+// least of those freed since.  The rest is per lane: an atom inserted in the
+// call and deleted later gets its final fields at once, an insertion's velocity
+// is the next one's normals (its own template's for the last), and who holds
+// an index at the end is kept in LDS and written once.  A deletion that takes
+// the template or the tail away ends its batch early.
+//
+// What bounds it: the loads of a batch (two round trips) and some 40 cycles a
+// move for the ranks.  Move by move, lane 0 storing 14 fields each, a call of
+// 8,192 trials took 2,480 us; now 1,045.
 __global__ void __launch_bounds__(WAVE) k_gb_commit(DevState s, int r, const double *g) {
   // universe values (the free indices of the start and those freed by the
-  // call's deletions: at most two per trial counting the appended ones)
-  __shared__ int32_t U[2 * DML_GCMC_BATCH_MAX];
-  __shared__ uint32_t ubl[GB_UW * WAVE];
-  __shared__ int32_t ibr[DML_GCMC_BATCH_MAX];  // hs%b rank of each insertion
-  __shared__ int32_t ibv[DML_GCMC_BATCH_MAX];  // and the index itself
+  // call's deletions: at most two per trial counting the appended ones) and
+  // the slot that holds each
+  __shared__ int32_t U[2 * DML_GCMC_BATCH_MAX], own[2 * DML_GCMC_BATCH_MAX];
+  __shared__ uint32_t ubl[GB_UW * WAVE];             // free ranks
+  __shared__ uint16_t ibr[DML_GCMC_BATCH_MAX];       // hs%b rank of each insertion
+  __shared__ int32_t lst[WAVE];
+  static_assert(2 * DML_GCMC_BATCH_MAX <= 65536, "ranks are kept in 16 bits");
   RepParams *Pw = s.rp + r;
   if (!gb_on(*Pw)) return;
   const RepParams &P = *Pw;
@@ -4938,24 +4951,28 @@ __global__ void __launch_bounds__(WAVE) k_gb_commit(DevState s, int r, const dou
   const GbView V = gb_view(P);
   const int off = P.gb_off, T = P.gb_t, poff = P.poff, ilen = P.gb_ilen;
   const int nins = P.gb_nins, ndel = P.gb_ndel, rlen = P.gb_rlen;
-  const int nUF = min(P.gb_nFB, T);
+  const int nUF = min(P.gb_nFB, T), b_amax0 = P.b_amax;
   const double mass[3] = {P.mass[0], P.mass[1], P.mass[2]};
   int nU = 0;
   for (int d = lane; d < ndel; d += WAVE) nU += s.gd_bso[off + d] >= 0;
   for (int o2 = WAVE / 2; o2 > 0; o2 >>= 1) nU += __shfl_xor(nU, o2);
-  nU += nUF;
+  nU = __builtin_amdgcn_readfirstlane(nU) + nUF;
   for (int q = lane; q < GB_UW * WAVE; q += WAVE) ubl[q] = 0u;
+  for (int q = lane; q < nU; q += WAVE) {
+    U[q] = s.gb_U[3 * off + q];
+    own[q] = -1;
+  }
   __syncthreads();
-  for (int q = lane; q < nU; q += WAVE) U[q] = s.gb_U[3 * off + q];
   for (int q = lane; q < nUF; q += WAVE) {
     const int rk = s.gb_frank[off + q];
     atomicOr(&ubl[rk >> 5], 1u << (rk & 31));
   }
+  for (int d = lane; d < ndel; d += WAVE)
+    if (s.gd_bso[off + d] >= 0) own[s.gd_brank[off + d]] = s.gd_slot[off + d];
   __syncthreads();
-  // the free ranks stay in the LDS bitmap; every rank below ulo is taken
-  // (an insertion takes the lowest free rank, a deletion can only lower it)
+  // every rank below ulo is taken (an insertion takes the lowest free rank,
+  // a deletion can only lower it)
   int ulo = 0;
-  int b_amax = P.b_amax, b_nat = P.b_nat;
   int nappend = 0;          // hs%b indices appended at b_amax (ranks nU + ...)
   int bmin = P.bfree_lo;    // lower bound of the free hs%b indices after the call
   // gcmc list: the staged list (glen entries) then the call's insertions
@@ -4978,158 +4995,188 @@ __global__ void __launch_bounds__(WAVE) k_gb_commit(DevState s, int r, const dou
     if (e < glen) return gb_del_time_v(s, V, gc[e]) <= t;
     return s.gi_del[off + (e - glen)] <= t;
   };
-  // three streams read 64 entries at a time, one per lane, into registers
-  // when the walk reaches the chunk, and taken lane by lane with readlane:
-  // the trials (decision, kind, normals), the deletions in order (atom,
-  // hs%b index and rank, ref position, flags) and the insertions' slots.
-  // Each chunk load is waited for where it is made (every memory operation
-  // of the wave before it included, stores too): a load still counted as in
-  // flight where the paths merge would make every later iteration wait.
-  int c_res = -1, c_kind = 0, c_is = 0, c_d[5] = {0, 0, 0, 0, 0};
-  double c_g[3] = {0.0, 0.0, 0.0};
+  const unsigned long long below = (1ull << lane) - 1ull;
   int ki = 0, kd = 0;
   int ta = gc[glen - 1];  // the tail atom
-  for (int t = 0; t < T; t++) {
-    // one wave in program order: the barrier only keeps the compiler (and a
-    // lane-by-lane CPU model of the wave) from moving LDS accesses across
-    // iterations
-    __builtin_amdgcn_wave_barrier();
-    const int tl = t & (WAVE - 1);
-    if (tl == 0) {
-      const int q = t + lane;
-      if (q < T) {
-        c_res = s.gb_res[off + q];
-        c_kind = s.gb_kind[off + q];
-        c_g[0] = s.gb_g[3 * (off + q)];
-        c_g[1] = s.gb_g[3 * (off + q) + 1];
-        c_g[2] = s.gb_g[3 * (off + q) + 2];
-      }
-      __builtin_amdgcn_s_waitcnt(0);
-      __builtin_amdgcn_wave_barrier();
+  // (decisions and kinds are read a batch ahead)
+  int n_res = lane < T ? s.gb_res[off + lane] : -1, n_kind = lane < T ? s.gb_kind[off + lane] : 2;
+  for (int t0 = 0; t0 < T; t0 += WAVE) {
+    const int t = t0 + lane, res = n_res, kind = n_kind;
+    const bool ins = res >= 0 && kind == 0, del = res >= 0 && kind != 0;
+    const unsigned long long mi = __ballot(ins), md = __ballot(del);
+    const int k = ki + __popcll(mi & below), d = kd + __popcll(md & below);
+    // the atom inserted or deleted, the rank it frees (an atom inserted in
+    // this batch: that of the lane src), the trial that deletes an insertion
+    int i = -1, rank = -1, rpos = -1, ofl = 0, bso = -1, src = lane, gone = 0x7fffffff;
+    double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+    if (t + WAVE < T) {
+      n_res = s.gb_res[off + t + WAVE];
+      n_kind = s.gb_kind[off + t + WAVE];
+    } else {
+      n_res = -1;
     }
-    const int res = __builtin_amdgcn_readlane(c_res, tl);
-    const int kind = __builtin_amdgcn_readlane(c_kind, tl);
-    if (res < 0) continue;
-    if (kind == 0) {
-      const int k = ki++;
-      if ((k & (WAVE - 1)) == 0) {
-        if (k + lane < nins) c_is = gb_ins_slot_v(s, V, k + lane);
-        __builtin_amdgcn_s_waitcnt(0);
+    if (ins) {
+      i = gb_ins_slot_v(s, V, k);
+      gone = s.gi_del[off + k];
+      g0 = s.gb_g[3 * (off + t)];
+      g1 = s.gb_g[3 * (off + t) + 1];
+      g2 = s.gb_g[3 * (off + t) + 2];
+    } else if (del) {
+      i = s.gd_slot[off + d];
+      if (res < ilen) {
+        bso = s.gd_bso[off + d];
+        rank = s.gd_brank[off + d];
+        rpos = s.gd_rpos[off + d];
+        ofl = s.gd_oflags[off + d];
+      } else if (res - ilen < ki) {
+        rank = ibr[res - ilen];
+      } else {
+        unsigned long long m = mi;
+        for (int q = res - ilen - ki; q > 0; q--) m &= m - 1;
+        src = __builtin_ctzll(m);
+      }
+    }
+    // every memory operation of the batches before is done: an atom's
+    // velocity may be written by two of them
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+    unsigned long long left = mi | md;
+    while (left) {
+      // the tail as this lane's trial finds it
+      const unsigned long long im = mi & left, ip = im & below;
+      const int tprev = __shfl(i, ip ? 63 - __builtin_clzll(ip) : 0);
+      const unsigned long long stop =
+          __ballot(del && (left >> lane & 1) && (i == tmpl || i == (ip ? tprev : ta)));
+      const int e = stop ? __builtin_ctzll(stop) : WAVE - 1;
+      const unsigned long long seg = left & (e == WAVE - 1 ? ~0ull : (2ull << e) - 1ull);
+      const unsigned long long si = mi & seg;
+      const int want = __popcll(si);
+      // the lowest free ranks, as many as insertions
+      int have = 0;
+      for (int w0 = ulo >> 5; have < want && w0 < GB_UW * WAVE; w0 += WAVE) {
+        const int w = w0 + lane;
+        uint32_t word = w < GB_UW * WAVE ? ubl[w] : 0u;
+        const int c = __popc(word), incl = wave_scan_incl(c);
+        for (int at = have + incl - c; word && at < want; at++, word &= word - 1)
+          lst[at] = w * 32 + __builtin_ctz(word);
+        have += __builtin_amdgcn_readlane(incl, WAVE - 1);
+      }
+      have = min(have, want);
+      __builtin_amdgcn_wave_barrier();
+      const int low = lane < have ? lst[lane] : 0x7fffffff;
+      __builtin_amdgcn_wave_barrier();
+      // the ranks, in trial order
+      int p = 0, fm = 0x7fffffff;
+      unsigned long long freed = 0;
+      for (unsigned long long m = seg; m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        int rk;
+        if (si >> l & 1) {
+          const int sp = p < have ? __builtin_amdgcn_readlane(low, p) : 0x7fffffff;
+          if (fm < sp) {
+            rk = fm;
+            freed &= ~__ballot((freed >> lane & 1) && rank == fm);
+            int v = (freed >> lane & 1) ? rank : 0x7fffffff;
+            if (freed)
+              for (int o2 = WAVE / 2; o2 > 0; o2 >>= 1) v = min(v, __shfl_xor(v, o2));
+            fm = __builtin_amdgcn_readfirstlane(v);
+          } else if (p < have) {
+            rk = sp;
+            p++;
+          } else {
+            rk = nU + nappend++;  // none is free: a new one at b_amax
+          }
+        } else {
+          rk = __builtin_amdgcn_readlane(rank, __builtin_amdgcn_readlane(src, l));
+          freed |= 1ull << l;
+          fm = min(fm, rk);
+        }
+        if (lane == l) {
+          rank = rk;
+          own[rk] = si >> l & 1 ? i : -1;
+        }
+        // (the LDS stores of two lanes to one rank stay in trial order)
         __builtin_amdgcn_wave_barrier();
       }
-      const int i = __builtin_amdgcn_readlane(c_is, k & (WAVE - 1));
-      // hs%b index: the lowest free one, or a new one at b_amax
-      int bs, rank;
-      if (b_amax >= b_nat + 1) {
-        int w = ulo >> 5;
-        uint32_t word = (uint32_t)rfl_i((int)ubl[w]);
-        uint32_t live = word & (0xffffffffu << (ulo & 31));
-        while (live == 0u && w + 1 < GB_UW * WAVE) {
-          w++;
-          word = (uint32_t)rfl_i((int)ubl[w]);
-          live = word;
+      if (lane < p) atomicAnd(&ubl[low >> 5], ~(1u << (low & 31)));
+      __builtin_amdgcn_wave_barrier();
+      if (freed >> lane & 1) atomicOr(&ubl[rank >> 5], 1u << (rank & 31));
+      __builtin_amdgcn_wave_barrier();
+      if (p > 0) ulo = __builtin_amdgcn_readlane(low, p - 1) + 1;
+      ulo = min(ulo, fm);
+      // the stores
+      const bool mine = seg >> lane & 1;
+      const int bs = mine ? (rank < nU ? U[rank] : b_amax0 + rank - nU) : 0;
+      const unsigned long long nx = si & ~below & ~(1ull << lane);
+      const int nl = nx ? __builtin_ctzll(nx) : 0;
+      const double n0 = __shfl(g0, nl), n1 = __shfl(g1, nl), n2 = __shfl(g2, nl);
+      if (mine && ins) {
+        // the velocity lands on the list's last live atom, the new atom
+        // copies the template (atom_asign, Groups.F90:484-502)
+        if (!(si & below)) {
+          s.vx[ta] = beta * g0;
+          s.vy[ta] = beta * g1;
+          s.vz[ta] = beta * g2;
         }
-        if (live == 0u) {  // cannot happen: b_amax - b_nat counts the set bits
-          if (lane == 0) rep_fail(s, r, ERR_UNSUP);
-          return;
-        }
-        const int bit = __builtin_ctz(live);
-        rank = w * 32 + bit;
-        if (lane == 0) ubl[w] = word & ~(1u << bit);
-        ulo = rank + 1;
-        bs = U[rank];
-      } else {
-        bs = b_amax++;
-        rank = nU + nappend++;
-        if (lane == 0) U[rank] = bs;
-      }
-      b_nat++;
-      // the velocity lands on the list's last live atom, the new atom copies
-      // the template (atom_asign, Groups.F90:484-502)
-      const double g0 = rdlane_d(c_g[0], tl), g1 = rdlane_d(c_g[1], tl), g2 = rdlane_d(c_g[2], tl);
-      if (lane == 0) {
-        s.vx[ta] = beta * g0;
-        s.vy[ta] = beta * g1;
-        s.vz[ta] = beta * g2;
-        s.vx[i] = tv[0];
-        s.vy[i] = tv[1];
-        s.vz[i] = tv[2];
+        s.vx[i] = nx ? beta * n0 : tv[0];
+        s.vy[i] = nx ? beta * n1 : tv[1];
+        s.vz[i] = nx ? beta * n2 : tv[2];
+        const bool dead = gone != 0x7fffffff;
         s.species[i] = tsp;
-        s.flags[i] = DML_FL_ALIVE | DML_FL_REF | DML_FL_GCMC;
+        s.flags[i] = dead ? DML_FL_LIMBO : DML_FL_ALIVE | DML_FL_REF | DML_FL_GCMC;
+        if (dead) s.nn[i] = 0;
         s.bkey[i] = bs;
-        s.b2slot[poff + bs] = i;
-        s.ref_order[poff + rlen + k] = i;
-        s.ref_pos[i] = rlen + k;
+        s.ref_order[poff + rlen + k] = dead ? -1 : i;
+        s.ref_pos[i] = dead ? -1 : rlen + k;
         s.wl[1][poff + glen + k] = i;
         s.gi_tmpl[off + k] = tmpl;
         s.gb_slot[off + t] = i;
-        ibr[k] = rank;
-        ibv[k] = bs;
-      }
-      e_tail = glen + k;
-      ta = i;
-    } else {
-      const int d = kd++;
-      if ((d & (WAVE - 1)) == 0) {
-        const int q = d + lane;
-        if (q < ndel) {
-          c_d[0] = s.gd_slot[off + q];
-          c_d[1] = s.gd_bso[off + q];
-          c_d[2] = s.gd_brank[off + q];
-          c_d[3] = s.gd_rpos[off + q];
-          c_d[4] = s.gd_oflags[off + q];
+        ibr[k] = (uint16_t)rank;
+      } else if (mine) {
+        bmin = min(bmin, res < ilen ? bso : bs);
+        if (res < ilen) {
+          s.flags[i] = (uint8_t)(DML_FL_LIMBO | (ofl & DML_FL_SKIP));
+          s.nn[i] = 0;
+          s.ref_order[poff + rpos] = -1;
+          s.ref_pos[i] = -1;
         }
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (si) {
+        const int l = 63 - __builtin_clzll(si);
+        ta = __builtin_amdgcn_readlane(i, l);
+        e_tail = glen + __builtin_amdgcn_readlane(k, l);
+      }
+      left &= ~seg;
+      if (stop) {
+        // the template and the tail step over dead entries (dana.F90:620,
+        // the gcmc list after gcmc%detach)
         __builtin_amdgcn_s_waitcnt(0);
         __builtin_amdgcn_wave_barrier();
-      }
-      const int dl = d & (WAVE - 1);
-      const int o = __builtin_amdgcn_readlane(c_d[0], dl);
-
-      int bso, rank, rpos, ofl;
-      if (res >= ilen) {
-        const int k = res - ilen;
-        bso = ibv[k];
-        rank = ibr[k];
-        rpos = rlen + k;
-        ofl = 0;
-      } else {
-        bso = __builtin_amdgcn_readlane(c_d[1], dl);
-        rank = __builtin_amdgcn_readlane(c_d[2], dl);
-        rpos = __builtin_amdgcn_readlane(c_d[3], dl);
-        ofl = __builtin_amdgcn_readlane(c_d[4], dl);
-      }
-      // the freed hs%b index is free again for the later insertions
-      if (lane == 0) atomicOr(&ubl[rank >> 5], 1u << (rank & 31));
-      ulo = min(ulo, rank);
-      b_nat--;
-      bmin = min(bmin, bso);
-      if (lane == 0) {
-        s.flags[o] = (uint8_t)(DML_FL_LIMBO | (ofl & DML_FL_SKIP));
-        s.nn[o] = 0;
-        s.ref_order[poff + rpos] = -1;
-        s.ref_pos[o] = -1;
-        s.b2slot[poff + bso] = -1;
-      }
-      // the template and the tail step over dead entries (dana.F90:620,
-      // the gcmc list after gcmc%detach)
-      // (values loaded here are taken into scalar registers at once: a load
-      // still in flight at the merge below would make every later
-      // iteration wait for it)
-      if (o == tmpl) {
-        while (entry_dead(hd, t)) hd++;
-        tmpl = __builtin_amdgcn_readfirstlane(entry_atom(hd));
-        tsp = (int8_t)__builtin_amdgcn_readfirstlane((int)s.species[tmpl]);
-        beta = sqrt(kB_ui * 300.0 / mass[tsp - 1]);
-        tv[0] = rdlane_d(s.vx[tmpl], 0);
-        tv[1] = rdlane_d(s.vy[tmpl], 0);
-        tv[2] = rdlane_d(s.vz[tmpl], 0);
-      }
-      if (o == ta) {
-        while (e_tail > hd && entry_dead(e_tail, t)) e_tail--;
-        ta = __builtin_amdgcn_readfirstlane(entry_atom(e_tail));
+        const int o = __builtin_amdgcn_readlane(i, e), te = t0 + e;
+        if (o == tmpl) {
+          while (entry_dead(hd, te)) hd++;
+          tmpl = __builtin_amdgcn_readfirstlane(entry_atom(hd));
+          tsp = (int8_t)__builtin_amdgcn_readfirstlane((int)s.species[tmpl]);
+          beta = sqrt(kB_ui * 300.0 / mass[tsp - 1]);
+          tv[0] = rdlane_d(s.vx[tmpl], 0);
+          tv[1] = rdlane_d(s.vy[tmpl], 0);
+          tv[2] = rdlane_d(s.vz[tmpl], 0);
+        }
+        if (o == ta) {
+          while (e_tail > hd && entry_dead(e_tail, te)) e_tail--;
+          ta = __builtin_amdgcn_readfirstlane(entry_atom(e_tail));
+        }
       }
     }
+    ki += __popcll(mi);
+    kd += __popcll(md);
   }
+  __builtin_amdgcn_wave_barrier();
+  for (int q = lane; q < nU + nappend; q += WAVE)
+    s.b2slot[poff + (q < nU ? U[q] : b_amax0 + q - nU)] = own[q];
+  for (int o2 = WAVE / 2; o2 > 0; o2 >>= 1) bmin = min(bmin, __shfl_xor(bmin, o2));
+  const int b_amax = b_amax0 + nappend, b_nat = P.b_nat + nins - ndel;
   if (lane == 0) {
     const int nF = P.gb_nF;
     const int nsl = P.gb_nslots + max(0, nins - nF);
