@@ -525,23 +525,60 @@ void assign_list_kernels(dml_ctx *c) {
 
 // gcs = 1: also re-sort the cells of the GCMC replicas (their trials read
 // them before the next test_update)
-void enq_cells_lists(dml_ctx *c, int gcs) {
-  c->fresh = 0;
-  dim3 gc(clamp_grid((c->d.n_cm + DML_BLOCK - 1) / DML_BLOCK));
-  dim3 gw(clamp_grid((c->d.n_cm + 3) / 4));
-  int nb = c->d.nblocks;
-  hipLaunchKernelGGL(k_zero_cells, gc, dim3(DML_BLOCK), 0, c->st, c->d, gcs);
-  hipLaunchKernelGGL(k_cell_key, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d, gcs);
-  hipLaunchKernelGGL(k_cell_sort_w, gw, dim3(DML_BLOCK), 0, c->st, c->d, gcs);
+void enq_sort_build(dml_ctx *c, int gcs) {
+  hipLaunchKernelGGL(k_cell_sort_w, dim3(clamp_grid((c->d.n_cm + 3) / 4)), dim3(DML_BLOCK), 0,
+                     c->st, c->d, gcs);
   if (by_cell(c))
     hipLaunchKernelGGL(k_force_order, dim3(clamp_grid((c->d.n_cm + 63) / 64)), dim3(FO_BLOCK), 0,
                        c->st, c->d);
   enq_listbuild(c);
 }
 
-// begin_ov: the overlap rounds follow
-void enq_test_update(dml_ctx *c, int gcs, int begin_ov = 0) {
+void enq_cells_lists(dml_ctx *c, int gcs) {
   c->fresh = 0;
+  dim3 gc(clamp_grid((c->d.n_cm + DML_BLOCK - 1) / DML_BLOCK));
+  int nb = c->d.nblocks;
+  hipLaunchKernelGGL(k_zero_cells, gc, dim3(DML_BLOCK), 0, c->st, c->d, gcs);
+  hipLaunchKernelGGL(k_cell_key, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d, gcs);
+  enq_sort_build(c, gcs);
+}
+
+// slots of the largest replica
+int most_slots(const dml_ctx *c) {
+  int n = 0;
+  for (auto &h : c->reps) n = std::max(n, h.p.pcap);
+  return n;
+}
+// Every replica small enough for the kernels that give it one workgroup.  They
+// take the place of 4, 2 and 5 to 7 launches, each 1.3 us or more of a step
+// whatever it does, and lose to them where a workgroup needs many passes:
+// 100 steps of a 1,000-slot electrode cell 9.3 -> 7.3 ms, of a GCMC run of 594
+// ions 20.6 -> 17.7, 60 steps of a dense Ermak system with piston of 1,000
+// 6.1 -> 4.9, 4,000 6.8 -> 6.3; (with up to 12 passes) 7,000 7.2 -> 7.4, 12,000
+// 8.0 -> 9.9
+bool small_reps(const dml_ctx *c) { return most_slots(c) <= SM_SLOTS; }
+
+void enq_step_small(dml_ctx *c, int ops, int rep_only = -1) {
+  hipLaunchKernelGGL(k_step_small, dim3(rep_only >= 0 ? 1 : c->nrep), dim3(SM_BLOCK), 0, c->st,
+                     c->d, ops, rep_only);
+}
+
+// begin_ov: the overlap rounds follow; fired: only the replicas that added a
+// block (small replicas)
+void enq_test_update(dml_ctx *c, int gcs, int begin_ov = 0, int fired = 0) {
+  c->fresh = 0;
+  if (small_reps(c)) {
+    const int m = most_slots(c);
+    const dim3 g(c->nrep), b(SM_BLOCK);
+    if (m <= SM_BLOCK)
+      hipLaunchKernelGGL(k_update_small<1>, g, b, 0, c->st, c->d, gcs, begin_ov, fired);
+    else if (m <= 2 * SM_BLOCK)
+      hipLaunchKernelGGL(k_update_small<2>, g, b, 0, c->st, c->d, gcs, begin_ov, fired);
+    else
+      hipLaunchKernelGGL(k_update_small<4>, g, b, 0, c->st, c->d, gcs, begin_ov, fired);
+    enq_sort_build(c, gcs);
+    return;
+  }
   hipLaunchKernelGGL(k_pbc_dispmax, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_dispmax_final, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d, begin_ov);
   enq_cells_lists(c, gcs);
@@ -568,6 +605,11 @@ void enq_forces(dml_ctx *c, int fuse_b, int only_ermak) {
     launch_force_lpa<1>(c, c->lpa, only_ermak);
   else
     launch_force_lpa<0>(c, c->lpa, only_ermak);
+  if (small_reps(c)) {
+    hipLaunchKernelGGL(k_ghost_small, dim3(c->nrep), dim3(SM_BLOCK), 0, c->st, c->d, only_ermak,
+                       fuse_b);
+    return;
+  }
   hipLaunchKernelGGL(k_ghost_scatter, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d,
                      only_ermak);
   if (fuse_b)
@@ -676,13 +718,21 @@ static void enq_gcmc_batch(dml_ctx *c, int r, const double *u, const double *g) 
 }
 
 static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g, double act,
-                     int nadj) {
+                     int nadj, int before = 0, int after = 0) {
   c->fresh = 0;
   const int nb = c->d.nblocks;
+  const bool small = small_reps(c);
+  int batched = 0;
+  for (auto &h : c->reps) batched |= h.p.gcmc_mode & DML_GCMC_BATCHED;
   for (int stage = 0; stage < 2; stage++) {
+    if (stage == 0 && small) {
+      enq_step_small(c, before | SM_GC0, rep_only);
+      continue;
+    }
     if (stage == 1) {
-      hipLaunchKernelGGL(k_gb_begin, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d,
-                         rep_only, act, nadj);
+      if (batched)
+        hipLaunchKernelGGL(k_gb_begin, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d,
+                           rep_only, act, nadj);
       for (int r = 0; r < c->nrep; r++) {
         const RepParams &p = c->reps[r].p;
         if ((rep_only < 0 || r == rep_only) && p.gb_cap > 0 && (p.gcmc_mode & DML_GCMC_BATCHED) &&
@@ -695,6 +745,10 @@ static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g,
       else
         hipLaunchKernelGGL(k_gcmc_run, dim3(c->nrep), dim3(DML_GCMC_BLOCK), 0, c->st, c->d, -1,
                            u, g, act, nadj);
+      if (small) {
+        enq_step_small(c, SM_GC1 | after, rep_only);
+        return;
+      }
     }
     hipLaunchKernelGGL(k_gc_count, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d, rep_only, stage);
     hipLaunchKernelGGL(k_gc_scan, dim3(c->nrep), dim3(1024), 0, c->st, c->d, rep_only, stage);
@@ -705,6 +759,10 @@ static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g,
 
 void enq_f2cg(dml_ctx *c) {
   c->fresh = 0;
+  if (small_reps(c)) {
+    enq_step_small(c, SM_F2CG);
+    return;
+  }
   int nb = c->d.nblocks;
   hipLaunchKernelGGL(k_f2cg_mark, dim3(nb), dim3(DML_BLOCK), 0, c->st, c->d);
   hipLaunchKernelGGL(k_f2cg_scan, dim3(c->nrep), dim3(1024), 0, c->st, c->d);
@@ -714,10 +772,16 @@ void enq_f2cg(dml_ctx *c) {
 }
 
 // bloques, then test_update of the replicas that added a block (dana.F90:771)
-void enq_bloques(dml_ctx *c) {
+// (after: phases that follow, of small replicas)
+void enq_bloques(dml_ctx *c, int after = 0) {
   c->fresh = 0;
   const int rb = (c->nrep + 63) / 64;
   hipLaunchKernelGGL(k_chunk_run, dim3(c->nrep), dim3(DML_BLOCK), 0, c->st, c->d);
+  if (small_reps(c)) {
+    enq_test_update(c, 1, 0, 1);
+    enq_step_small(c, SM_UNMASK | after);
+    return;
+  }
   hipLaunchKernelGGL(k_mask_fired, dim3(rb), dim3(64), 0, c->st, c->d, 1);
   enq_test_update(c, 1);
   hipLaunchKernelGGL(k_mask_fired, dim3(rb), dim3(64), 0, c->st, c->d, 0);
@@ -739,6 +803,21 @@ void enq_step(dml_ctx *c) {
   enq_test_update(c, 0, c->any_rounds);
   enq_overlap(c);
   enq_test_update(c, 1);
+  if (small_reps(c)) {
+    // the same phases, as many as go together in a launch
+    int ops = SM_F2CG;
+    const int rho = c->any_piston || c->any_chunks ? SM_RHO : 0;
+    const int end = (c->any_piston ? SM_MAXZ : 0) | SM_END;
+    if (c->any_gcmc) {
+      enq_gcmc(c, -1, nullptr, nullptr, 0.0, 0, ops, rho | (c->any_chunks ? 0 : end));
+      ops = 0;
+    } else {
+      ops |= rho | (c->any_chunks ? 0 : end);
+    }
+    if (ops) enq_step_small(c, ops);
+    if (c->any_chunks) enq_bloques(c, end);
+    return;
+  }
   enq_f2cg(c);
   if (c->any_gcmc)  // gcmc_run after F -> CG (dana.F90:238-241)
     enq_gcmc(c, -1, nullptr, nullptr, 0.0, 0);

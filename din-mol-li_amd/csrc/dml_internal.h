@@ -21,6 +21,16 @@
 #define OVT_BLOCK 512 // threads of the overlap tail
 #define OVX_MAX 16  // row entries listed per atom for the reference-order overlap pass
 #define OVX_BLOCK 1024
+#define SM_BLOCK 1024  // threads of the kernels that take a small replica each
+#define SM_SLOTS (4 * SM_BLOCK)  // most slots of a small replica
+// phases of k_step_small, in this order
+#define SM_UNMASK 1
+#define SM_F2CG 2
+#define SM_GC0 4
+#define SM_GC1 8
+#define SM_RHO 16
+#define SM_MAXZ 32
+#define SM_END 64
 #define FO_BLOCK 512  // threads of k_force_order
 #define FO_LEAST 200000  // slots from which the force kernel takes the atoms cell by cell
 #define NEAR_MAX 4  // row positions within rcut listed per atom by the row build

@@ -9,6 +9,10 @@ __global__ void k_load_state(DevState s, int poff, int n, int nref, int ngc, int
 __global__ void k_pack_state(DevState s, int poff, int n, int want, unsigned char *out);
 __global__ void k_force_rebuild(DevState s);
 __global__ void k_force_order(DevState s);
+template <int PER>
+__global__ void k_update_small(DevState s, int gcs, int begin, int fired);
+__global__ void k_ghost_small(DevState s, int only_ermak, int fuse_b);
+__global__ void k_step_small(DevState s, int ops, int rep_only);
 __global__ void k_zero_cells(DevState s, int gcs);
 __global__ void k_cell_key(DevState s, int gcs);
 __global__ void k_cell_sort(DevState s, int gcs);

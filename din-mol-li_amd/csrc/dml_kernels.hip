@@ -93,33 +93,37 @@ __device__ inline void block_top2(double &a1, double &a2, double *sh) {
 // (Neighbor.F90:635-666) with the rebuild decision of Neighbor.F90:696-710.
 // The last block of a replica merges the per-block top-2 values.
 // ------------------------------------------------------------------------
+// an atom at (x, y, z) with pos_old (ox, oy, oz) back into the box; its
+// squared displacement
+__device__ inline double pbc_one(const DevState &s, const RepParams &P, int slot, double &x,
+                                 double &y, double z, double ox, double oy, double oz) {
+  double bx = P.box[0], by = P.box[1];
+  int moved = 0;
+  if (x >= bx) {
+    x -= bx; s.px[slot] = x; ox -= bx; s.ox[slot] = ox; moved = 1;
+  } else if (x < 0.0) {
+    x += bx; s.px[slot] = x; ox += bx; s.ox[slot] = ox; moved = 1;
+  }
+  if (y >= by) {
+    y -= by; s.py[slot] = y; oy -= by; s.oy[slot] = oy; moved = 1;
+  } else if (y < 0.0) {
+    y += by; s.py[slot] = y; oy += by; s.oy[slot] = oy; moved = 1;
+  }
+  if (moved) put_pf4(s, slot, x, y, z, s.species[slot]);
+  return dot3(x - ox, y - oy, z - oz);
+}
+
 __global__ void __launch_bounds__(DML_BLOCK) k_pbc_dispmax(DevState s) {
   __shared__ double sh[2 * DML_BLOCK / WAVE];
   int r;
   const RepParams &P = rep_of_block(s, blockIdx.x, &r);
   if (P.halted) return;
   int slot = blockIdx.x * DML_BLOCK + threadIdx.x;
-  int local = slot - P.poff;
-  double d = -1.0;
-  if (local < P.nslots && (s.flags[slot] & DML_FL_ALIVE)) {
+  double a1 = -1.0, a2 = -1.0;
+  if (slot - P.poff < P.nslots && (s.flags[slot] & DML_FL_ALIVE)) {
     double x = s.px[slot], y = s.py[slot];
-    double bx = P.box[0], by = P.box[1];
-    int moved = 0;
-    if (x >= bx) {
-      x -= bx; s.px[slot] = x; s.ox[slot] -= bx; moved = 1;
-    } else if (x < 0.0) {
-      x += bx; s.px[slot] = x; s.ox[slot] += bx; moved = 1;
-    }
-    if (y >= by) {
-      y -= by; s.py[slot] = y; s.oy[slot] -= by; moved = 1;
-    } else if (y < 0.0) {
-      y += by; s.py[slot] = y; s.oy[slot] += by; moved = 1;
-    }
-    double z = s.pz[slot];
-    if (moved) put_pf4(s, slot, x, y, z, s.species[slot]);
-    d = dot3(x - s.ox[slot], y - s.oy[slot], z - s.oz[slot]);
+    a1 = pbc_one(s, P, slot, x, y, s.pz[slot], s.ox[slot], s.oy[slot], s.oz[slot]);
   }
-  double a1 = d, a2 = -1.0;
   block_top2(a1, a2, sh);
   if (threadIdx.x == 0) {
     s.part_d[2 * blockIdx.x] = a1;
@@ -131,6 +135,26 @@ __global__ void __launch_bounds__(DML_BLOCK) k_pbc_dispmax(DevState s) {
 __device__ inline void ov_begin_rep(const DevState &s, int r) {
   s.rp[r].ov_round += OV_STAMPS;
   s.ov_last[r] = -1;
+}
+
+// the skin test of a replica's two largest displacements (one thread)
+__device__ inline int dispmax_decide(const DevState &s, int r, double a1, double a2) {
+  RepParams *Pw = s.rp + r;
+  top2_merge(a1, a2, 1e-16, 1e-16);  // initial values of inq_dispmax
+  Pw->d1 = a1;
+  Pw->d2 = a2;
+  int reb = (!Pw->listed) || (sqrt(a1) + sqrt(a2) > Pw->skin);
+  Pw->rebuild = reb;
+  if (reb) {
+    Pw->listed = 1;
+    Pw->any_ghost = 0;
+    Pw->nlimbo = 0;  // the rebuild cleans the limbo (Groups.F90:1036-1053)
+    // new rows: the cell-tile and wave-per-cell row builds list their
+    // entries within rcut
+    Pw->ovn_stamp = Pw->lb_kind != 1 ? Pw->step + 1 : 0;
+    atomicAdd(&cnt_of(s, r, 0).nupd, 1ull);
+  }
+  return reb;
 }
 
 // one block per replica merges the block partials (a kernel boundary orders
@@ -150,22 +174,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_dispmax_final(DevState s, int beg
   for (int q = threadIdx.x; q < nb; q += blockDim.x)
     top2_merge(a1, a2, s.part_d[2 * (b0 + q)], s.part_d[2 * (b0 + q) + 1]);
   block_top2(a1, a2, sh);
-  if (threadIdx.x == 0) {
-    top2_merge(a1, a2, 1e-16, 1e-16);  // initial values of inq_dispmax
-    Pw->d1 = a1;
-    Pw->d2 = a2;
-    int reb = (!Pw->listed) || (sqrt(a1) + sqrt(a2) > Pw->skin);
-    Pw->rebuild = reb;
-    if (reb) {
-      Pw->listed = 1;
-      Pw->any_ghost = 0;
-      Pw->nlimbo = 0;  // the rebuild cleans the limbo (Groups.F90:1036-1053)
-      // new rows: the cell-tile and wave-per-cell row builds list their
-      // entries within rcut
-      Pw->ovn_stamp = Pw->lb_kind != 1 ? Pw->step + 1 : 0;
-      atomicAdd(&cnt_of(s, r, 0).nupd, 1ull);
-    }
-  }
+  if (threadIdx.x == 0) dispmax_decide(s, r, a1, a2);
 }
 
 __global__ void k_force_rebuild(DevState s) {
@@ -207,23 +216,16 @@ __global__ void k_zero_cells(DevState s, int gcs) {
   }
 }
 
-__global__ void __launch_bounds__(DML_BLOCK) k_cell_key(DevState s, int gcs) {
-  int r;
-  const RepParams &P = rep_of_block(s, blockIdx.x, &r);
-  if (P.halted) return;
-  if (!want_cells(P, gcs)) return;
-  int slot = blockIdx.x * DML_BLOCK + threadIdx.x;
-  int local = slot - P.poff;
-  if (local >= P.nslots) return;
-  uint8_t f = s.flags[slot];
-  if (P.rebuild && (f & DML_FL_LIMBO)) {  // igroup_clean (Groups.F90:1036-1053)
+// an atom (flags f) into its cell's bucket
+__device__ inline void cell_key_one(const DevState &s, const RepParams &P, int r, int slot,
+                                    int rebuild, uint8_t f, double x, double y, double z) {
+  if (rebuild && (f & DML_FL_LIMBO)) {  // igroup_clean (Groups.F90:1036-1053)
     s.flags[slot] = f & (uint8_t)~DML_FL_LIMBO;
-    atomicMin(&s.rp[r].free_lo, local);
+    atomicMin(&s.rp[r].free_lo, slot - P.poff);
     return;
   }
   if (!(f & DML_FL_ALIVE)) return;
-  double x = s.px[slot], y = s.py[slot], z = s.pz[slot];
-  if (P.rebuild) {  // update(): pos_old = pos (Neighbor.F90:620-624)
+  if (rebuild) {  // update(): pos_old = pos (Neighbor.F90:620-624)
     s.ox[slot] = x;
     s.oy[slot] = y;
     s.oz[slot] = z;
@@ -248,6 +250,89 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_key(DevState s, int gcs) {
   }
   s.bucket[P.boff + (int64_t)cell * P.bcap + rank] = slot;
 }
+
+__global__ void __launch_bounds__(DML_BLOCK) k_cell_key(DevState s, int gcs) {
+  int r;
+  const RepParams &P = rep_of_block(s, blockIdx.x, &r);
+  if (P.halted) return;
+  if (!want_cells(P, gcs)) return;
+  int slot = blockIdx.x * DML_BLOCK + threadIdx.x;
+  if (slot - P.poff >= P.nslots) return;
+  cell_key_one(s, P, r, slot, P.rebuild, s.flags[slot], s.px[slot], s.py[slot], s.pz[slot]);
+}
+
+// a[0, n) = 0 by a workgroup, 16 bytes a store between the ends
+__device__ inline void blk_zero_i32(int32_t *a, int64_t n) {
+  const int64_t head = min(n, (int64_t)(-(uintptr_t)a >> 2 & 3));
+  const int64_t n4 = (n - head) / 4;
+  for (int64_t q = threadIdx.x; q < n4; q += blockDim.x)
+    reinterpret_cast<int4 *>(a + head)[q] = make_int4(0, 0, 0, 0);
+  if ((int64_t)threadIdx.x < head) a[threadIdx.x] = 0;
+  const int64_t t = head + 4 * n4 + threadIdx.x;
+  if (t < n) a[t] = 0;
+}
+
+// The first half of a test_update of small replicas, one workgroup each:
+// do_pbc, the skin test, the cells cleared and filled (k_pbc_dispmax,
+// k_dispmax_final, k_zero_cells, k_cell_key).  begin as for k_dispmax_final;
+// fired: the replicas that added no block sit it out (HALT_MASK).
+// Bound by its barriers and a handful of round trips; a thread holds PER slots.
+template <int PER>
+__global__ void __launch_bounds__(SM_BLOCK) k_update_small(DevState s, int gcs, int begin,
+                                                           int fired) {
+  __shared__ double sh[2 * SM_BLOCK / WAVE];
+  __shared__ int sh_go, sh_reb;
+  const int r = blockIdx.x, tid = threadIdx.x;
+  RepParams *Pw = s.rp + r;
+  const RepParams &P = *Pw;
+  if (tid == 0) {
+    if (begin) {
+      ov_begin_rep(s, r);
+      if (r == 0) s.wl_cnt[0] = s.wl_cnt[1] = s.wl_cnt[2] = 0;
+    }
+    if (fired && !Pw->chunk_fired) Pw->halted |= HALT_MASK;
+    sh_go = !Pw->halted;
+  }
+  __syncthreads();
+  // (a replica's cells lie together in the flat list, from coff on)
+  blk_zero_i32(s.cm_nref + P.coff, P.creg);
+  if (!sh_go) return;
+  const int poff = P.poff, n = P.nslots;
+  // the slots of this thread, loaded at once and kept
+  uint8_t f[PER];
+  double x[PER], y[PER], z[PER], ox[PER], oy[PER], oz[PER];
+#pragma unroll
+  for (int u = 0; u < PER; u++) {
+    const int q = u * SM_BLOCK + tid, i = poff + (q < n ? q : 0);
+    f[u] = s.flags[i];
+    x[u] = s.px[i]; y[u] = s.py[i]; z[u] = s.pz[i];
+    ox[u] = s.ox[i]; oy[u] = s.oy[i]; oz[u] = s.oz[i];
+    if (q >= n) f[u] = 0;
+  }
+  double a1 = -1.0, a2 = -1.0;
+#pragma unroll
+  for (int u = 0; u < PER; u++)
+    if (f[u] & DML_FL_ALIVE)
+      top2_merge(a1, a2, pbc_one(s, P, poff + u * SM_BLOCK + tid, x[u], y[u], z[u], ox[u], oy[u],
+                                 oz[u]), -1.0);
+  block_top2(a1, a2, sh);
+  if (tid == 0) {
+    sh_reb = dispmax_decide(s, r, a1, a2);
+    if (sh_reb) Pw->fo_n = 0;
+  }
+  __syncthreads();
+  const int reb = sh_reb;
+  if (!reb && !(gcs && P.reservoir == DML_GCMC)) return;
+  blk_zero_i32(s.cell_cnt + P.coff, ncell_total(P));
+  __builtin_amdgcn_s_waitcnt(0);  // the counts are clear before any wave adds
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < PER; u++)
+    if (f[u]) cell_key_one(s, P, r, poff + u * SM_BLOCK + tid, reb, f[u], x[u], y[u], z[u]);
+}
+template __global__ void k_update_small<1>(DevState, int, int, int);
+template __global__ void k_update_small<2>(DevState, int, int, int);
+template __global__ void k_update_small<4>(DevState, int, int, int);
 
 // order each bucket like the head/next chain: descending hs%b slot for
 // cells (push-front, Cells.F90:299-300), ascending for the Verlet scan
@@ -1764,15 +1849,7 @@ INST_FORCE(32)
 INST_FORCE(64)
 
 // reactions of rows built from ghost-layer cells (nobody lists those atoms)
-__global__ void __launch_bounds__(DML_BLOCK) k_ghost_scatter(DevState s, int only_ermak) {
-  int t = blockIdx.x * DML_BLOCK + threadIdx.x;
-  int r;
-  const RepParams &P = rep_of_block(s, blockIdx.x, &r);
-  if (P.halted) return;
-  if (!P.any_ghost) return;
-  if (only_ermak && P.integrator != DML_ERMAK) return;
-  if (t - P.poff >= P.nref) return;
-  int i = s.ref_order[t];
+__device__ inline void ghost_one(const DevState &s, const RepParams &P, int i) {
   if (!(s.rowflag[i] & 1)) return;
   int k = s.species[i];
   double xi = s.px[i], yi = s.py[i], zi = s.pz[i];
@@ -1806,6 +1883,35 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ghost_scatter(DevState s, int onl
     double u = eps * b * (b - 2);
     u = u + eps;
     atomicAdd(&s.epot[j], u * .5);
+  }
+}
+
+__global__ void __launch_bounds__(DML_BLOCK) k_ghost_scatter(DevState s, int only_ermak) {
+  int t = blockIdx.x * DML_BLOCK + threadIdx.x;
+  int r;
+  const RepParams &P = rep_of_block(s, blockIdx.x, &r);
+  if (P.halted) return;
+  if (!P.any_ghost) return;
+  if (only_ermak && P.integrator != DML_ERMAK) return;
+  if (t - P.poff >= P.nref) return;
+  ghost_one(s, P, s.ref_order[t]);
+}
+
+// the same of small replicas, one workgroup each, then ermak_b (fuse_b)
+__global__ void __launch_bounds__(SM_BLOCK) k_ghost_small(DevState s, int only_ermak, int fuse_b) {
+  const RepParams &P = s.rp[blockIdx.x];
+  if (P.halted || !P.any_ghost) return;
+  if (only_ermak && P.integrator != DML_ERMAK) return;
+  const int32_t *ord = s.ref_order + P.poff;
+  const int n = P.nref;
+  for (int t = threadIdx.x; t < n; t += SM_BLOCK) ghost_one(s, P, ord[t]);
+  if (!fuse_b || P.integrator != DML_ERMAK) return;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  for (int t = threadIdx.x; t < n; t += SM_BLOCK) {
+    const int i = ord[t];
+    ermak_b_one(s, P, i, atomic_load_d(&s.fx[i]), atomic_load_d(&s.fy[i]),
+                atomic_load_d(&s.fz[i]));
   }
 }
 
@@ -2786,6 +2892,15 @@ __device__ inline void rep_exscan2(int32_t *part, int stride, int b0, int nb, in
 // F -> CG at step end and removal from hs%ref (dana.F90:228-236): stable
 // compaction of each replica's ref order
 // ------------------------------------------------------------------------
+// a fresh deposit becomes an electrode atom and leaves the ref list (0)
+__device__ inline int f2cg_one(const DevState &s, int i) {
+  if (s.species[i] != SP_F) return 1;
+  s.species[i] = SP_CG;
+  put_pf4_sp(s, i, SP_CG);
+  s.flags[i] &= (uint8_t)~(DML_FL_REF | DML_FL_GCMC);
+  s.ref_pos[i] = -1;
+  return 0;
+}
 __global__ void __launch_bounds__(DML_BLOCK) k_f2cg_mark(DevState s) {
   __shared__ int cnt;
   int t = blockIdx.x * DML_BLOCK + threadIdx.x;
@@ -2796,15 +2911,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_f2cg_mark(DevState s) {
   __syncthreads();
   if (P.any_f && t - P.poff < P.nref) {
     int i = s.ref_order[t];
-    int keep = 1;
-    if (s.species[i] == SP_F) {
-      s.species[i] = SP_CG;
-      put_pf4_sp(s, i, SP_CG);
-      s.flags[i] &= (uint8_t)~(DML_FL_REF | DML_FL_GCMC);
-      s.ref_pos[i] = -1;
-      keep = 0;
-    }
-    if (keep) atomicAdd(&cnt, 1);
+    if (f2cg_one(s, i)) atomicAdd(&cnt, 1);
   }
   __syncthreads();
   if (threadIdx.x == 0) s.part_i[blockIdx.x] = cnt;
@@ -2868,6 +2975,13 @@ __global__ void k_f2cg_end(DevState s) {
 // ------------------------------------------------------------------------
 // piston: calc_rho (dana.F90:521-549) and maxz (776-794)
 // ------------------------------------------------------------------------
+__device__ inline bool in_band(const DevState &s, const RepParams &P, int slot) {
+  const uint8_t f = s.flags[slot];
+  const double z = s.pz[slot];
+  if (!(f & DML_FL_ALIVE)) return false;
+  const double zt = P.reservoir == DML_CHUNKS ? P.z1 : P.zmax;  // the chunks sensor
+  return z > P.z0 && z < zt;
+}
 __global__ void __launch_bounds__(DML_BLOCK) k_calc_rho(DevState s) {
   __shared__ int cnt;
   int slot = blockIdx.x * DML_BLOCK + threadIdx.x;
@@ -2876,12 +2990,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_calc_rho(DevState s) {
   if (P.halted) return;
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
-  int local = slot - P.poff;
-  if (local < P.nslots && (s.flags[slot] & DML_FL_ALIVE)) {
-    double z = s.pz[slot];
-    const double zt = P.reservoir == DML_CHUNKS ? P.z1 : P.zmax;  // the chunks sensor
-    if (z > P.z0 && z < zt) atomicAdd(&cnt, 1);
-  }
+  if (slot - P.poff < P.nslots && in_band(s, P, slot)) atomicAdd(&cnt, 1);
   __syncthreads();
   if (threadIdx.x == 0 && cnt) atomicAdd(&s.rp[r].rho_count, cnt);
 }
@@ -2967,6 +3076,15 @@ __device__ inline double piston_lohi(const RepParams &P) {
   return ((P.h / tau) * ((P.rho0 - rho) / rho));
 }
 
+__device__ inline void maxz_one(const DevState &s, const RepParams &P, int slot, double lohi) {
+  if (!(s.flags[slot] & DML_FL_ALIVE)) return;
+  double z = s.pz[slot];
+  if (z > P.z0) {
+    double nz = z - lohi * (z - P.z0);
+    s.pz[slot] = nz;
+    put_pf4(s, slot, s.px[slot], s.py[slot], nz, s.species[slot]);
+  }
+}
 __global__ void __launch_bounds__(DML_BLOCK) k_maxz(DevState s) {
   int slot = blockIdx.x * DML_BLOCK + threadIdx.x;
   int r;
@@ -2974,16 +3092,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_maxz(DevState s) {
   if (P.halted) return;
   if (!P.piston) return;
   if (slot == P.poff) s.rp[r].ovn_stamp = 0;  // positions move
-  int local = slot - P.poff;
-  if (local < P.nslots && (s.flags[slot] & DML_FL_ALIVE)) {
-    double z = s.pz[slot];
-    if (z > P.z0) {
-      double lohi = piston_lohi(P);
-      double nz = z - lohi * (z - P.z0);
-      s.pz[slot] = nz;
-      put_pf4(s, slot, s.px[slot], s.py[slot], nz, s.species[slot]);
-    }
-  }
+  if (slot - P.poff < P.nslots) maxz_one(s, P, slot, piston_lohi(P));
 }
 
 // per-replica bookkeeping of the per-routine entry points: 0 = clear the
@@ -3011,9 +3120,7 @@ __global__ void k_rep_op(DevState s, int op) {
 
 // step end: advance the per-replica step counter (and the piston zmax,
 // which no kernel of k_maxz reads)
-__global__ void k_step_end(DevState s) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= s.nrep) return;
+__device__ inline void step_end_rep(const DevState &s, int r) {
   RepParams *Pw = s.rp + r;
   if (Pw->halted) return;
   if (Pw->piston) {
@@ -3026,6 +3133,10 @@ __global__ void k_step_end(DevState s) {
   cnt_of(s, r, 0).steps += 1;
   cnt_of(s, r, 0).particle_steps += (unsigned long long)Pw->nat;
   if (Pw->step_limit > 0 && Pw->step >= Pw->step_limit) Pw->halted |= HALT_PAUSED;
+}
+__global__ void k_step_end(DevState s) {
+  int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < s.nrep) step_end_rep(s, r);
 }
 
 // hold the replicas that already have lists out of the first rebuild of
@@ -3393,6 +3504,111 @@ __global__ void __launch_bounds__(DML_BLOCK) k_gc_copy(DevState s, int rep_only)
     s.ref_order[t] = v;
     s.ref_pos[v] = local;
   }
+}
+
+// The phases of a step after its second test_update (and the list work
+// around gcmc_run) for small replicas, one workgroup each: the phases of ops
+// in the order of the bits below.  The compactions are those of k_f2cg_* and
+// k_gc_*, SM_BLOCK entries at a time, the ref list in place (an entry only
+// moves down, and a pass reads its entries before any is written).  Bound by a
+// few round trips a pass; 5 launches for f_to_cg alone, 7 around a gcmc_run,
+// took 3 to 4.5 us each.
+__global__ void __launch_bounds__(SM_BLOCK) k_step_small(DevState s, int ops, int rep_only) {
+  __shared__ int sh[SM_BLOCK / WAVE];
+  const int r = rep_only >= 0 ? rep_only : (int)blockIdx.x, tid = threadIdx.x;
+  RepParams *Pw = s.rp + r;
+  const RepParams &P = *Pw;
+  if (ops & SM_UNMASK) {
+    if (tid == 0) {
+      Pw->halted &= ~HALT_MASK;
+      Pw->chunk_fired = 0;
+    }
+    __syncthreads();
+  }
+  const int halted = P.halted, poff = P.poff;
+  int32_t *rord = s.ref_order + poff;
+  int tot;
+  if ((ops & SM_F2CG) && !halted && P.any_f) {
+    const int n = P.nref;
+    int at = 0;
+    for (int t0 = 0; t0 < n; t0 += SM_BLOCK) {
+      const int i = t0 + tid < n ? rord[t0 + tid] : -1;
+      const int keep = i >= 0 && f2cg_one(s, i);
+      const int p = at + blk_scan01(keep, sh, &tot);
+      if (keep) {
+        rord[p] = i;
+        s.ref_pos[i] = p;
+      }
+      at += tot;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      Pw->nref = at;
+      Pw->any_f = 0;
+    }
+    __syncthreads();
+  }
+  if ((ops & SM_GC0) && gc_sel(P, r, rep_only)) {
+    if (halted) {
+      if (tid == 0) Pw->gc_pending = 0;  // nothing staged for this call
+    } else {
+      int a1 = 0, a2 = 0;
+      const int n = P.ngc;
+      for (int t0 = 0; t0 < n; t0 += SM_BLOCK) {
+        int v1, k1, v2, k2;
+        gc_keep(s, P, poff + t0 + tid, 0, &v1, &k1, &v2, &k2);
+        const int p1 = a1 + blk_scan01(k1, sh, &tot);
+        a1 += tot;
+        const int p2 = a2 + blk_scan01(k2, sh, &tot);
+        a2 += tot;
+        if (k1) s.wl[1][poff + p1] = v1;
+        if (k2) s.ref_tmp[poff + p2] = v2;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        Pw->gc_len = a1;
+        Pw->gc_inv = a2;
+        Pw->gc_pending = 1;
+      }
+    }
+  }
+  if ((ops & SM_GC1) && gc_sel(P, r, rep_only) && P.gc_pending == 2) {
+    int a1 = 0, a2 = 0;
+    const int n = max(P.gc_len, P.ref_len);
+    for (int t0 = 0; t0 < n; t0 += SM_BLOCK) {
+      int v1, k1, v2, k2;
+      gc_keep(s, P, poff + t0 + tid, 1, &v1, &k1, &v2, &k2);
+      const int p1 = a1 + blk_scan01(k1, sh, &tot);
+      a1 += tot;
+      const int p2 = a2 + blk_scan01(k2, sh, &tot);
+      a2 += tot;
+      if (k1) s.gc_order[poff + p1] = v1;
+      if (k2) {
+        rord[p2] = v2;
+        s.ref_pos[v2] = p2;
+      }
+    }
+    __syncthreads();
+    if (tid == 0) {
+      Pw->ngc = a1;
+      Pw->nref = a2;
+      Pw->gc_pending = 3;
+    }
+  }
+  if ((ops & SM_RHO) && !halted) {
+    int c = 0;
+    for (int q = tid; q < P.nslots; q += SM_BLOCK) c += in_band(s, P, poff + q);
+    const int all = blk_sum(c, sh);
+    if (tid == 0) Pw->rho_count += all;
+    __syncthreads();
+  }
+  if ((ops & SM_MAXZ) && !halted && P.piston) {
+    const double lohi = piston_lohi(P);
+    for (int q = tid; q < P.nslots; q += SM_BLOCK) maxz_one(s, P, poff + q, lohi);
+    if (tid == 0) Pw->ovn_stamp = 0;  // positions move
+    __syncthreads();
+  }
+  if ((ops & SM_END) && tid == 0) step_end_rep(s, r);
 }
 
 #define GC_TRACK 256
