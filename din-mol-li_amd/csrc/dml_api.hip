@@ -271,10 +271,14 @@ int take_table(dml_ctx *c) {
   return DML_OK;
 }
 
-// pinned staging of at least n bytes, null when it would be too large to keep
-constexpr size_t kPinMost = 4u << 20;
+// pinned staging of at least n bytes, null when it would be too large to keep;
+// the first kPinFirst lie behind the table's copy (pinning is a good 0.1 ms a
+// call: 8,192 trials in a new context took 0.66 ms, 0.38 in an old one)
+constexpr size_t kPinMost = 4u << 20, kPinFirst = 256u << 10;
+size_t pin_at(const dml_ctx *c) { return (table_bytes(c) + 64 + 255) / 256 * 256; }
 unsigned char *pinned(dml_ctx *c, size_t n) {
   if (n > kPinMost) return nullptr;
+  if (n <= kPinFirst) return c->h_rp + pin_at(c);
   if (n > c->h_cap) {
     if (c->h_pin) hipHostFree(c->h_pin);
     c->h_pin = nullptr;
@@ -1098,7 +1102,8 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
     d.rp = (RepParams *)q;
     d.err = q ? (int32_t *)(q + table_bytes(c)) : nullptr;
   }
-  if (hipHostMalloc((void **)&c->h_rp, table_bytes(c) + 64, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc((void **)&c->h_rp, pin_at(c) + kPinFirst, hipHostMallocDefault) !=
+      hipSuccess) {
     c->h_rp = nullptr;
     e |= 1;
   }
