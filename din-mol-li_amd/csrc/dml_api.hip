@@ -106,7 +106,9 @@ struct dml_ctx {
   int64_t gb_total = 0;      // batched-GCMC trial pool (sum of the replicas' capacities)
   int dev = 0;               // the GPU current at creation
   // the host mirror (reps[].p) holds what the device table does: set by every
-  // fetch and upload, cleared by whatever may change the table
+  // fetch and upload, cleared by whatever may change the table.  A call that
+  // may yet refuse or fail leaves the mirror alone: it works on a copy and
+  // stores that once nothing can fail but the upload
   int fresh = 0;
   int err_seen = 0;          // error bits of the last fetch
   unsigned char *h_rp = nullptr;    // pinned: the table and the error word
@@ -374,6 +376,7 @@ int upload_params(dml_ctx *c) {
   assign_list_kernels(c);
   std::vector<RepParams> v(c->nrep);
   for (int r = 0; r < c->nrep; r++) v[r] = c->reps[r].p;
+  c->fresh = 0;
   HIPCHECK(hipMemcpyAsync(c->d.rp, v.data(), sizeof(RepParams) * c->nrep, hipMemcpyHostToDevice,
                           c->st));
   c->fresh = 1;
@@ -427,7 +430,12 @@ int alloc_cells(dml_ctx *c) {
   e |= dalloc(&c->d.gb_chead, CS);
   e |= dalloc(&c->d.gb_ccnt, CS);
   e |= dalloc(&c->d.gb_claim, CS);
-  if (e) return DML_E_NOMEM;
+  if (e) {
+    // the next call that needs cells tries again, on the layout of the device table
+    c->cells_dirty = 1;
+    c->fresh = 0;
+    return DML_E_NOMEM;
+  }
   HIPCHECK(hipMemsetAsync(c->d.cell_cnt, 0, sizeof(int32_t) * C, c->st));
   HIPCHECK(hipMemsetAsync(c->d.gb_chead, 0, sizeof(unsigned long long) * CS, c->st));
   HIPCHECK(hipMemsetAsync(c->d.gb_ccnt, 0, sizeof(unsigned long long) * CS, c->st));
@@ -927,11 +935,8 @@ double *upload_tmp(dml_ctx *c, const double *h, int64_t n) {
 }
 
 // the lists of the reference-order overlap pass, once a replica asks for it
-int ensure_exact(dml_ctx *c) {
-  if (c->d.ovx_n) return DML_OK;
-  int any = 0;
-  for (auto &h : c->reps) any |= h.p.overlap_mode == DML_OVERLAP_EXACT;
-  if (!any) return DML_OK;
+int ensure_exact(dml_ctx *c, int overlap_mode) {
+  if (c->d.ovx_n || overlap_mode != DML_OVERLAP_EXACT) return DML_OK;
   uint8_t *n = nullptr;
   uint32_t *b = nullptr;
   unsigned long long *l = nullptr, *m = nullptr;
@@ -1180,7 +1185,9 @@ int dml_create_ensemble(int32_t nrep, const dml_config *cfgs, dml_ctx **out) {
     for (int q = 0; q < c->reps[r].p.pcap / DML_BLOCK; q++)
       b2r[c->reps[r].p.poff / DML_BLOCK + q] = r;
   hipMemcpyAsync(d.blk2rep, b2r.data(), sizeof(int32_t) * b2r.size(), hipMemcpyHostToDevice, c->st);
-  if (ensure_exact(c) || alloc_cells(c) || upload_params(c)) {
+  int no_exact = 0;
+  for (auto &h : c->reps) no_exact |= ensure_exact(c, h.p.overlap_mode);
+  if (no_exact || alloc_cells(c) || upload_params(c)) {
     dml_destroy(c);
     return DML_E_NOMEM;
   }
@@ -1349,14 +1356,17 @@ int dml_set_order(dml_ctx *c, int32_t rep, int32_t nref, const int32_t *ref_orde
   if (!c || rep < 0 || rep >= c->nrep) return DML_E_ARG;
   int rc = fetch_params(c);
   if (rc) return rc;
-  RepParams &p = c->reps[rep].p;
+  RepParams p = c->reps[rep].p;
   int64_t o = p.poff;
   int n = p.nslots;
+  std::vector<uint8_t> fl(std::max(n, 1));
+  HIPCHECK(hipMemcpy(fl.data(), c->d.flags + o, n, hipMemcpyDeviceToHost));
+  // both lists are checked before either is written
+  std::vector<int32_t> g, rpos, b2s;
   if (ref_order) {
     if (nref < 0 || nref > n) return DML_E_ARG;
-    std::vector<int32_t> g(std::max(nref, 1)), rpos(std::max(n, 1), -1);
-    std::vector<uint8_t> fl(std::max(n, 1));
-    HIPCHECK(hipMemcpy(fl.data(), c->d.flags + o, n, hipMemcpyDeviceToHost));
+    g.resize(std::max(nref, 1));
+    rpos.assign(std::max(n, 1), -1);
     for (int t = 0; t < nref; t++) {
       const int i = ref_order[t];
       // each listed atom once, and alive
@@ -1364,19 +1374,10 @@ int dml_set_order(dml_ctx *c, int32_t rep, int32_t nref, const int32_t *ref_orde
       g[t] = (int32_t)(o + i);
       rpos[i] = t;
     }
-    // hs%ref membership is exactly the list: the force and overlap kernels
-    // read it from the flags
-    for (int i = 0; i < n; i++)
-      fl[i] = (uint8_t)(rpos[i] >= 0 ? (fl[i] | DML_FL_REF) : (fl[i] & ~DML_FL_REF));
-    HIPCHECK(hipMemcpy(c->d.flags + o, fl.data(), n, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->d.ref_order + o, g.data(), sizeof(int32_t) * nref, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->d.ref_pos + o, rpos.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
     p.nref = nref;
   }
   if (bkey) {
-    std::vector<uint8_t> fl(std::max(n, 1));
-    HIPCHECK(hipMemcpy(fl.data(), c->d.flags + o, n, hipMemcpyDeviceToHost));
-    std::vector<int32_t> b2s(p.pcap, -1);
+    b2s.assign(p.pcap, -1);
     int amax = 0;
     for (int i = 0; i < n; i++) {
       if (!(fl[i] & DML_FL_ALIVE)) continue;
@@ -1384,13 +1385,25 @@ int dml_set_order(dml_ctx *c, int32_t rep, int32_t nref, const int32_t *ref_orde
       b2s[bkey[i]] = (int32_t)(o + i);
       amax = std::max(amax, bkey[i] + 1);
     }
-    HIPCHECK(hipMemcpy(c->d.bkey + o, bkey, sizeof(int32_t) * n, hipMemcpyHostToDevice));
-    HIPCHECK(hipMemcpy(c->d.b2slot + o, b2s.data(), sizeof(int32_t) * p.pcap, hipMemcpyHostToDevice));
     p.b_amax = amax;
     p.bfree_lo = 0;
   }
+  if (ref_order) {
+    // hs%ref membership is exactly the list: the force and overlap kernels
+    // read it from the flags
+    for (int i = 0; i < n; i++)
+      fl[i] = (uint8_t)(rpos[i] >= 0 ? (fl[i] | DML_FL_REF) : (fl[i] & ~DML_FL_REF));
+    HIPCHECK(hipMemcpy(c->d.flags + o, fl.data(), n, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(c->d.ref_order + o, g.data(), sizeof(int32_t) * nref, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(c->d.ref_pos + o, rpos.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
+  }
+  if (bkey) {
+    HIPCHECK(hipMemcpy(c->d.bkey + o, bkey, sizeof(int32_t) * n, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(c->d.b2slot + o, b2s.data(), sizeof(int32_t) * p.pcap, hipMemcpyHostToDevice));
+  }
   p.ovn_stamp = 0;  // another set of ref atoms: no lists for the new ones
   p.fo_n = 0;
+  c->reps[rep].p = p;
   return upload_params(c);
 }
 
@@ -1475,20 +1488,20 @@ int dml_set_box(dml_ctx *c, int32_t rep, const double box[3]) {
     else if (box[k] > DML_MAX_BOX) return DML_E_UNSUPPORTED;
   int rc = fetch_params(c);
   if (rc) return rc;
-  RepParams &p = c->reps[rep].p;
+  RepParams p = c->reps[rep].p;
   for (int k = 0; k < 3; k++) {
     p.box[k] = box[k];
     p.one_box[k] = 1.0 / box[k];
   }
   p.ovn_stamp = 0;  // distances change with the box
-  int oldcap = p.ccap;
   if ((rc = tessellate(p, 0))) return rc;
-  int nb = bucket_cap(p);
-  if (ncells_total(p) > oldcap || nb > p.bcap) {
-    p.bcap = std::max(p.bcap, nb);
-    if ((rc = alloc_cells(c))) return rc;
-  } else {
-    p.ccap = oldcap;
+  const int nb = bucket_cap(p);
+  const bool grow = ncells_total(p) > p.ccap || nb > p.bcap;
+  if (grow) p.bcap = std::max(p.bcap, nb);
+  std::swap(c->reps[rep].p, p);
+  if (grow && (rc = alloc_cells(c))) {
+    c->reps[rep].p = p;
+    return rc;
   }
   // (a captured step is taken again when a buffer it holds has moved)
   return upload_params(c);
@@ -1718,22 +1731,43 @@ int dml_set_chunk(dml_ctx *c, int32_t rep, int32_t n, const double *pos, double 
   int rc = fetch_params(c);
   if (rc) return rc;
   HostRep &h = c->reps[rep];
-  RepParams &p = h.p;
+  RepParams p = h.p;
   if (p.reservoir != DML_CHUNKS) return DML_E_STATE;
   // config_chunk (dana.F90:552-587): the template at zmax + z, its pos_old
   // another zmax higher
-  h.chunk.assign(6 * (size_t)n, 0.0);
+  std::vector<double> chunk(6 * (size_t)n);
   for (int j = 0; j < n; j++) {
     for (int k = 0; k < 3; k++) {
-      h.chunk[(size_t)k * n + j] = pos[(int64_t)k * n + j];
-      h.chunk[(size_t)(3 + k) * n + j] = pos[(int64_t)k * n + j];
+      chunk[(size_t)k * n + j] = pos[(int64_t)k * n + j];
+      chunk[(size_t)(3 + k) * n + j] = pos[(int64_t)k * n + j];
     }
-    h.chunk[(size_t)2 * n + j] = h.chunk[(size_t)2 * n + j] + p.zmax;
-    h.chunk[(size_t)5 * n + j] = h.chunk[(size_t)2 * n + j] + p.zmax;
+    chunk[(size_t)2 * n + j] = chunk[(size_t)2 * n + j] + p.zmax;
+    chunk[(size_t)5 * n + j] = chunk[(size_t)2 * n + j] + p.zmax;
   }
+  // the device pool: templates appended, the pool doubled when full
+  double **arr[6] = {&c->d.chx, &c->d.chy, &c->d.chz, &c->d.chox, &c->d.choy, &c->d.choz};
+  if (c->chunk_used + n > c->chunk_cap) {
+    int64_t cap = std::max<int64_t>(2 * c->chunk_cap, c->chunk_used + n);
+    for (auto a : arr) {
+      double *q = nullptr;
+      if (dalloc(&q, cap)) return DML_E_NOMEM;
+      if (*a && c->chunk_used)
+        HIPCHECK(hipMemcpy(q, *a, sizeof(double) * c->chunk_used, hipMemcpyDeviceToDevice));
+      hipFree(*a);
+      *a = q;
+    }
+    c->chunk_cap = cap;
+  }
+  for (int k = 0; k < 6 && n > 0; k++)
+    HIPCHECK(hipMemcpy(*arr[k] + c->chunk_used, chunk.data() + (size_t)k * n, sizeof(double) * n,
+                       hipMemcpyHostToDevice));
+  p.chunk_off = c->chunk_used;
+  c->chunk_used += n;
   p.nchunk = n;
   p.dist = dist;
   p.z1 = z1;
+  h.p = p;
+  h.chunk.swap(chunk);
   // cell memory for the tallest box the slots allow: each block adds dist
   if (n > 0) {
     int64_t blocks = std::max<int64_t>(0, (p.pcap - p.nslots) / n);
@@ -1752,25 +1786,6 @@ int dml_set_chunk(dml_ctx *c, int32_t rep, int32_t n, const double *pos, double 
       }
     }
   }
-  // the device pool: templates appended, the pool doubled when full
-  double **arr[6] = {&c->d.chx, &c->d.chy, &c->d.chz, &c->d.chox, &c->d.choy, &c->d.choz};
-  if (c->chunk_used + n > c->chunk_cap) {
-    int64_t cap = std::max<int64_t>(2 * c->chunk_cap, c->chunk_used + n);
-    for (auto a : arr) {
-      double *q = nullptr;
-      if (dalloc(&q, cap)) return DML_E_NOMEM;
-      if (*a && c->chunk_used)
-        HIPCHECK(hipMemcpy(q, *a, sizeof(double) * c->chunk_used, hipMemcpyDeviceToDevice));
-      hipFree(*a);
-      *a = q;
-    }
-    c->chunk_cap = cap;
-  }
-  p.chunk_off = c->chunk_used;
-  c->chunk_used += n;
-  for (int k = 0; k < 6 && n > 0; k++)
-    HIPCHECK(hipMemcpy(*arr[k] + p.chunk_off, h.chunk.data() + (size_t)k * n, sizeof(double) * n,
-                       hipMemcpyHostToDevice));
   refresh_modes(c);
   return upload_params(c);
 }
@@ -2187,9 +2202,7 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   p.nslots = 0;
   p.nref = 0;
   p.halted = HALT_PAUSED;  // until dml_set_state
-  h.cfg = g;
-  h.p = p;
-  if ((rc = ensure_exact(c))) return rc;
+  if ((rc = ensure_exact(c, p.overlap_mode))) return rc;
   if (rows_for(g) > c->d.maxnn) {
     // wider rows than the context has: grow them (keeps every row)
     int nm = next_pow2(rows_for(g));
@@ -2203,6 +2216,8 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
     c->d.nbr = nbr2;
     c->d.maxnn = nm;
   }
+  h.cfg = g;
+  h.p = p;
   hipMemsetAsync(c->d.cell_cnt + p.coff, 0, sizeof(int32_t) * p.ccap, c->st);
   hipMemsetAsync(c->d.cnt + (int64_t)rep * c->d.ncsh, 0, sizeof(DevCounters) * c->d.ncsh, c->st);
   hipMemsetAsync(c->d.ov_near + p.poff, 0xff, (size_t)p.pcap, c->st);

@@ -1,0 +1,113 @@
+"""Checks of the host side that need the CPU build of libdml: its hipMalloc
+fails on request.  Run by test_simt_host.py in a process of its own."""
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def _fail_malloc(dml, k):
+    """the k-th hipMalloc from now fails (0: none)"""
+    ctypes.c_int.in_dll(dml.lib(), "simt_fail_malloc").value = k
+
+
+def _left(dml):
+    return ctypes.c_int.in_dll(dml.lib(), "simt_fail_malloc").value
+
+
+def _chunks(dml, zmax=60.0, overlap=None):
+    box = [40.0, 40.0, zmax]
+    return dml.dana_config(box, 2.0, 256, z0=30.0, zmax=zmax, integrator=dml.BROWNIAN,
+                           reservoir=dml.CHUNKS, seed=5,
+                           overlap_mode=dml.OVERLAP_ROUNDS if overlap is None else overlap)
+
+
+def _system(dml):
+    rng = np.random.default_rng(3)
+    c = dml.Context(_chunks(dml))
+    block = rng.random((20, 3)) * [40.0, 40.0, 9.0]
+    c.set_chunk(block, 9.0 + 3.2, 55.0)
+    c.set_state(rng.random((60, 3)) * [39.0, 39.0, 58.0] + 0.5, species=np.ones(60, np.int8))
+    c.test_update()
+    return c
+
+
+def _fail(dml, c, call):
+    rng = np.random.default_rng(4)
+    k = 0
+    while True:  # each allocation of the call in turn
+        k += 1
+        _fail_malloc(dml, k)
+        try:
+            if call == "chunk":
+                c.set_chunk(rng.random((50, 3)) * 9.0, 30.0, 40.0)
+            elif call == "exact":
+                c.reconfigure(_chunks(dml, 50.0, dml.OVERLAP_EXACT), 0)
+            else:  # wider rows
+                g = _chunks(dml, 50.0)
+                g.max_neighbors = 4096
+                c.reconfigure(g, 0)
+        except dml.DmlError as e:
+            assert e.status == -3
+            continue
+        finally:
+            left = _left(dml)
+            _fail_malloc(dml, 0)
+        assert left > 0  # the call allocates k - 1 times
+        return k - 1
+
+
+@pytest.mark.parametrize("call", ["chunk", "exact", "rows"])
+def test_out_of_memory_changes_nothing(dml, call):
+    n = _fail(dml, _system(dml), call)
+    assert n > 0
+    for k in sorted({1, n}):
+        a, b = _system(dml), _system(dml)
+        _fail_malloc(dml, k)
+        with pytest.raises(dml.DmlError):
+            if call == "chunk":
+                a.set_chunk(np.random.default_rng(4).random((50, 3)) * 9.0, 30.0, 40.0)
+            else:
+                g = _chunks(dml, 50.0, dml.OVERLAP_EXACT if call == "exact" else None)
+                if call == "rows":
+                    g.max_neighbors = 4096
+                a.reconfigure(g, 0)
+        _fail_malloc(dml, 0)
+        for c in (a, b):
+            c.set_zmax(58.0, 30.0)
+            c.update()
+            c.bloques()
+        np.testing.assert_array_equal(a.calc_rho(), b.calc_rho())
+        sa, sb = a.state(), b.state()
+        for q in sa:
+            np.testing.assert_array_equal(sa[q], sb[q], err_msg="%s %d %s" % (call, k, q))
+        a.close()
+        b.close()
+
+
+def test_out_of_memory_box_can_be_set_again(dml):
+    """no memory for the cells of a taller box: the old box stays, and the call
+    can be made again"""
+    rng = np.random.default_rng(6)
+    pos = rng.random((60, 3)) * [39.0, 39.0, 58.0] + 0.5
+    out = []
+    for k in (0, 1, 9):
+        c = dml.Context(dml.dana_config([40.0, 40.0, 60.0], 2.0, 256, z0=30.0, zmax=60.0,
+                                        integrator=dml.BROWNIAN, reservoir=dml.PISTON, seed=5))
+        c.set_state(pos, species=np.ones(60, np.int8))
+        c.test_update()
+        if k:
+            _fail_malloc(dml, k)
+            with pytest.raises(dml.DmlError):
+                c.set_box([40.0, 40.0, 200.0])
+            _fail_malloc(dml, 0)
+            c.set_zmax(60.0, 30.0)
+            c.update()
+            assert c.cells()[0][2] == 11  # int(60 / 5.2)
+        c.set_box([40.0, 40.0, 200.0])
+        c.update()
+        assert c.cells()[0][2] == 38
+        out.append(c.lists())
+        for x, y in zip(out[0], out[-1]):
+            np.testing.assert_array_equal(x, y)
+        c.close()

@@ -328,7 +328,14 @@ sim_tidx sim_thread_idx() { return sim_tidx{sim::g_cur ? sim::g_cur->tid : 0u, 0
 
 extern "C" long long simt_inactive_reads() { return sim::g_diag_inactive; }
 
+// the simt_fail_malloc-th allocation from now fails (0: none)
+extern "C" int simt_fail_malloc;
+int simt_fail_malloc = 0;
 hipError_t hipMalloc(void **p, size_t n) {
+  if (simt_fail_malloc > 0 && --simt_fail_malloc == 0) {
+    *p = nullptr;
+    return hipErrorOutOfMemory;
+  }
   *p = malloc(n ? n : 1);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -1,0 +1,37 @@
+"""Tests of the host side and of the launch-shape edges on the CPU, against the
+SIMT build of the same sources under AddressSanitizer (see test_simt.py)."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def simt():
+    if not shutil.which("g++"):
+        pytest.skip("g++ not available")
+    sys.path.insert(0, os.path.join(HERE, "simt"))
+    import sim
+    sim.build(asan=True)
+    return sim
+
+
+def _run(sim, name, order="forward", **env):
+    e = sim.env(asan=True)
+    e.update(DML_SIMT="1", SIMT_ORDER=order, **env)
+    r = subprocess.run([sys.executable, "-u", "-m", "pytest", os.path.join(HERE, name), "-q", "-x",
+                        "-s", "-p", "no:cacheprovider"],
+                       env=e, cwd=ROOT, capture_output=True, text=True, timeout=1200)
+    tail = (r.stdout + r.stderr)[-4000:]
+    assert r.returncode == 0, tail
+    assert "AddressSanitizer" not in r.stdout + r.stderr, tail
+
+
+@pytest.mark.parametrize("name", ["test_refused_calls.py", os.path.join("simt", "host_checks.py")])
+def test_host_side(simt, name):
+    _run(simt, name)
