@@ -2177,7 +2177,8 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   if (g.capacity <= 0 || g.box[0] <= 0 || g.box[1] <= 0 || g.box[2] <= 0 || g.rcut <= 0 ||
       g.nadj < 0 || g.nadj > (1 << 21))
     return DML_E_ARG;
-  int rc = fetch_params(c);
+  // the cell region that the new box is checked against is the one in place
+  int rc = c->cells_dirty ? ensure_cells(c) : fetch_params(c);
   if (rc) return rc;
   HostRep &h = c->reps[rep];
   if (round_up(g.capacity, DML_BLOCK) > h.p.pcap) return DML_E_NOMEM;

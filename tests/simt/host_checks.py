@@ -111,3 +111,23 @@ def test_out_of_memory_box_can_be_set_again(dml):
         for x, y in zip(out[0], out[-1]):
             np.testing.assert_array_equal(x, y)
         c.close()
+
+
+def test_reconfigure_before_the_larger_cells_are_there(dml):
+    """dml_set_chunk asks for the cells of the tallest box its blocks can make;
+    a box that needs them all, set before any call that sorts cells"""
+    c = dml.Context(_chunks(dml))
+    c.set_chunk(np.random.default_rng(3).random((4, 3)) * [40.0, 40.0, 9.0], 12.2, 55.0)
+    g = dml.dana_config([40.0, 40.0, 700.0], 2.0, 256, z0=30.0, zmax=700.0,
+                        integrator=dml.BROWNIAN, reservoir=dml.NO_RESERVOIR)
+    c.reconfigure(g, 0)
+    pos = np.random.default_rng(6).random((60, 3)) * [39.0, 39.0, 690.0] + 0.5
+    c.set_state(pos, species=np.ones(60, np.int8))
+    c.test_update()
+    fresh = dml.Context(g)
+    fresh.set_state(pos, species=np.ones(60, np.int8))
+    fresh.test_update()
+    for x, y in zip(c.lists(), fresh.lists()):
+        np.testing.assert_array_equal(x, y)
+    c.close()
+    fresh.close()
