@@ -2189,6 +2189,7 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   // keep the slot range, the reserved cell regions and the trial pool
   p.gb_off = h.p.gb_off;
   p.gb_cap = h.p.gb_cap;
+  p.gb_stamp = h.p.gb_stamp;
   p.poff = h.p.poff;
   p.coff = h.p.coff;
   p.boff = h.p.boff;

@@ -135,7 +135,10 @@ struct RepParams {
   int32_t gb_ilen, gb_glen, gb_rlen, gb_nslots, gb_bamax;
   int32_t gb_nF, gb_nFB;   // free slots below nslots / free hs%b indices below b_amax
   int32_t gb_nins, gb_ndel, gb_nalist;
-  uint32_t gb_stamp;       // gcmc_calls + 1 of this call (stamped per-cell / per-slot marks)
+  // stamp of this call in the per-cell and per-slot marks.  It counts on when
+  // the replica is given another state or configuration: the marks of the calls
+  // before are still there
+  uint32_t gb_stamp;
   double gb_act;
   int32_t fo_n;  // entries of the force kernel's list in cell order (0: ref order)
 };

@@ -4323,7 +4323,7 @@ __global__ void k_gb_begin(DevState s, int rep_only, double act_in, int nadj_in)
   P.gb_bamax = P.b_amax;
   P.gb_nF = P.gb_nFB = 0;
   P.gb_nins = P.gb_ndel = P.gb_nalist = 0;
-  P.gb_stamp = (uint32_t)P.gcmc_calls + 1u;
+  P.gb_stamp += 1u;
   const bool ok = P.use_cells && P.listed && nadj > 0 && nadj <= P.gb_cap &&
                   (int64_t)P.gc_inv + nadj <= (int64_t)GB_VWORDS * 32 && P.gc_len >= nadj + 2;
   P.gb_state = ok ? GB_ON : GB_FALLBACK;

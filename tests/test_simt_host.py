@@ -32,6 +32,7 @@ def _run(sim, name, order="forward", **env):
     assert "AddressSanitizer" not in r.stdout + r.stderr, tail
 
 
-@pytest.mark.parametrize("name", ["test_refused_calls.py", os.path.join("simt", "host_checks.py")])
+@pytest.mark.parametrize("name", ["test_refused_calls.py", "test_gcmc_reuse.py",
+                                  os.path.join("simt", "host_checks.py")])
 def test_host_side(simt, name):
     _run(simt, name)
