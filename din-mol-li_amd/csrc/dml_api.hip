@@ -103,6 +103,7 @@ struct dml_ctx {
   int64_t cap_cm = 0, cap_tm = 0, cap_wm = 0;
   int64_t graph_modes = -1;  // mode signature the captured step was built for
   uint64_t graph_dsig = 0;   // device-state bytes the captured step was built with
+  uint64_t graph_gb = 0;     // replicas whose trials it runs as batches
   int64_t gb_total = 0;      // batched-GCMC trial pool (sum of the replicas' capacities)
   int dev = 0;               // the GPU current at creation
   // the host mirror (reps[].p) holds what the device table does: set by every
@@ -729,13 +730,18 @@ static void enq_gcmc_batch(dml_ctx *c, int r, const double *u, const double *g) 
   hipLaunchKernelGGL(k_gb_cells, dim3(2 * cap), dim3(64), 0, st, d, r);
 }
 
+// a replica whose trials run as batches: it has a pool of them and asks for it
+bool gcmc_batched(const RepParams &p) {
+  return p.gb_cap > 0 && (p.gcmc_mode & DML_GCMC_BATCHED) && p.reservoir == DML_GCMC;
+}
+
 static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g, double act,
                      int nadj, int before = 0, int after = 0) {
   c->fresh = 0;
   const int nb = c->d.nblocks;
   const bool small = small_reps(c);
   int batched = 0;
-  for (auto &h : c->reps) batched |= h.p.gcmc_mode & DML_GCMC_BATCHED;
+  for (auto &h : c->reps) batched |= gcmc_batched(h.p);
   for (int stage = 0; stage < 2; stage++) {
     if (stage == 0 && small) {
       enq_step_small(c, before | SM_GC0, rep_only);
@@ -746,9 +752,7 @@ static void enq_gcmc(dml_ctx *c, int rep_only, const double *u, const double *g,
         hipLaunchKernelGGL(k_gb_begin, dim3((c->nrep + 63) / 64), dim3(64), 0, c->st, c->d,
                            rep_only, act, nadj);
       for (int r = 0; r < c->nrep; r++) {
-        const RepParams &p = c->reps[r].p;
-        if ((rep_only < 0 || r == rep_only) && p.gb_cap > 0 && (p.gcmc_mode & DML_GCMC_BATCHED) &&
-            p.reservoir == DML_GCMC)
+        if ((rep_only < 0 || r == rep_only) && gcmc_batched(c->reps[r].p))
           enq_gcmc_batch(c, r, u, g);
       }
       if (rep_only >= 0)
@@ -2026,7 +2030,11 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     const unsigned char *b = (const unsigned char *)&c->d;
     for (size_t q = 0; q < sizeof(DevState); q++) dsig = (dsig ^ b[q]) * 1099511628211ull;
   }
-  if (use_graph && (!c->gexec || c->graph_modes != modes || c->graph_dsig != dsig)) {
+  // and so are the replicas that run batches (enq_gcmc launches by replica)
+  uint64_t gb = 1469598103934665603ull;
+  for (auto &h : c->reps) gb = (gb ^ (uint64_t)gcmc_batched(h.p)) * 1099511628211ull;
+  if (use_graph && (!c->gexec || c->graph_modes != modes || c->graph_dsig != dsig ||
+                    c->graph_gb != gb)) {
     if (c->gexec) {
       hipGraphExecDestroy(c->gexec);
       hipGraphDestroy(c->graph);
@@ -2039,6 +2047,7 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     c->graph_rounds = c->rounds;
     c->graph_modes = modes;
     c->graph_dsig = dsig;
+    c->graph_gb = gb;
   }
   c->fresh = 0;
   HIPCHECK(hipEventRecord(c->e0, c->st));
