@@ -297,7 +297,9 @@ unsigned char *pinned(dml_ctx *c, size_t n) {
   return c->h_pin;
 }
 
-// device staging of at least n bytes (the stream is idle: the old one may go)
+// device staging of at least n bytes (the stream is idle: the old one may go).
+// A block above kStageMost is not kept (TrimStaging)
+constexpr size_t kStageMost = 64u << 20;
 unsigned char *staging(dml_ctx *c, size_t n) {
   if (n > c->d_cap) {
     hipFree(c->d_stage);
@@ -312,6 +314,15 @@ unsigned char *staging(dml_ctx *c, size_t n) {
   }
   return c->d_stage;
 }
+struct TrimStaging {
+  dml_ctx *c;
+  ~TrimStaging() {
+    if (c->d_cap <= kStageMost) return;
+    hipFree(c->d_stage);
+    c->d_stage = nullptr;
+    c->d_cap = 0;
+  }
+};
 
 void assign_list_kernels(dml_ctx *c);
 
@@ -1264,57 +1275,67 @@ int dml_set_state(dml_ctx *c, int32_t rep, int32_t n, const double *pos, const d
   const int64_t o = p.poff;
   // one block of everything that the caller gave or that is listed here, one
   // copy, one kernel (k_load_state) that also resets what a reused replica
-  // still holds: 15 copies and 12 fills of ~10 us each before.  Layout: pos
-  // and the given of vel, acel, pos_old, old_cg (24 n each); ref_pos, ref_order,
-  // gc_order (4 n each); species, flags (n each)
-  const size_t m = (size_t)n;
+  // still holds: 15 copies and 12 fills of ~10 us each before.  Layout, of m
+  // atoms: pos and the given of vel, acel, pos_old, old_cg (24 m each);
+  // ref_pos, ref_order, gc_order (4 m each); species, flags (m each).  A large
+  // state goes in pieces of kStageMost, a nearly full device takes smaller ones
   const double *given[5] = {pos, vel, acel, pos_old, old_cg};
   int have = 0;
-  size_t bytes = 0;
+  size_t each = 14;
   for (int k = 0; k < 5; k++)
     if (given[k]) {
       have |= 1 << k;
-      bytes += 24 * m;
+      each += 24;
     }
-  const size_t ints = bytes;
-  bytes += 12 * m + 2 * m;
-  unsigned char *dev = staging(c, std::max<size_t>(bytes, 16));
+  int piece = (int)std::min<size_t>((size_t)n, kStageMost / each);
+  unsigned char *dev = staging(c, std::max<size_t>(each * piece, 16));
+  while (!dev && piece > 4096) {
+    piece /= 2;
+    dev = staging(c, each * piece);
+  }
   if (!dev) return DML_E_NOMEM;
   std::vector<unsigned char> big;
-  unsigned char *h = pinned(c, bytes);
+  unsigned char *h = pinned(c, each * piece);
   if (!h) {
-    big.resize(bytes + 1);
+    big.resize(each * piece + 1);
     h = big.data();
   }
-  {
+  int nref = 0, ngc = 0, nat = 0, k0 = 0;
+  do {
+    const int m = std::min(n - k0, piece), last = k0 + m == n;
     size_t at = 0;
     for (int k = 0; k < 5; k++)
-      if (given[k]) {
-        memcpy(h + at, given[k], 24 * m);
-        at += 24 * m;
+      if (given[k])
+        for (int x = 0; x < 3; x++, at += 8 * (size_t)m)
+          memcpy(h + at, given[k] + (int64_t)x * n + k0, 8 * (size_t)m);
+    int32_t *rpos = (int32_t *)(h + at), *rord = rpos + m, *gco = rord + m;
+    int8_t *sp = (int8_t *)(gco + m);
+    uint8_t *fl = (uint8_t *)(sp + m);
+    const int nref0 = nref, ngc0 = ngc;
+    for (int q = 0; q < m; q++) {
+      const int i = k0 + q;
+      sp[q] = species ? species[i] : (int8_t)SP_LI;
+      fl[q] = flags ? flags[i]
+                    : (uint8_t)(DML_FL_ALIVE | (sp[q] != SP_CG ? DML_FL_REF : 0) |
+                                ((p.reservoir == DML_GCMC && sp[q] == SP_LI) ? DML_FL_GCMC : 0));
+      rpos[q] = -1;
+      if (fl[q] & DML_FL_REF) {
+        rpos[q] = nref;
+        rord[nref++ - nref0] = (int32_t)(o + i);
       }
-  }
-  int32_t *rpos = (int32_t *)(h + ints), *rord = rpos + m, *gco = rord + m;
-  int8_t *sp = (int8_t *)(gco + m);
-  uint8_t *fl = (uint8_t *)(sp + m);
-  int nref = 0, ngc = 0, nat = 0;
-  for (int i = 0; i < n; i++) {
-    sp[i] = species ? species[i] : (int8_t)SP_LI;
-    fl[i] = flags ? flags[i]
-                  : (uint8_t)(DML_FL_ALIVE | (sp[i] != SP_CG ? DML_FL_REF : 0) |
-                              ((p.reservoir == DML_GCMC && sp[i] == SP_LI) ? DML_FL_GCMC : 0));
-    rpos[i] = -1;
-    if (fl[i] & DML_FL_REF) {
-      rpos[i] = nref;
-      rord[nref++] = (int32_t)(o + i);
+      // the gcmc group in sys order (dana.F90:505-513)
+      if (fl[q] & DML_FL_GCMC) gco[ngc++ - ngc0] = (int32_t)(o + i);
+      nat += fl[q] & DML_FL_ALIVE;
     }
-    // the gcmc group in sys order (dana.F90:505-513)
-    if (fl[i] & DML_FL_GCMC) gco[ngc++] = (int32_t)(o + i);
-    nat += fl[i] & DML_FL_ALIVE;
-  }
-  if (n > 0) HIPCHECK(hipMemcpyAsync(dev, h, bytes, hipMemcpyHostToDevice, c->st));
-  hipLaunchKernelGGL(k_load_state, dim3((unsigned)(p.pcap / DML_BLOCK)), dim3(DML_BLOCK), 0, c->st,
-                     c->d, p.poff, n, nref, ngc, have, (const unsigned char *)dev);
+    if (m > 0)
+      HIPCHECK(hipMemcpyAsync(dev, h, each * (size_t)m, hipMemcpyHostToDevice, c->st));
+    const int slots = last ? p.pcap - k0 : m;  // the last one empties the rest
+    hipLaunchKernelGGL(k_load_state, dim3((unsigned)((slots + DML_BLOCK - 1) / DML_BLOCK)),
+                       dim3(DML_BLOCK), 0, c->st, c->d, p.poff, k0, slots, m, nref0, nref - nref0,
+                       ngc0, ngc - ngc0, have, (const unsigned char *)dev);
+    if (!last) HIPCHECK(hipStreamSynchronize(c->st));  // the block is filled again
+    k0 += m;
+  } while (k0 < n);
   p.ov_round = 0;
   p.ov_pending = 0;
   p.rho_count = 0;
@@ -1423,7 +1444,7 @@ int dml_get_state(dml_ctx *c, int32_t rep, int32_t n, double *pos, double *vel, 
   }
   // the asked-for arrays packed by one kernel; in one copy through pinned
   // memory when they are small (a copy per component, 21 of ~10 us, before), in
-  // one copy an array otherwise
+  // one copy an array otherwise; without a block for them, a copy per component
   void *dst[9] = {pos, vel, acel, force, pos_old, old_cg, epot, species, flags};
   const size_t m = (size_t)n, size[9] = {24 * m, 24 * m, 24 * m, 24 * m, 24 * m, 24 * m,
                                          8 * m,  m,      m};
@@ -1436,8 +1457,20 @@ int dml_get_state(dml_ctx *c, int32_t rep, int32_t n, double *pos, double *vel, 
     }
   HIPCHECK(hipStreamSynchronize(c->st));
   if (!want) return DML_OK;
-  unsigned char *dev = staging(c, bytes);
-  if (!dev) return DML_E_NOMEM;
+  unsigned char *dev = bytes <= kStageMost ? staging(c, bytes) : nullptr;
+  if (!dev) {
+    const DevState &d = c->d;
+    const int64_t o = p.poff;
+    const double *src[6][3] = {{d.px, d.py, d.pz}, {d.vx, d.vy, d.vz}, {d.ax, d.ay, d.az},
+                               {d.fx, d.fy, d.fz}, {d.ox, d.oy, d.oz}, {d.cx, d.cy, d.cz}};
+    for (int k = 0; k < 6; k++)
+      for (int x = 0; x < 3 && dst[k]; x++)
+        HIPCHECK(hipMemcpy((double *)dst[k] + x * m, src[k][x] + o, 8 * m, hipMemcpyDeviceToHost));
+    if (epot) HIPCHECK(hipMemcpy(epot, d.epot + o, 8 * m, hipMemcpyDeviceToHost));
+    if (species) HIPCHECK(hipMemcpy(species, d.species + o, m, hipMemcpyDeviceToHost));
+    if (flags) HIPCHECK(hipMemcpy(flags, d.flags + o, m, hipMemcpyDeviceToHost));
+    return DML_OK;
+  }
   hipLaunchKernelGGL(k_pack_state, dim3((unsigned)((n + DML_BLOCK - 1) / DML_BLOCK)),
                      dim3(DML_BLOCK), 0, c->st, c->d, p.poff, n, want, dev);
   unsigned char *h = pinned(c, bytes);
@@ -1918,6 +1951,7 @@ int dml_gcmc_trial_energy(dml_ctx *c, int32_t rep, int32_t ntrial, const double 
   // trials 490
   const size_t n = (size_t)ntrial, np = pos3 ? 24 * n : 0, nx = exclude ? 4 * n : 0;
   const size_t up = np + nx, off = (up + 15) / 16 * 16, down = 12 * n;
+  TrimStaging trim{c};
   unsigned char *d = staging(c, off + down);
   if (!d) return DML_E_NOMEM;
   std::vector<unsigned char> big;

@@ -4,8 +4,8 @@
 
 __global__ void k_pbc_dispmax(DevState s);
 __global__ void k_dispmax_final(DevState s, int begin);
-__global__ void k_load_state(DevState s, int poff, int n, int nref, int ngc, int have,
-                             const unsigned char *in);
+__global__ void k_load_state(DevState s, int poff, int k0, int slots, int n, int nref0, int nref,
+                             int ngc0, int ngc, int have, const unsigned char *in);
 __global__ void k_pack_state(DevState s, int poff, int n, int want, unsigned char *out);
 __global__ void k_force_rebuild(DevState s);
 __global__ void k_force_order(DevState s);

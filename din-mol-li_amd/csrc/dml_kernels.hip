@@ -2748,13 +2748,17 @@ __global__ void k_ov_end(DevState s, int rounds) {
 
 // dml_set_state: n atoms from one block (pos, then the given of vel, acel,
 // pos_old, old_cg: bits 0-4 of `have`, 3 n doubles each; ref_pos, ref_order,
-// gc_order; species; flags) into the replica at poff, with the defaults of
-// atom_allocate / config_inic, and the slots beyond n emptied
-__global__ void __launch_bounds__(DML_BLOCK) k_load_state(DevState s, int poff, int n, int nref,
+// gc_order; species; flags) into the slots k0 on of the replica at poff, with
+// the defaults of atom_allocate / config_inic, and of `slots` slots those
+// beyond n emptied.  The block's nref ref and ngc gcmc atoms are the lists'
+// entries nref0 and ngc0 on
+__global__ void __launch_bounds__(DML_BLOCK) k_load_state(DevState s, int poff, int k0, int slots,
+                                                          int n, int nref0, int nref, int ngc0,
                                                           int ngc, int have,
                                                           const unsigned char *in) {
-  const int k = blockIdx.x * DML_BLOCK + threadIdx.x;  // (a block per 256 slots of the replica)
-  const int i = poff + k;
+  const int k = blockIdx.x * DML_BLOCK + threadIdx.x;
+  if (k >= slots) return;
+  const int i = poff + k0 + k;
   s.nn[i] = 0;
   s.ovq[0][i] = s.ovq[1][i] = 0;
   s.rowflag[i] = 0;
@@ -2793,13 +2797,13 @@ __global__ void __launch_bounds__(DML_BLOCK) k_load_state(DevState s, int poff, 
   s.cx[i] = cx; s.cy[i] = cy; s.cz[i] = cz;
   s.species[i] = sp[k];
   s.flags[i] = fl;
-  s.bkey[i] = k;
-  s.pid[i] = (uint32_t)k;
-  s.seq[i] = k;
+  s.bkey[i] = k0 + k;
+  s.pid[i] = (uint32_t)(k0 + k);
+  s.seq[i] = k0 + k;
   s.b2slot[i] = (fl & DML_FL_ALIVE) ? i : -1;
   s.ref_pos[i] = q[k];
-  if (k < nref) s.ref_order[i] = q[n + k];
-  if (k < ngc) s.gc_order[i] = q[2 * (int64_t)n + k];
+  if (k < nref) s.ref_order[poff + nref0 + k] = q[n + k];
+  if (k < ngc) s.gc_order[poff + ngc0 + k] = q[2 * (int64_t)n + k];
   put_pf4(s, i, x, y, z, sp[k]);
 }
 

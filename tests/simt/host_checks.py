@@ -131,3 +131,19 @@ def test_reconfigure_before_the_larger_cells_are_there(dml):
         np.testing.assert_array_equal(x, y)
     c.close()
     fresh.close()
+
+
+def test_state_is_read_without_memory_to_stage_it(dml):
+    c = dml.Context(dml.dana_config([40.0, 40.0, 60.0], 2.0, 4096, z0=30.0))
+    pos = np.random.default_rng(8).random((4096, 3)) * 39.0
+    c.set_state(pos)  # 38 bytes an atom staged, 170 to read it back
+    _fail_malloc(dml, 1)
+    got = c.state()
+    assert _left(dml) == 0  # an allocation was asked for and refused
+    np.testing.assert_array_equal(got["pos"], pos)
+    np.testing.assert_array_equal(got["pos_old"], pos)
+    np.testing.assert_array_equal(got["vel"], np.zeros((4096, 3)))
+    np.testing.assert_array_equal(got["old_cg"], np.full((4096, 3), 1e8))
+    np.testing.assert_array_equal(got["species"], np.ones(4096, np.int8))
+    np.testing.assert_array_equal(got["flags"], np.full(4096, dml.FL_ALIVE | dml.FL_REF))
+    c.close()
