@@ -343,7 +343,7 @@ struct DevState {
   double *chox, *choy, *choz;
   // flat work lists (rebuilt by the host when the layout changes)
   int32_t *cm_rep, *cm_cell; // every reserved cell of every replica
-  int32_t *cm_nref;          // its ref atoms, where the row build has to do it
+  int32_t *cm_nref;          // its ref atoms and first entries, where the row build has to do it
   int32_t *tm_rep, *tm_cell; // cells of the replicas built by cell tiles
   int32_t *wm_blk;           // particle blocks of the replicas built wave per atom
   int64_t n_cm, n_tm, n_wm;

@@ -1003,6 +1003,14 @@ k_listbuild_wc(DevState s) {
   }
 }
 
+// a cell's word in cm_nref: its ref atoms (25 bits) and, of its entries, how
+// many a wave loads at once (up to 64)
+__device__ inline int cm_pack(int refs, int cnt) {
+  return (int)((uint32_t)refs | (uint32_t)min(cnt, WAVE) << 25);
+}
+__device__ inline int cm_refs(int v) { return v & 0x1ffffff; }
+__device__ inline int cm_first(int v) { return (int)((uint32_t)v >> 25); }
+
 // ------------------------------------------------------------------------
 // Rows of a centre cell with its candidates held in registers: a wave loads
 // up to NCH chunks of 64 candidates of the 27-cell stream at a time, then
@@ -1019,9 +1027,13 @@ k_listbuild_wc(DevState s) {
 // while an XCD's L2 still holds the candidates of neighbouring cells; inside an XCD
 // its nwx waves take the cells one by one in list order.  2^sl waves share a
 // cell (LB_PART ref atoms a wave or more): wave v takes part v % 2^sl of every
-// (nwx >> sl)-th cell.  The cells to do come from cm_nref (ref atoms per cell,
-// by k_cell_sort_w; 0 for a cell that is not rebuilt), 64 per load, so an
-// empty cell costs a lane of one load.
+// (nwx >> sl)-th cell.  The cells to do come from cm_nref (ref atoms and first
+// entries per cell, by k_cell_sort_w; 0 for a cell that is not rebuilt), 64 per
+// load, so an empty cell costs a lane of one load, and the centre atoms are
+// loaded beside the stencil's counts without a read past the cell's own (with
+// all 64 lanes reading, 256 dense replicas rebuilt at once took 2.34 ms, now
+// 2.06; with cells in contiguous runs per wave 1.90, but the step, which
+// rebuilds some of them, 6.3 ms against 6.05).
 //
 // What bounds it: instruction issue (about 30 instructions a chunk of 64 pair
 // tests) with the wait for a pass's candidates behind it.  Before, each wave
@@ -1081,13 +1093,14 @@ k_listbuild_wr(DevState s, int sl) {
       }
     }
     // a cell of few ref atoms is not split into all the parts
-    unsigned long long work = __ballot(ln > part * LB_PART);
+    unsigned long long work = __ballot(cm_refs(ln) > part * LB_PART);
     while (work) {
       const int q = __builtin_ctzll(work);
       work &= work - 1;
       const int r = __builtin_amdgcn_readlane(lr, q);
       const int c = __builtin_amdgcn_readlane(lc, q);
-      const int nrefc = __builtin_amdgcn_readlane(ln, q);
+      const int lnq = __builtin_amdgcn_readlane(ln, q);
+      const int nrefc = cm_refs(lnq), first = cm_first(lnq);
       const int parts = min(1 << sl, (nrefc + LB_PART - 1) / LB_PART);
       const RepParams &P = s.rp[r];
       if (r != cur_r) {
@@ -1130,12 +1143,11 @@ k_listbuild_wr(DevState s, int sl) {
       }
       // the image reference point: the midpoint of the centre cell
       const float mxf = ((float)ci0 - 0.5f) * q_cx, myf = ((float)ci1 - 0.5f) * q_cy;
-      // the first 64 centre atoms' entries (entries past the cell's count
-      // are read and dropped: a cell's bucket holds them), loaded with the
-      // stencil counts (one wait for both)
+      // the first 64 centre atoms' entries, loaded with the stencil counts
+      // (one wait for both)
       int cs = -1;
       float4 cf = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (lane < q_bcap) {
+      if (lane < first) {
         cs = s.bucket[cbase + lane];
         cf = s.bf4[cbase + lane];
       }
@@ -1577,7 +1589,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_cell_sort_w(DevState s, int gcs) 
     // ref atoms per cell, for the row build of the replicas that rebuild
     if (lref > 0) {
       const RepParams &Q = s.rp[lr];
-      if (Q.rebuild && Q.lb_kind == 3) s.cm_nref[g0 + lane] = lref;
+      if (Q.rebuild && Q.lb_kind == 3) s.cm_nref[g0 + lane] = cm_pack(lref, lcnt);
     }
   }
 }
@@ -1597,7 +1609,7 @@ __global__ void __launch_bounds__(FO_BLOCK) k_force_order(DevState s) {
   for (int64_t g0 = (int64_t)blockIdx.x * WAVE; g0 < s.n_cm; g0 += (int64_t)gridDim.x * WAVE) {
     int lr = -1, lc = 0, ln = 0;
     if (g0 + lane < s.n_cm) {
-      ln = s.cm_nref[g0 + lane];
+      ln = cm_refs(s.cm_nref[g0 + lane]);
       if (ln > 0) {
         lr = s.cm_rep[g0 + lane];
         lc = s.cm_cell[g0 + lane];
