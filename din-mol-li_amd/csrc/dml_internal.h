@@ -16,7 +16,12 @@
 #include "../../include/dml.h"
 
 #define DML_BLOCK 256
+#ifndef OV_STAMPS
 #define OV_STAMPS 40  // work-list stamps per overlap call (more than its rounds)
+#endif
+// a call that reaches this base clears the stamps at its end, and the next one
+// starts over (after some 54 million calls on one state)
+#define OV_LAST (INT32_MAX - 2 * OV_STAMPS)
 #define OVB_MAX 2048  // list entries a workgroup of an overlap round collects in LDS
 #define OVT_BLOCK 512 // threads of the overlap tail
 #define OVX_MAX 16  // row entries listed per atom for the reference-order overlap pass

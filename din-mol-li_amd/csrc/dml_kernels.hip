@@ -133,7 +133,8 @@ __global__ void __launch_bounds__(DML_BLOCK) k_pbc_dispmax(DevState s) {
 
 // before the first overlap round: stamps past every earlier call's, no round with progress
 __device__ inline void ov_begin_rep(const DevState &s, int r) {
-  s.rp[r].ov_round += OV_STAMPS;
+  const int base = s.rp[r].ov_round;
+  s.rp[r].ov_round = (base >= OV_LAST ? 0 : base) + OV_STAMPS;
   s.ov_last[r] = -1;
 }
 
@@ -2724,7 +2725,10 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ov_finish(DevState s, int rounds)
       if (last == rounds - 1) atomicAdd(&cnt_of(s, r, 0).ov_unfinished, 1ull);
     }
   }
-  if (i - P.poff >= P.nslots) return;
+  const bool in = i - P.poff < P.nslots;
+  const int listed = in ? max(s.ovq[0][i], s.ovq[1][i]) : 0;
+  if (P.ov_round >= OV_LAST) s.ovq[0][i] = s.ovq[1][i] = 0;
+  if (!in) return;
   const int w = __float_as_int(s.pf4[i].w);
   if (OVW_AT(w)) {
     const double x = s.cx[i], y = s.cy[i], z = s.cz[i];
@@ -2737,7 +2741,7 @@ __global__ void __launch_bounds__(DML_BLOCK) k_ov_finish(DevState s, int rounds)
   }
   if (P.halted) return;
   const uint8_t f = s.flags[i];
-  const int at = max(s.ovq[0][i], s.ovq[1][i]) - P.ov_round;  // the last round it was listed for
+  const int at = listed - P.ov_round;  // the last round it was listed for
   uint8_t g = f;
   if (at > 0) {
     // resolved there if that round came to it

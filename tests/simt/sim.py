@@ -12,8 +12,8 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 LIB = os.environ.get("SIMT_LIB") or os.path.join(HERE, "_build", "libdml_sim.so")
 
 
-def build(asan=True):
-    env = dict(os.environ, SIMT_ASAN="1" if asan else "0")
+def build(asan=True, **more):
+    env = dict(os.environ, SIMT_ASAN="1" if asan else "0", **more)
     subprocess.check_call(["bash", os.path.join(HERE, "build.sh")], env=env)
 
 

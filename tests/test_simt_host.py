@@ -36,3 +36,9 @@ def _run(sim, name, order="forward", **env):
                                   os.path.join("simt", "host_checks.py")])
 def test_host_side(simt, name):
     _run(simt, name)
+
+
+def test_overlap_stamps_start_over(simt, tmp_path):
+    lib = str(tmp_path / "libdml_stamps.so")
+    simt.build(asan=True, SIMT_OUT=lib, SIMT_FLAGS="-DOV_STAMPS=0x10000000")
+    _run(simt, os.path.join("simt", "stamp_checks.py"), STAMP_LIB=lib)
