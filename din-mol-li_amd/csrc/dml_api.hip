@@ -111,6 +111,7 @@ struct dml_ctx {
   // may yet refuse or fail leaves the mirror alone: it works on a copy and
   // stores that once nothing can fail but the upload
   int fresh = 0;
+  int pending = 0;           // the stream may hold copies or fills of a setter
   int err_seen = 0;          // error bits of the last fetch
   unsigned char *h_rp = nullptr;    // pinned: the table and the error word
   unsigned char *h_pin = nullptr;   // pinned staging of small transfers, kept
@@ -271,6 +272,7 @@ int take_table(dml_ctx *c) {
   memcpy(&e, c->h_rp + table_bytes(c), sizeof(e));
   c->err_seen = e;
   c->fresh = 1;
+  c->pending = 0;
   return DML_OK;
 }
 
@@ -389,15 +391,23 @@ int upload_params(dml_ctx *c) {
   std::vector<RepParams> v(c->nrep);
   for (int r = 0; r < c->nrep; r++) v[r] = c->reps[r].p;
   c->fresh = 0;
+  c->pending = 1;
   HIPCHECK(hipMemcpyAsync(c->d.rp, v.data(), sizeof(RepParams) * c->nrep, hipMemcpyHostToDevice,
                           c->st));
   c->fresh = 1;
   return DML_OK;
 }
 
-// the mutable device fields are authoritative: fetch them into the mirror
+// the mutable device fields are authoritative: fetch them into the mirror.
+// Afterwards the stream is idle: what a caller reads with a plain copy, which
+// does not wait for it, is there
 int fetch_params(dml_ctx *c) {
-  if (c->fresh) return DML_OK;
+  if (c->fresh && !c->pending) return DML_OK;
+  if (c->fresh) {
+    if (hipStreamSynchronize(c->st) != hipSuccess) return DML_E_HIP;
+    c->pending = 0;
+    return DML_OK;
+  }
   copy_table(c);
   return take_table(c);
 }
@@ -974,6 +984,7 @@ int ensure_exact(dml_ctx *c, int overlap_mode) {
 int read_counters(dml_ctx *c, int rep, DevCounters *out) {
   const int n = c->d.ncsh;
   std::vector<DevCounters> v(n);
+  HIPCHECK(hipStreamSynchronize(c->st));
   HIPCHECK(hipMemcpy(v.data(), c->d.cnt + (int64_t)rep * n, sizeof(DevCounters) * n,
                      hipMemcpyDeviceToHost));
   constexpr int words = sizeof(DevCounters) / sizeof(unsigned long long);

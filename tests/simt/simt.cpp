@@ -314,12 +314,14 @@ static void run_launch(dim3 grid, dim3 block, const std::function<void()> &body)
   g_body = nullptr;
 }
 
+static void (*flush_hook)() = nullptr;  // the stream's fills come before its next launch
 void launch(dim3 grid, dim3 block, void *stream, std::function<void()> body) {
   sim_stream *st = (sim_stream *)stream;
   if (st && st->capturing) {
     st->rec.push_back(Rec{grid, block, std::move(body)});
     return;
   }
+  if (flush_hook) flush_hook();
   run_launch(grid, block, body);
 }
 }  // namespace sim
@@ -339,7 +341,16 @@ hipError_t hipMalloc(void **p, size_t n) {
   *p = malloc(n ? n : 1);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
+// with SIMT_LAZY a stream's fills and uploads happen when its next kernel or a
+// wait comes: a plain copy does not wait for them
+static const bool g_lazy = getenv("SIMT_LAZY") != nullptr;
+static std::vector<std::function<void()>> g_fills;
+static void flush_fills() {
+  for (auto &f : g_fills) f();
+  g_fills.clear();
+}
 hipError_t hipFree(void *p) {
+  flush_fills();
   free(p);
   return hipSuccess;
 }
@@ -352,10 +363,18 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
     fprintf(stderr, "simt: copy recorded into a graph\n");
     abort();
   }
+  if (g_lazy && k == hipMemcpyHostToDevice) {
+    std::vector<char> v((const char *)s, (const char *)s + n);
+    sim::flush_hook = flush_fills;
+    g_fills.push_back([d, v]() { memcpy(d, v.data(), v.size()); });
+    return hipSuccess;
+  }
+  flush_fills();
   return hipMemcpy(d, s, n, k);
 }
 hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h,
                             hipMemcpyKind, hipStream_t) {
+  flush_fills();
   for (size_t r = 0; r < h; r++) memmove((char *)d + r * dp, (const char *)s + r * sp, w);
   return hipSuccess;
 }
@@ -368,6 +387,11 @@ hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) {
     fprintf(stderr, "simt: memset recorded into a graph\n");
     abort();
   }
+  if (g_lazy) {
+    sim::flush_hook = flush_fills;
+    g_fills.push_back([=]() { hipMemset(d, v, n); });
+    return hipSuccess;
+  }
   return hipMemset(d, v, n);
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *st, unsigned) {
@@ -378,8 +402,11 @@ hipError_t hipStreamDestroy(hipStream_t st) {
   delete st;
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  flush_fills();
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipStreamSynchronize(nullptr); }
 hipError_t hipGetLastError() { return hipSuccess; }
 void sincospi(double x, double *s, double *c) {
   *s = sin(M_PI * x);
@@ -411,6 +438,7 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t g, hipGraphNode_t *
   return hipSuccess;
 }
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
+  flush_fills();
   for (auto &r : e->rec) sim::run_launch(r.g, r.b, r.body);
   return hipSuccess;
 }

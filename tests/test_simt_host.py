@@ -42,3 +42,7 @@ def test_overlap_stamps_start_over(simt, tmp_path):
     lib = str(tmp_path / "libdml_stamps.so")
     simt.build(asan=True, SIMT_OUT=lib, SIMT_FLAGS="-DOV_STAMPS=0x10000000")
     _run(simt, os.path.join("simt", "stamp_checks.py"), STAMP_LIB=lib)
+
+
+def test_reads_wait_for_the_stream(simt):
+    _run(simt, os.path.join("simt", "wait_checks.py"), SIMT_LAZY="1")
