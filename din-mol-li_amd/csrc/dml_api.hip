@@ -1005,7 +1005,10 @@ void refresh_modes(dml_ctx *c) {
     if (h.p.reservoir == DML_GCMC) c->any_gcmc = 1;
     if (h.p.reservoir == DML_CHUNKS && h.p.nchunk > 0) c->any_chunks = 1;
     if (h.p.integrator == DML_ERMAK) c->any_ermak = 1; else c->any_brown = 1;
-    if (h.p.overlap_mode == DML_OVERLAP_ROUNDS) c->any_rounds = 1; else c->any_exact = 1;
+    // (the reference-order pass looks at every slot of the context: not for a
+    // replica that sits the run out, such as a free slot of a serving pool)
+    if (h.p.overlap_mode == DML_OVERLAP_ROUNDS) c->any_rounds = 1;
+    else if (!h.p.halted) c->any_exact = 1;
     if (h.p.piston) c->any_piston = 1;
   }
 }
@@ -2055,6 +2058,7 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     if (c->any_ermak) enq_forces(c, 0, 1);
     hipLaunchKernelGGL(k_mask_listed, dim3(rb), dim3(64), 0, c->st, c->d, 0);
     if ((rc = finish(c, 0))) return rc;
+    refresh_modes(c);  // a replica halted by an overflow may run again
   }
   // what the captured step depends on: the phases present and the launch
   // shapes (rounds <= 32, lanes <= 64)

@@ -19,9 +19,12 @@ import numpy as np
 
 from . import Context, dana_config, lib
 
-# bytes per slot held on the device: FP64 state (22 x 8), narrow per-slot
-# arrays (~30), the FP32 mirror (16), plus the neighbour row (4 x maxnn)
-STATE_BYTES_PER_SLOT = 22 * 8 + 30 + 16
+# bytes per slot held on the device: FP64 state (22 x 8), 16 index arrays of 4,
+# 4 of a byte, the list of near entries (16), the FP32 mirror (16) and the
+# reference-order overlap pass's entries (16 x 8, count and masks), which a
+# pool has from the start for requests of that schedule; plus the neighbour
+# row (4 x maxnn)
+STATE_BYTES_PER_SLOT = 22 * 8 + 16 * 4 + 4 + 16 + 16 + 16 * 8 + 2
 
 
 class Request:
