@@ -15,7 +15,6 @@ __global__ void k_ghost_small(DevState s, int only_ermak, int fuse_b);
 __global__ void k_step_small(DevState s, int ops, int rep_only);
 __global__ void k_zero_cells(DevState s, int gcs);
 __global__ void k_cell_key(DevState s, int gcs);
-__global__ void k_cell_sort(DevState s, int gcs);
 __global__ void k_cell_sort_w(DevState s, int gcs);
 __global__ void k_listbuild_cells(DevState s);
 template <int LPA>
@@ -38,7 +37,6 @@ __global__ void k_ov_tail(DevState s, const double *u_round, int64_t u_stride, i
                           int64_t ptotal);
 __global__ void k_ov_finish(DevState s, int rounds);
 __global__ void k_ov_end(DevState s, int rounds);
-__global__ void k_zero_i32(int32_t *a, int64_t n);
 __global__ void k_f2cg_mark(DevState s);
 __global__ void k_f2cg_scan(DevState s);
 __global__ void k_f2cg_scatter(DevState s);

@@ -335,43 +335,6 @@ template __global__ void k_update_small<1>(DevState, int, int, int);
 template __global__ void k_update_small<2>(DevState, int, int, int);
 template __global__ void k_update_small<4>(DevState, int, int, int);
 
-// order each bucket like the head/next chain: descending hs%b slot for
-// cells (push-front, Cells.F90:299-300), ascending for the Verlet scan
-// (Neighbor.F90:397); then copy positions into bucket order.
-__global__ void k_cell_sort(DevState s, int gcs) {
-  int r = blockIdx.y;
-  const RepParams &P = s.rp[r];
-  if (P.halted) return;
-  if (!want_cells(P, gcs)) return;
-  int nc = ncell_total(P);
-  int desc = P.use_cells;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x) {
-    int cnt = s.cell_cnt[P.coff + c];
-    if (cnt > P.bcap) cnt = P.bcap;
-    if (cnt == 0) continue;
-    int64_t base = P.boff + (int64_t)c * P.bcap;
-    int32_t *b = s.bucket + base;
-    for (int q = 1; q < cnt; q++) {
-      int v = b[q], kv = s.bkey[v];
-      int w = q - 1;
-      while (w >= 0) {
-        int kw = s.bkey[b[w]];
-        if (desc ? (kw >= kv) : (kw <= kv)) break;
-        b[w + 1] = b[w];
-        w--;
-      }
-      b[w + 1] = v;
-    }
-    for (int q = 0; q < cnt; q++) {
-      int v = b[q];
-      s.bx[base + q] = s.px[v];
-      s.by[base + q] = s.py[v];
-      s.bz[base + q] = s.pz[v];
-      s.bf4[base + q] = bucket_f4(s, v);
-    }
-  }
-}
-
 // ------------------------------------------------------------------------
 // neighbour rows: ngroup_cells (Neighbor.F90:465-548) -- one wave per ref
 // atom; candidates of the 27 stencil cells in stencil order, then chain
@@ -1410,7 +1373,10 @@ template __global__ void k_listbuild_wr<3, 7>(DevState s, int sl);
 template __global__ void k_listbuild_wr<2, 8>(DevState s, int sl);
 
 
-// bucket order by a rank sort inside one wave (cells of up to 256 atoms,
+// each bucket ordered like the head/next chain: descending hs%b slot for cells
+// (push-front, Cells.F90:299-300), ascending for the Verlet scan
+// (Neighbor.F90:397); positions and flags copied into that order.
+// A rank sort inside one wave (cells of up to 256 atoms,
 // four per lane: electrode cells hold ~100; larger cells fall back to an
 // insertion sort by lane 0)
 #define SORT_W 4
@@ -2855,11 +2821,6 @@ __global__ void __launch_bounds__(DML_BLOCK) k_pack_state(DevState s, int poff, 
     b += n;
   }
   if (want >> 8 & 1) b[k] = s.flags[i];
-}
-
-__global__ void k_zero_i32(int32_t *a, int64_t n) {
-  int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q < n) a[q] = 0;
 }
 
 // exclusive prefix sums of two per-block counters over one replica's
