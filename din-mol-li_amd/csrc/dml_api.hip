@@ -658,12 +658,20 @@ void enq_overlap_rounds(dml_ctx *c, const double *u_round, int64_t stride, int r
     hipLaunchKernelGGL(k_ov_begin, dim3((std::max(c->nrep, 3) + 63) / 64), dim3(64), 0, c->st,
                        c->d);
   // rounds from `tail` on run in one workgroup, one launch (their lists are
-  // short; most of them are empty).  Ermak moves ~0.06 A a step, its lists are
-  // short from round 3 on (100,000 particles: from 3 294 us a step, from 8
-  // 307, from 2 616); Brownian moves ~4 A and its lists shrink slowly (100,000
-  // particles: from 8 608 us, from 6 669; 12,000: from 6 308, from 3 605)
+  // short; most of them are empty).  Us a step with the tail from round 3, 4, 6
+  // and 8 on, ions at 0.01 / A^3 beside an electrode:
+  //   Ermak      12,000 atoms  141  146  151  153    Brownian   2,100  126  127  130  134
+  //              25,000        169  172  177  183              12,000  151  153  156  159
+  //              50,000        229  227  234  238              24,000  219  200  201  205
+  //             100,000        296  291  296  300              33,000  334  261  252  256
+  //             290,000        662  615  620  633              60,000  836  445  314  316
+  //             400,000        880  830  837  839             100,000 2432  959  419  390
+  // Ermak moves ~0.06 A a step, so its lists are short by then; Brownian moves
+  // ~4 A, its lists shrink slowly, and more so in a crowded system (12,000
+  // crowded atoms: from 3 605, from 6 308).  Its lines therefore lie where a
+  // late tail costs a few microseconds, not where an early one first pays
   const int tail = c->ov_tail >= 0  ? c->ov_tail
-                   : !c->any_brown  ? (c->P <= 300000 ? 3 : 4)
+                   : !c->any_brown  ? (c->P < 50000 ? 3 : 4)
                    : c->P <= 2048   ? 3
                    : c->P <= 24576  ? 6
                                     : 8;
