@@ -476,9 +476,12 @@ unsigned clamp_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<
 // below 24,000 ref atoms (4,000 particles 83 -> 31 us, 12,000 59 -> 36), 2
 // below 200,000 (37,000: 92 -> 68, 100,000: 94 -> 79), none above (2M: 835,
 // split 930); sparse cells (a few atoms) are never split (1,505 ions of a
-// chunks run: 10.6, split 12.3).  Dense cells want more workgroups than
-// resident ones to even out the tail (16 dense replicas 141 -> 115 us, 2M 980
-// -> 835), sparse ones the fewest (24 mixed replicas 336 -> 320)
+// chunks run: 10.6, split 12.3).  Workgroups: 7,168, four times the resident
+// ones, even out the tail where there is work for them (us with 1,792 and
+// 7,168: 16 dense replicas 141, 115; 2M dense 980, 835; 8 replicas of 206,000
+// atoms in all 107, 97; 24 of 326,000 218, 184; 400,000 dilute ions 211, 179;
+// 150,000 dilute 75, 75); fewer dilute ions are done sooner by the resident
+// ones alone (60,000: 35, 40; 20,000: 18, 21; a chunks run's step 290, 301)
 void wr_shape(const dml_ctx *c, int *sl, int *g) {
   int64_t nref = 0, cells = 0;
   for (auto &h : c->reps) {
@@ -489,7 +492,8 @@ void wr_shape(const dml_ctx *c, int *sl, int *g) {
   }
   const bool dense = nref >= 4 * cells;
   *sl = !dense || nref >= 200000 ? 0 : nref >= 24000 ? 1 : 2;
-  const int64_t need = ((c->d.n_cm << *sl) + 3) / 4, most = dense ? 7168 : 1792;
+  const int64_t need = ((c->d.n_cm << *sl) + 3) / 4;
+  const int64_t most = dense || nref >= 150000 ? 7168 : 1792;
   *g = (int)(std::min(std::max<int64_t>(need, 8), most) + 7) / 8 * 8;
 }
 
