@@ -1671,6 +1671,11 @@ int dml_forces(dml_ctx *c) {
 int dml_brownian(dml_ctx *c, const double *noise, const double *u_dep) {
   if (!c) return DML_E_ARG;
   double *dn = upload_tmp(c, noise, 3 * c->P), *du = upload_tmp(c, u_dep, c->P);
+  if ((noise && !dn) || (u_dep && !du)) {
+    hipFree(dn);
+    hipFree(du);
+    return DML_E_NOMEM;
+  }
   hipLaunchKernelGGL(k_brownian, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d,
                      (const double *)dn, (const double *)du);
   int rc = finish(c);
@@ -1682,6 +1687,11 @@ int dml_brownian(dml_ctx *c, const double *noise, const double *u_dep) {
 int dml_ermak_a(dml_ctx *c, const double *noise, const double *u_dep) {
   if (!c) return DML_E_ARG;
   double *dn = upload_tmp(c, noise, 6 * c->P), *du = upload_tmp(c, u_dep, c->P);
+  if ((noise && !dn) || (u_dep && !du)) {
+    hipFree(dn);
+    hipFree(du);
+    return DML_E_NOMEM;
+  }
   hipLaunchKernelGGL(k_ermak_a, dim3(c->d.nblocks), dim3(DML_BLOCK), 0, c->st, c->d,
                      (const double *)dn, (const double *)du);
   int rc = finish(c);
@@ -1701,6 +1711,7 @@ int dml_overlap_moveback(dml_ctx *c, const double *u_contact, int64_t n_u, int32
   // n_u uniforms per replica, replica r at [r*n_u, (r+1)*n_u)
   if (u_contact && n_u <= 0) return DML_E_ARG;
   double *du = u_contact ? upload_tmp(c, u_contact, n_u * c->nrep) : nullptr;
+  if (u_contact && !du) return DML_E_NOMEM;
   enq_overlap_exact(c, du, n_u, max_passes > 0 ? max_passes : 100000);
   int rc = finish(c);
   hipFree(du);
@@ -1710,6 +1721,7 @@ int dml_overlap_moveback(dml_ctx *c, const double *u_contact, int64_t n_u, int32
 int dml_overlap_rounds(dml_ctx *c, const double *u_round, int32_t max_rounds) {
   if (!c || max_rounds <= 0 || max_rounds > kMaxRounds) return DML_E_ARG;
   double *du = u_round ? upload_tmp(c, u_round, (int64_t)max_rounds * c->P) : nullptr;
+  if (u_round && !du) return DML_E_NOMEM;
   enq_overlap_rounds(c, du, c->P, max_rounds, 0, 1);
   int rc = finish(c);
   hipFree(du);

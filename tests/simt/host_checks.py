@@ -147,3 +147,28 @@ def test_state_is_read_without_memory_to_stage_it(dml):
     np.testing.assert_array_equal(got["species"], np.ones(4096, np.int8))
     np.testing.assert_array_equal(got["flags"], np.full(4096, dml.FL_ALIVE | dml.FL_REF))
     c.close()
+
+
+@pytest.mark.parametrize("call", ["brownian", "ermak_a", "overlap", "overlap_rounds"])
+def test_no_memory_for_injected_numbers(dml, call):
+    """the call fails, and does not draw numbers of its own instead"""
+    rng = np.random.default_rng(3)
+    c = dml.Context(dml.dana_config([40.0, 40.0, 60.0], 2.0, 256, z0=60.0, zmax=60.0, seed=5,
+                                    integrator=dml.ERMAK if call == "ermak_a" else dml.BROWNIAN,
+                                    reservoir=dml.NO_RESERVOIR,
+                                    overlap_mode=dml.OVERLAP_EXACT if call == "overlap"
+                                    else dml.OVERLAP_ROUNDS))
+    c.set_state(rng.random((60, 3)) * [39.0, 39.0, 58.0] + 0.5)
+    c.test_update()
+    before = c.state()
+    args = {"brownian": (np.zeros(180), np.zeros(60)), "ermak_a": (np.zeros(360), np.zeros(60)),
+            "overlap": (np.zeros((1, 64)),), "overlap_rounds": (np.zeros((4, 256)), 4)}[call]
+    for k in (1, 2)[:1 if call.startswith("overlap") else 2]:
+        _fail_malloc(dml, k)
+        with pytest.raises(dml.DmlError) as e:
+            getattr(c, call)(*args)
+        assert e.value.status == -3 and _left(dml) == 0
+        after = c.state()
+        for x in before:
+            np.testing.assert_array_equal(after[x], before[x], err_msg=x)
+    c.close()
