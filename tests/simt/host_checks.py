@@ -172,3 +172,16 @@ def test_no_memory_for_injected_numbers(dml, call):
         for x in before:
             np.testing.assert_array_equal(after[x], before[x], err_msg=x)
     c.close()
+
+
+def test_failed_allocation_is_not_reported_by_a_later_call(dml):
+    c = _system(dml)
+    _fail_malloc(dml, 1)
+    with pytest.raises(dml.DmlError):
+        c.set_chunk(np.random.default_rng(4).random((50, 3)) * 9.0, 30.0, 40.0)
+    pts = np.array([[1.0, 2.0, 3.0], [20.0, 20.0, 20.0]])
+    du, hard = c.gcmc_trial_energy(pts, noalloc=True)
+    want, hard2 = c.gcmc_trial_energy(pts)
+    np.testing.assert_array_equal(du, want)
+    np.testing.assert_array_equal(hard, hard2)
+    c.close()

@@ -333,10 +333,11 @@ extern "C" long long simt_inactive_reads() { return sim::g_diag_inactive; }
 // the simt_fail_malloc-th allocation from now fails (0: none)
 extern "C" int simt_fail_malloc;
 int simt_fail_malloc = 0;
+static hipError_t g_last = hipSuccess;
 hipError_t hipMalloc(void **p, size_t n) {
   if (simt_fail_malloc > 0 && --simt_fail_malloc == 0) {
     *p = nullptr;
-    return hipErrorOutOfMemory;
+    return g_last = hipErrorOutOfMemory;
   }
   *p = malloc(n ? n : 1);
   return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -407,7 +408,11 @@ hipError_t hipStreamSynchronize(hipStream_t) {
   return hipSuccess;
 }
 hipError_t hipDeviceSynchronize() { return hipStreamSynchronize(nullptr); }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 void sincospi(double x, double *s, double *c) {
   *s = sin(M_PI * x);
   *c = cos(M_PI * x);
