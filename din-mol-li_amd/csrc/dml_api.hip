@@ -101,9 +101,7 @@ struct dml_ctx {
   uint64_t map_sig = 0;     // layout the flat work lists were built for
   int64_t map_version = 0;  // bumped at every rebuild of the work lists
   int64_t cap_cm = 0, cap_tm = 0, cap_wm = 0;
-  int64_t graph_modes = -1;  // mode signature the captured step was built for
-  uint64_t graph_dsig = 0;   // device-state bytes the captured step was built with
-  uint64_t graph_gb = 0;     // replicas whose trials it runs as batches
+  uint64_t graph_key = 0;    // what the captured step was built for
   int64_t gb_total = 0;      // batched-GCMC trial pool (sum of the replicas' capacities)
   int dev = 0;               // the GPU current at creation
   // the host mirror (reps[].p) holds what the device table does: set by every
@@ -491,7 +489,11 @@ unsigned clamp_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<
 // 7,168: 16 dense replicas 141, 115; 2M dense 980, 835; 8 replicas of 206,000
 // atoms in all 107, 97; 24 of 326,000 218, 184; 400,000 dilute ions 211, 179;
 // 150,000 dilute 75, 75); fewer dilute ions are done sooner by the resident
-// ones alone (60,000: 35, 40; 20,000: 18, 21; a chunks run's step 290, 301)
+// ones alone (60,000: 35, 40; 20,000: 18, 21; a chunks run's step 290, 301).
+// Above 1.4 million reserved cells a workgroup for 200 of them: dispatched in
+// list order, they keep the waves of an XCD near each other in the list (256
+// replicas, 4.3 million cells: 7,168 2.03 ms, 21,504 1.94, 65,528 1.93; 418,000
+// cells: 184 us, 215, 249)
 void wr_shape(const dml_ctx *c, int *sl, int *g) {
   int64_t nref = 0, cells = 0;
   for (auto &h : c->reps) {
@@ -503,7 +505,9 @@ void wr_shape(const dml_ctx *c, int *sl, int *g) {
   const bool dense = nref >= 4 * cells;
   *sl = !dense || nref >= 200000 ? 0 : nref >= 24000 ? 1 : 2;
   const int64_t need = ((c->d.n_cm << *sl) + 3) / 4;
-  const int64_t most = dense || nref >= 150000 ? 7168 : 1792;
+  const int64_t most = dense || nref >= 150000
+                           ? std::min<int64_t>(std::max<int64_t>(7168, c->d.n_cm / 200), 65528)
+                           : 1792;
   *g = (int)(std::min(std::max<int64_t>(need, 8), most) + 7) / 8 * 8;
 }
 
@@ -2093,30 +2097,25 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     if ((rc = finish(c, 0))) return rc;
     refresh_modes(c);  // a replica halted by an overflow may run again
   }
-  // what the captured step depends on: the phases present and the launch
-  // shapes (rounds <= 32, lanes <= 64)
+  // what the captured step depends on: the phases present, the launch shapes,
+  // the replicas that run batches (enq_gcmc launches by replica) and the device
+  // state, which it holds by value (a reallocation or resize of rows, cells,
+  // work lists or the chunk pool needs a new capture)
   int lb_sl, lb_g;
   wr_shape(c, &lb_sl, &lb_g);
-  const int64_t modes = (int64_t)lb_sl << 36 | (int64_t)lb_g << 38 | (int64_t)c->any_ermak | c->any_brown << 1 | c->any_rounds << 2 |
-                        c->any_exact << 3 | c->any_piston << 4 | c->any_gcmc << 5 |
-                        (int64_t)c->any_chunks << 31 |
-                        (int64_t)c->rounds << 6 | (int64_t)c->lpa << 12 |
-                        (int64_t)c->lpa_ov << 19 | (int64_t)c->ov_lanes_set << 52 |
-                        (int64_t)(live_slots(c) < 300000) << 53 | (int64_t)by_cell(c) << 54 | (int64_t)c->lb_mode << 26 |
-                        (int64_t)c->any_lb[0] << 32 | (int64_t)c->any_lb[1] << 33 |
-                        (int64_t)c->any_lb[2] << 34 | (int64_t)c->any_lb[3] << 35;
-  // a captured step holds the device state by value: any reallocation or
-  // resize (rows, cells, work lists, chunk pool) needs a new capture
-  uint64_t dsig = 1469598103934665603ull;
+  uint64_t key = 1469598103934665603ull;
+  auto mix = [&](uint64_t v) { key = (key ^ v) * 1099511628211ull; };
+  for (int v : {c->any_ermak, c->any_brown, c->any_rounds, c->any_exact, c->any_piston,
+                c->any_gcmc, c->any_chunks, c->any_lb[0], c->any_lb[1], c->any_lb[2],
+                c->any_lb[3], c->rounds, c->lpa, c->lpa_ov, c->ov_lanes_set, c->lb_mode, lb_sl,
+                lb_g, (int)(live_slots(c) < 300000), (int)by_cell(c)})
+    mix((uint64_t)(uint32_t)v);
+  for (auto &h : c->reps) mix((uint64_t)gcmc_batched(h.p));
   {
     const unsigned char *b = (const unsigned char *)&c->d;
-    for (size_t q = 0; q < sizeof(DevState); q++) dsig = (dsig ^ b[q]) * 1099511628211ull;
+    for (size_t q = 0; q < sizeof(DevState); q++) mix(b[q]);
   }
-  // and so are the replicas that run batches (enq_gcmc launches by replica)
-  uint64_t gb = 1469598103934665603ull;
-  for (auto &h : c->reps) gb = (gb ^ (uint64_t)gcmc_batched(h.p)) * 1099511628211ull;
-  if (use_graph && (!c->gexec || c->graph_modes != modes || c->graph_dsig != dsig ||
-                    c->graph_gb != gb)) {
+  if (use_graph && (!c->gexec || c->graph_key != key)) {
     if (c->gexec) {
       hipGraphExecDestroy(c->gexec);
       hipGraphDestroy(c->graph);
@@ -2127,9 +2126,7 @@ int dml_run(dml_ctx *c, int32_t nsteps, int32_t use_graph) {
     HIPCHECK(hipStreamEndCapture(c->st, &c->graph));
     HIPCHECK(hipGraphInstantiate(&c->gexec, c->graph, nullptr, nullptr, 0));
     c->graph_rounds = c->rounds;
-    c->graph_modes = modes;
-    c->graph_dsig = dsig;
-    c->graph_gb = gb;
+    c->graph_key = key;
   }
   c->fresh = 0;
   HIPCHECK(hipEventRecord(c->e0, c->st));

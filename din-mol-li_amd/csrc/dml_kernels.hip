@@ -995,9 +995,9 @@ __device__ inline int cm_first(int v) { return (int)((uint32_t)v >> 25); }
 // entries per cell, by k_cell_sort_w; 0 for a cell that is not rebuilt), 64 per
 // load, so an empty cell costs a lane of one load, and the centre atoms are
 // loaded beside the stencil's counts without a read past the cell's own (with
-// all 64 lanes reading, 256 dense replicas rebuilt at once took 2.34 ms, now
-// 2.06; with cells in contiguous runs per wave 1.90, but the step, which
-// rebuilds some of them, 6.3 ms against 6.05).
+// all 64 lanes reading, 256 replicas rebuilt at once took 2.34 ms, without 2.06,
+// with the grid that wr_shape chooses 1.94; with cells in contiguous runs per
+// wave 1.90, but the step, which rebuilds some of them, 6.3 ms against 5.86).
 //
 // What bounds it: instruction issue (about 30 instructions a chunk of 64 pair
 // tests) with the wait for a pass's candidates behind it.  Before, each wave
@@ -1052,8 +1052,10 @@ k_listbuild_wr(DevState s, int sl) {
       const int64_t g = (j / LB_BLK * 8 + xcd) * LB_BLK + j % LB_BLK;
       if (g < s.n_cm) {
         ln = s.cm_nref[g];
-        lr = s.cm_rep[g];
-        lc = s.cm_cell[g];
+        if (ln != 0) {
+          lr = s.cm_rep[g];
+          lc = s.cm_cell[g];
+        }
       }
     }
     // a cell of few ref atoms is not split into all the parts
