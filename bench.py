@@ -649,13 +649,15 @@ def main():
         if args.replicas == 256 and os.path.exists(tf):
             measured = json.load(open(tf))["hbm_bytes_per_launch"]
         # priced against HBM (its compulsory bytes); what holds it back is
-        # latency: its waves wait on memory about half their cycles and
-        # issue VALU a fifth of them (instruction counters under profiles/)
+        # HBM and its latency: it reads candidates more than once (`traffic`)
+        # and its waves wait on memory about half their cycles and issue VALU
+        # a tenth of them (counters under profiles/)
         res["roofline"] = {"kernel": kname, "bound": "hbm", "achieved": ach,
                            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                            "traffic": measured, "avg_launch_ms": batched["list_ms"],
                            "algorithmic_bytes_per_launch": traffic,
-                           "limiter": "memory latency (waits ~50% of wave cycles, VALU issue ~20%)"}
+                           "limiter": "HBM and its latency (3.7 TB/s drawn, waits ~53% of wave "
+                                      "cycles, VALU issue ~11%)"}
         res["kernel_ms"] = {kname: batched["list_ms"], "k_force": batched["force_ms"]}
         res["particles_stepped_mean"] = batched["particles_stepped"]
         res["c3_full_run"] = batched["full_run"]
