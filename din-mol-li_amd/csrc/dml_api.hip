@@ -486,7 +486,7 @@ unsigned clamp_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<
 // split 930); sparse cells (a few atoms) are never split (1,505 ions of a
 // chunks run: 10.6, split 12.3).  Workgroups: 7,168, four times the resident
 // ones, even out the tail where there is work for them (us with 1,792 and
-// 7,168: 16 dense replicas 141, 115; 2M dense 980, 835; 8 replicas of 206,000
+// 7,168: 16 mixed replicas 176, 147; 2M dense 980, 835; 8 replicas of 206,000
 // atoms in all 107, 97; 24 of 326,000 218, 184; 400,000 dilute ions 211, 179;
 // 150,000 dilute 75, 75); fewer dilute ions are done sooner by the resident
 // ones alone (60,000: 35, 40; 20,000: 18, 21; a chunks run's step 290, 301).

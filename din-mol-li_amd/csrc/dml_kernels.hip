@@ -1000,11 +1000,13 @@ __device__ inline int cm_first(int v) { return (int)((uint32_t)v >> 25); }
 // wave 1.90, but the step, which rebuilds some of them, 6.3 ms against 5.86).
 //
 // What bounds it: instruction issue (about 30 instructions a chunk of 64 pair
-// tests) with the wait for a pass's candidates behind it.  Before, each wave
+// tests) with the wait for a pass's candidates behind it; in a large ensemble
+// HBM, 3.7 TB/s, since several XCDs read a cell's candidates.  Before, each wave
 // took one contiguous run of cells, an XCD one eighth of the list, every cell
 // was looked at through its replica's parameters and a stencil lane wrote its
-// cell's entries one by one: 100,000 particles 265 -> 79 us a build, 24 mixed
-// replicas 472 -> 320, 2M 1,775 -> 835, 1,505 ions in sparse cells 37 -> 11.
+// cell's entries one by one: 100,000 dense atoms 253 -> 80 us a build, 24 mixed
+// replicas 833 -> 184, 2M 1,764 -> 826, 1,505 ions in sparse cells 36 -> 10,
+// but 256 replicas at once 1.78 -> 1.94 ms.
 // ------------------------------------------------------------------------
 #define LB_PART 6
 #define LB_BLK 64
