@@ -64,6 +64,7 @@ struct HostRep {
   RepParams p;         // host mirror of the static parameters
   int64_t creg = 0;    // cell-count entries reserved for this replica
   int64_t breg = 0;    // bucket entries reserved for this replica
+  int64_t chas = 0, bhas = 0;  // of both, what is in place (less while cells_dirty)
   std::vector<double> chunk;  // block template (config_chunk), 6 x nchunk SoA
 };
 
@@ -462,6 +463,7 @@ int alloc_cells(dml_ctx *c) {
   e |= dalloc(&c->d.gb_claim, CS);
   if (e) {
     // the next call that needs cells tries again, on the layout of the device table
+    for (auto &h : c->reps) h.chas = h.bhas = 0;
     c->cells_dirty = 1;
     c->fresh = 0;
     return DML_E_NOMEM;
@@ -472,6 +474,10 @@ int alloc_cells(dml_ctx *c) {
   HIPCHECK(hipMemsetAsync(c->d.gb_claim, 0, sizeof(int32_t) * CS, c->st));
   c->C = C;
   c->B = B;
+  for (auto &h : c->reps) {
+    h.chas = h.creg;
+    h.bhas = h.breg;
+  }
   return DML_OK;
 }
 
@@ -1622,6 +1628,8 @@ int dml_cells(dml_ctx *c, int32_t rep, int32_t ncells[3], double cell[3], int32_
     for (int i = 0; i < 3 * n; i++) cell_of[i] = -1;
     if (!p.use_cells) return DML_OK;
     int nc = ncells_total(p);
+    // nothing is sorted into cells that are not in place yet
+    if (nc > c->reps[rep].chas || (int64_t)nc * p.bcap > c->reps[rep].bhas) return DML_OK;
     std::vector<int32_t> cnt(nc);
     std::vector<int32_t> bk((size_t)nc * p.bcap);
     HIPCHECK(hipMemcpy(cnt.data(), c->d.cell_cnt + p.coff, sizeof(int32_t) * nc, hipMemcpyDeviceToHost));
@@ -2265,8 +2273,7 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   if (g.capacity <= 0 || g.box[0] <= 0 || g.box[1] <= 0 || g.box[2] <= 0 || g.rcut <= 0 ||
       g.nadj < 0 || g.nadj > (1 << 21))
     return DML_E_ARG;
-  // the cell region that the new box is checked against is the one in place
-  int rc = c->cells_dirty ? ensure_cells(c) : fetch_params(c);
+  int rc = fetch_params(c);
   if (rc) return rc;
   HostRep &h = c->reps[rep];
   if (round_up(g.capacity, DML_BLOCK) > h.p.pcap) return DML_E_NOMEM;
@@ -2308,7 +2315,9 @@ int dml_reconfigure(dml_ctx *c, int32_t rep, const dml_config *cfg) {
   }
   h.cfg = g;
   h.p = p;
-  hipMemsetAsync(c->d.cell_cnt + p.coff, 0, sizeof(int32_t) * p.ccap, c->st);
+  // (cells that are only reserved yet are clear when they are put in place)
+  if (p.ccap <= h.chas)
+    hipMemsetAsync(c->d.cell_cnt + p.coff, 0, sizeof(int32_t) * p.ccap, c->st);
   hipMemsetAsync(c->d.cnt + (int64_t)rep * c->d.ncsh, 0, sizeof(DevCounters) * c->d.ncsh, c->st);
   hipMemsetAsync(c->d.ov_near + p.poff, 0xff, (size_t)p.pcap, c->st);
   refresh_modes(c);

@@ -133,6 +133,25 @@ def test_reconfigure_before_the_larger_cells_are_there(dml):
     fresh.close()
 
 
+def test_cells_that_are_not_in_place_hold_nothing(dml):
+    c = dml.Context(_chunks(dml))
+    pos = np.random.default_rng(6).random((60, 3)) * [39.0, 39.0, 58.0] + 0.5
+    c.set_state(pos)
+    c.test_update()
+    sorted_now = c.cells()[3]
+    assert (sorted_now >= 0).all()
+    c.set_chunk(np.random.default_rng(3).random((4, 3)) * [40.0, 40.0, 9.0], 12.2, 55.0)
+    np.testing.assert_array_equal(c.cells()[3], sorted_now)  # the box is what it was
+    c.reconfigure(dml.dana_config([40.0, 40.0, 600.0], 2.0, 256, z0=30.0, zmax=600.0,
+                                  integrator=dml.BROWNIAN, reservoir=dml.NO_RESERVOIR), 0)
+    c.set_state(pos)
+    nc, cell, use, of = c.cells()
+    assert nc[2] == 115 and use and (of == -1).all()
+    c.test_update()
+    assert (c.cells()[3] >= 0).all()
+    c.close()
+
+
 def test_state_is_read_without_memory_to_stage_it(dml):
     c = dml.Context(dml.dana_config([40.0, 40.0, 60.0], 2.0, 4096, z0=30.0))
     pos = np.random.default_rng(8).random((4096, 3)) * 39.0
